@@ -560,9 +560,8 @@ def main():
         kernels["ssa_bwd_dq_kernel"]["alg_bytes"] = ds_bytes + (B * Hkv + B * Hq) * S * D * esize
     pre_bytes = 2 * B * Hq * S * D * esize + 4 * B * Hq * S
     kernels["ssa_bwd_preprocess_kernel"]["alg_bytes"] = pre_bytes
-    # fp32 inputs run on the vector ALU: priced against the published fp32 peak
-    # (157.3, which needs packed fp32) and, as frac_valu_peak, against what
-    # non-packed fp32 FMAs can reach (78.6)
+    # fp32 inputs run on the fp32 MFMA: priced against its published peak (157.3)
+    # and, as frac_valu_peak, against what non-packed fp32 FMAs can reach (78.6)
     peak_flops = PEAK_FP32_TFLOPS if dtype == torch.float32 else PEAK_BF16_TFLOPS
     traffic = measured_traffic(args.config) if args.dtype == "bf16" else {}
     counters = measured_counters(args.config) if args.dtype == "bf16" else {}

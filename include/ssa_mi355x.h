@@ -60,12 +60,12 @@ enum {
  * Element types of q/k/v/out/dout/dq/dk/dv.  bf16 / fp16 run on the MFMA
  * kernels at head dims 32, 64, 128.  fp32 -- the reference's fp32-operand
  * path (training/train/train_ssa_triton/SSA/ssa_triton_kernel.py:766-772,
- * 819-825) -- runs on fp32 vector-ALU kernels (head dims 16, 32, 64, 128,
- * 256) that keep every product in fp32: full precision, a fraction of the
+ * 819-825) -- runs on kernels of its own (head dims 16, 32, 64, 128, 256)
+ * that keep every product and sum in fp32: full precision, a fraction of the
  * bf16 throughput.  bf16 / fp16 at head dim 256 (the reference takes every
  * power-of-two head dim, ssa_triton_kernel.py:761-764) run on the same
- * vector-ALU kernels, elements widened to fp32 on load.  On the vector-ALU
- * kernels the dS' workspace is not used (dq recomputes the scores); the
+ * kernels, with fp32 probabilities and score gradients.  On these
+ * fp32-precision kernels the dS' workspace is not used (dq recomputes the scores); the
  * decode step takes bf16 / fp16 at head dims 32, 64, 128.
  */
 enum { SSA_DTYPE_BF16 = 0, SSA_DTYPE_FP16 = 1, SSA_DTYPE_FP32 = 2 };
@@ -116,7 +116,7 @@ typedef struct ssa_bwd_args {
                            both steps must get the same pointer.  Packed
                            sequences (ssa_varlen_bwd) need
                            ssa_varlen_bwd_ds_workspace_bytes() bytes.  The
-                           vector-ALU kernels (fp32; head dim 256) ignore it:
+                           fp32-precision kernels (fp32; head dim 256) ignore it:
                            their dq always recomputes. */
 } ssa_bwd_args;
 

@@ -33,10 +33,10 @@ fp16, head dim 16 (the smallest the reference's Triton kernel takes) runs on
 the D = 32 kernels with its operands zero-padded to 32 columns, which changes
 no score, dP or Delta, and the results are sliced back (the decode step is not
 offered at D = 16).  fp32 inputs (the reference's fp32-operand path) run on
-fp32 vector-ALU kernels for head dims 16-256 that keep every product in fp32,
+kernels of their own for head dims 16-256 (fp32 matrix-core products and sums),
 without the dS' workspace; bf16 / fp16 at head dim 256 (the largest power of
-two the reference takes) run on the same kernels, widened on load (coverage,
-not speed); the decode step takes bf16 / fp16 only.  Errors:
+two the reference takes) run on the same kernels, whose fp32 weights enter the
+16-bit products as two halves; the decode step takes bf16 / fp16 only.  Errors:
 ``AssertionError`` for ``Hq % Hkv != 0`` and a non-power-of-two head dim, as in
 the reference; ``ValueError`` for other head dims and other dtypes.
 """
@@ -145,9 +145,9 @@ def ssa_flash_attn_forward(q, k, v, softmax_scale, ssa_n, ssa_b, causal=True):
 
 def _has_ds_path(dtype: torch.dtype, head_dim: int) -> bool:
     """Whether the backward kernels for ``dtype`` / ``head_dim`` can use a dS'
-    workspace: the matrix-core kernels (bf16 / fp16 at head dims up to 128)
-    can; the fp32-arithmetic vector-ALU kernels (fp32, and head dim 256) always
-    recompute the scores in dq and ignore it."""
+    workspace: the 16-bit kernels (bf16 / fp16 at head dims up to 128) can; the
+    fp32-precision kernels (fp32, and head dim 256) always recompute the scores
+    in dq and ignore it."""
     return dtype != torch.float32 and head_dim <= 128
 
 

@@ -1,27 +1,48 @@
-// SSA attention forward and backward with fp32 arithmetic, on the vector ALU:
-// the kernels of fp32 inputs at every head dim, and of bf16 / fp16 inputs at
-// head dim 256 (the matrix-core kernels cover bf16 / fp16 at 32, 64 and 128).
+// SSA attention forward and backward with every product and sum kept in fp32
+// precision, on the matrix cores: the kernels of fp32 inputs at every head
+// dim, and of bf16 / fp16 inputs at head dim 256 (the kernels of ssa_fwd.hip
+// and ssa_bwd*.hip cover bf16 / fp16 at 32, 64 and 128).
 //
 // The reference runs its Triton kernels on fp32 tensors with fp32 operands in
 // the dot products (MATMUL_PRECISION = tl.float32,
 // training/train/train_ssa_triton/SSA/ssa_triton_kernel.py:766-772, 819-825)
 // and checks them to atol 5e-4 / rtol 1e-3 and scalar 5e-5 + 1e-4 |ref|
 // (check_ssa_triton_parity.py:1064-1069), a bar that no bf16 rounding of the
-// operands meets.  These kernels keep every product in fp32 FMA and every
-// transcendental in the hardware's f32 exp2 / log2 / rcp.  They follow the
-// equations of ssa_fwd.hip / ssa_bwd.hip with simple structures: each row of
-// the register-resident operand is split over P adjacent lanes (P = D / 32
-// from head dim 64 on, so a lane holds at most 32 columns of each row; the
-// partial dot products meet by butterfly shuffles), and the other operand's
-// rows are shared through LDS, converted to fp32 on the way in, and read as
-// broadcasts.  bf16 / fp16 elements are widened on load and rounded to
-// nearest even on store.  Masks, GQA, packed sequences and the dn / db
-// partials (one per 128-key block, the layout ssa_reduce_partials_kernel
-// sums) are those of the matrix-core path; the reference accepts every
-// power-of-two head dim (ssa_triton_kernel.py:761-764), and head dim 256 is
-// the largest its Triton tiles hold.
+// operands meets.  Masks, GQA, packed sequences and the dn / db partials (one
+// per 128-key block, the layout ssa_reduce_partials_kernel sums) are those of
+// the other kernels; the reference accepts every power-of-two head dim
+// (ssa_triton_kernel.py:761-764), and head dim 256 is the largest its Triton
+// tiles hold.
+//
+// One structure for all three kernels.  A wave owns 32 rows (queries in the
+// forward and dQ, keys in dK/dV), one per lane pair (l, l + 32), and holds
+// their operand fragments in registers; the other side streams through LDS in
+// blocks of 32 rows (direct-to-LDS loads, the next stage in flight under the
+// current one).  Two operations do all the work (Mat below):
+//   scores: S = X_streamed X_own^T, the streamed row on the accumulator's row
+//           axis, so lane l holds the scores of its own row with streamed
+//           rows crow(r, hh);
+//   outer:  acc^T += X_streamed^T w, w the 16 weights (P or dS') of the lane's
+//           own row, straight from the accumulator they were computed in.
+// fp32: v_mfma_f32_32x32x2_f32, whose products and sums are fp32.  bf16 / fp16
+// at head dim 256: the score products take the inputs as they are (exact in
+// fp32), and the weights, which are fp32, go in as the sum of two 16-bit
+// halves (w = hi + lo, relative error 2^-17 in bf16, 2^-22 in fp16), each
+// multiplied on the matrix cores, so no probability is rounded to 16 bits.
+//
+// What bounds it: an fp32 MFMA takes 64 cycles for 4096 FLOPs, so the fp32
+// kernels run at the rate of the matrix cores' fp32 form (138 TFLOP/s in a
+// large library product) and need little of LDS or the vector ALU.  The
+// streamed rows are split over the waves of a workgroup (kw = 2 or 4 blocks
+// at a time) up to head dim 128, so that a workgroup owns 32 or 64 rows: a
+// grid of one sequence then fills the chip, and causal blocks balance.
+// Measured (us, the earlier vector-ALU kernels -> these): fp32, B = 1, H = 16,
+// N = 1024, D = 64 causal: forward 376 -> 42, dK/dV 498 -> 144, dQ 380 -> 51;
+// bf16, B = 1, H = 16, N = 2048, D = 256 causal: 3792 -> 126, 4622 -> 252,
+// 4332 -> 126.
 #include "ssa_common.hpp"
 #include "ssa_launch.hpp"
+#include "ssa_tile.hpp"
 
 namespace ssa {
 
@@ -50,126 +71,332 @@ __device__ __forceinline__ void st4(T* p, f32x4 v) {
 // sL = sign(x) log2(1 + c|x|) for a raw score x = q.k, c = scale b; u1 = 1 + c|x|
 __device__ __forceinline__ float ssa_sl(float x, float u1) { return copysignf(fast_log2(u1), x); }
 
-constexpr int kF32Rows = 64;   // query rows per forward workgroup
-constexpr int kF32Tile = 32;   // rows per LDS tile of the streamed operand
-constexpr int kF32Pair = 128;  // keys (dK/dV) or queries (dQ) per backward workgroup
-
-// Lanes per row: the forward splits rows from head dim 64 on, the backward
-// (which holds two or three row operands per lane) always.
-template <int D>
-constexpr int fwd_parts() {
-  return D >= 64 ? D / 32 : 1;
-}
-template <int D>
-constexpr int bwd_parts() {
-  return D >= 64 ? D / 32 : 2;
-}
-// Rows of the backward block held at once: all 128 up to head dim 128; at 256
-// (8 lanes per row) 64, in two passes, so that a workgroup stays at 512 lanes
-// and each lane keeps its four 32-column row shares (128 registers) in the
-// 256 registers of two waves per SIMD.
-template <int D>
-constexpr int bwd_rows() {
-  return D >= 256 ? 64 : kF32Pair;
-}
-template <int D>
-constexpr int fwd_threads() {
-  return kF32Rows * fwd_parts<D>();
-}
-template <int D>
-constexpr int bwd_threads() {
-  return bwd_rows<D>() * bwd_parts<D>();
-}
-
-// Dot product of a lane's CP four-column chunks with the same chunks of an
-// LDS row.
-template <int CP>
-__device__ __forceinline__ float part_dot(const f32x4* reg, const f32x4* lds) {
-  float s = 0.f;
-#pragma unroll
-  for (int c = 0; c < CP; ++c) {
-    const f32x4 x = lds[c];
-    s = fmaf(reg[c].x, x.x, s);
-    s = fmaf(reg[c].y, x.y, s);
-    s = fmaf(reg[c].z, x.z, s);
-    s = fmaf(reg[c].w, x.w, s);
+// The two matrix operations on a streamed block of 32 rows x D in LDS, stored
+// in the block-chunk-major layout of ssa_tile.hpp (LD: its width in 16-bit
+// columns, so fp32 blocks are 2 D wide and the same loaders move them).
+template <typename T, int D>
+struct Mat {  // bf16 / fp16
+  static constexpr int LD = D, BLOCK = BlockLayout<LD>::BLOCK, ND = D / 32, NF = D / 16;
+  // fp16 holds 2^-24 .. 65504: probabilities (at most 1) are scaled up so that
+  // the halves of all that matter stay normal; bf16 has fp32's range.
+  static constexpr bool F16 = sizeof(T) == 2 && !__is_same(T, __bf16);
+  static constexpr float P_SHIFT = F16 ? 12.f : 0.f;
+  typedef typename Vec8<T>::type frag;
+  typedef T v4 __attribute__((ext_vector_type(4)));
+  RowBase<LD> rb;
+  TrBase<LD> tb;
+  __device__ __forceinline__ explicit Mat(int lane) : rb(lane & 31, lane >> 5), tb(lane) {}
+  // fragment f of the row at `row`: columns 16 f + 8 hh + (0..7)
+  __device__ static __forceinline__ frag load(const T* row, int f, int hh) {
+    return load16<frag>(row + 16 * f + 8 * hh);
   }
-  return s;
-}
-
-// Sum over the P adjacent lanes of a row (P in {1, 2, 4, 8}); every lane gets it.
-template <int P>
-__device__ __forceinline__ float sum_parts(float x) {
-  if constexpr (P >= 2) x += __shfl_xor(x, 1, 64);
-  if constexpr (P >= 4) x += __shfl_xor(x, 2, 64);
-  if constexpr (P >= 8) x += __shfl_xor(x, 4, 64);
-  return x;
-}
-
-// ---------------------------------------------------------------------------
-// Forward: P lanes = one query row, the lane's share of q and of the
-// accumulator in registers, K / V tiles of 32 keys in LDS; exact running max
-// (online softmax in base 2), the same in the P lanes of a row.
-template <typename T, int D, bool CAUSAL>
-__global__ __launch_bounds__(fwd_threads<D>()) void ssa_fwd_f32_kernel(FwdParams p) {
-  constexpr int P = fwd_parts<D>(), C4 = D / 4, CP = C4 / P, NT = fwd_threads<D>();
-  __shared__ f32x4 ks[kF32Tile * C4], vs[kF32Tile * C4];
-  const int tid = threadIdx.x, part = tid % P;
-  const int nqb = (p.N + kF32Rows - 1) / kF32Rows;
-  const int qb = blockIdx.x % nqb, bh = blockIdx.x / nqb;
-  const int b = bh % p.B, h = bh / p.B, hk = h / (p.Hq / p.Hkv);
-  const SeqView sv(p.cu_seqlens, p.T, p.N, b);
-  const int N = sv.N;
-  const int q0 = qb * kF32Rows;
-  if (q0 >= N) return;  // packed: past the end of a shorter document
-  const int i = q0 + tid / P;
-  const T* qg = static_cast<const T*>(p.q.ptr) + sv.off(p.q, b) + h * p.q.sh;
-  const T* kg = static_cast<const T*>(p.k.ptr) + sv.off(p.k, b) + hk * p.k.sh;
-  const T* vg = static_cast<const T*>(p.v.ptr) + sv.off(p.v, b) + hk * p.v.sh;
-  T* og = static_cast<T*>(const_cast<void*>(p.o.ptr)) + sv.off(p.o, b) + h * p.o.sh;
-  const float n = *p.n_ptr, bv = *p.b_ptr, c = p.scale * bv;
-
-  f32x4 qv[CP], acc[CP];
+  __device__ __forceinline__ f32x16 scores(uint32_t lds, const frag* own) const {
+    const RowBase<LD> r = at_tile(rb, lds);
+    f32x16 s = f32x16{};
 #pragma unroll
-  for (int c4 = 0; c4 < CP; ++c4) {
-    qv[c4] = i < N ? ld4(qg + i * p.q.ss + 4 * (part * CP + c4)) : f32x4{0.f, 0.f, 0.f, 0.f};
-    acc[c4] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int f = 0; f < NF; ++f) s = mfma32(tile_read_row<LD, frag>(r, 0, f), own[f], s);
+    return s;
   }
-  float m = -__builtin_inff(), l = 0.f;
-  const int kv_end = CAUSAL ? min(N, q0 + kF32Rows) : N;
-  for (int k0 = 0; k0 < kv_end; k0 += kF32Tile) {
-    __syncthreads();  // the previous tile is consumed
-    for (int idx = tid; idx < kF32Tile * C4; idx += NT) {
-      const int row = min(k0 + idx / C4, N - 1), c4 = idx % C4;
-      ks[idx] = ld4(kg + row * p.k.ss + 4 * c4);
-      vs[idx] = ld4(vg + row * p.v.ss + 4 * c4);
+  __device__ __forceinline__ void outer(uint32_t lds, const float* w, f32x16* acc) const {
+    const TrBase<LD> t = at_tile(tb, lds);
+    frag hi[2], lo[2];
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      const T h = static_cast<T>(w[r]);
+      hi[r >> 3][r & 7] = h;
+      lo[r >> 3][r & 7] = static_cast<T>(w[r] - static_cast<float>(h));
     }
-    __syncthreads();
-    const int kn = min(kF32Tile, kv_end - k0);
-    for (int j = 0; j < kn; ++j) {
-      const float s = sum_parts<P>(part_dot<CP>(qv, ks + j * C4 + part * CP));
-      if (i < N && (!CAUSAL || k0 + j <= i)) {
-        const float t2 = n * ssa_sl(s, fmaf(c, fabsf(s), 1.f));
-        if (t2 > m) {  // the running max moves: rescale what is summed so far
-          const float alpha = fast_exp2(m - t2);
-          l *= alpha;
 #pragma unroll
-          for (int c4 = 0; c4 < CP; ++c4) acc[c4] *= alpha;
-          m = t2;
-        }
-        const float pv = fast_exp2(t2 - m);
-        l += pv;
-        const f32x4* vrow = vs + j * C4 + part * CP;
+    for (int ks = 0; ks < 2; ++ks) {
 #pragma unroll
-        for (int c4 = 0; c4 < CP; ++c4) acc[c4] += pv * vrow[c4];
+      for (int d0 = 0; d0 < ND; d0 += 2) {
+        frag a[2];
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+          a[i] = __builtin_shufflevector(tile_read_tr<LD, v4>(t, 0, ks, 0, d0 + i),
+                                         tile_read_tr<LD, v4>(t, 0, ks, 1, d0 + i), 0, 1, 2, 3, 4, 5, 6, 7);
+#pragma unroll
+        for (int i = 0; i < 2; ++i) acc[d0 + i] = mfma32(a[i], hi[ks], acc[d0 + i]);
+#pragma unroll
+        for (int i = 0; i < 2; ++i) acc[d0 + i] = mfma32(a[i], lo[ks], acc[d0 + i]);
       }
     }
   }
-  if (i < N) {
-    const float inv = 1.f / l;  // every row has a key (causal: itself)
+};
+
+template <int D>
+struct Mat<float, D> {
+  static constexpr int LD = 2 * D, BLOCK = BlockLayout<LD>::BLOCK, ND = D >= 32 ? D / 32 : 1, NF = D / 8;
+  static constexpr bool F16 = false;
+  static constexpr float P_SHIFT = 0.f;
+  typedef f32x4 frag;
+  RowBase<LD> rb;
+  uint32_t ob[2];
+  // ob: streamed row 8 a + 4 hh + e, column 32 db + l32 sits in chunk c = 8 db +
+  // l32 / 4 at row position (row ^ 4 (c & 3)); the XOR splits into the lane's
+  // part and the parity of a, so every fetch is ob[a & 1] plus an immediate.
+  // Head dim 16 has four chunks: lanes 16-31 fetch copies, and the accumulator
+  // rows they feed (columns 16-31) are never stored.
+  __device__ __forceinline__ explicit Mat(int lane) : rb(lane & 31, lane >> 5) {
+    const int l32 = lane & 31, hh = lane >> 5;
+    const int c = (l32 >> 2) & (D / 4 >= 8 ? 7 : D / 4 - 1), x = c & 3;
 #pragma unroll
-    for (int c4 = 0; c4 < CP; ++c4) st4(og + i * p.o.ss + 4 * (part * CP + c4), acc[c4] * inv);
-    if (part == 0) p.m[sv.mrow(b, h, p.Hq, p.T, p.N) + i] = m + log2f(l);
+    for (int par = 0; par < 2; ++par)
+      ob[par] = static_cast<uint32_t>(c * 512 + (8 * (par ^ (x >> 1)) + 4 * (hh ^ (x & 1))) * 16 + (l32 & 3) * 4);
+  }
+  // fragment f: columns 8 f + 4 hh + (0..3), one MFMA step each
+  __device__ static __forceinline__ frag load(const float* row, int f, int hh) { return ld4(row + 8 * f + 4 * hh); }
+  __device__ __forceinline__ f32x16 scores(uint32_t lds, const frag* own) const {
+    const RowBase<LD> r = at_tile(rb, lds);
+    f32x16 s = f32x16{};
+#pragma unroll
+    for (int f = 0; f < NF; ++f) {
+      const f32x4 a = tile_read_row<LD, f32x4>(r, 0, f);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) s = __builtin_amdgcn_mfma_f32_32x32x2f32(a[e], own[f][e], s, 0, 0, 0);
+    }
+    return s;
+  }
+  __device__ __forceinline__ void outer(uint32_t lds, const float* w, f32x16* acc) const {
+    const uint32_t b[2] = {opaque(ob[0] + lds), opaque(ob[1] + lds)};
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      const uint32_t imm = (r >> 3) * 256 + (r & 3) * 16;
+#pragma unroll
+      for (int db = 0; db < ND; ++db) {
+        const float a =
+            *(const __attribute__((address_space(3))) float*)(uintptr_t)(b[(r >> 2) & 1] + imm + db * 4096);
+        acc[db] = __builtin_amdgcn_mfma_f32_32x32x2f32(a, w[r], acc[db], 0, 0, 0);
+      }
+    }
+  }
+};
+
+// Weights (dS') of any size on the fp16 halves: a power of two per wave, set by
+// the first block with a nonzero weight and lowered (exactly) whenever a larger
+// one comes, keeps the largest weight seen below 2^15; the accumulators hold
+// the scaled sums.  Nothing on bf16 and fp32.
+template <typename M>
+struct WeightScale {
+  float s = 0.f;
+  __device__ __forceinline__ void apply(float* w, f32x16* acc) {
+    if constexpr (M::F16) {
+      float a = 0.f;
+#pragma unroll
+      for (int r = 0; r < 16; ++r) a = fmaxf(a, fabsf(w[r]));
+      if (__any(a * s > 32768.f || (s == 0.f && a > 0.f))) {  // wave-uniform
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) a = fmaxf(a, __shfl_xor(a, off, 64));
+        // 2^14 / 2^floor(log2 a), at most 2^60
+        int ex = 0;
+        (void)frexpf(a, &ex);
+        const float sn = ldexpf(1.f, min(15 - ex, 60));
+        if (s != 0.f) {
+          const float f = sn / s;
+#pragma unroll
+          for (int d = 0; d < M::ND; ++d) acc[d] *= f;
+        }
+        s = sn;
+      }
+#pragma unroll
+      for (int r = 0; r < 16; ++r) w[r] *= s;
+    }
+  }
+  __device__ __forceinline__ float inverse() const {
+    if constexpr (M::F16) return s != 0.f ? 1.f / s : 0.f;
+    return 1.f;
+  }
+};
+
+// Streamed blocks per stage (= waves that share 32 owned rows) of the forward
+// and dQ, and of dK/dV (whose workgroups own 128 keys, the unit of the dn / db
+// partials).  A stage holds two blocks (K and V, or Q and dO) per kw, twice
+// buffered, in at most 128 KB of LDS.
+template <typename T, int D>
+struct Cfg {
+  static constexpr int BB = Mat<T, D>::BLOCK;
+  static constexpr int KW = 4 * BB <= 32768 ? 4 : (BB <= 16384 ? 2 : 1);
+  static constexpr int QW = 4 / KW;  // waves on different rows (forward, dQ): 32 QW rows per workgroup
+  static constexpr int BM = 32 * QW, BN = 32 * KW;
+  static constexpr int LDS_BYTES = 2 * KW * 2 * BB;
+  // dK/dV: two waves per 32 keys up to head dim 64 (two waves per SIMD); at
+  // 256 the accumulators of dK and dV do not fit one wave beside the K and V
+  // fragments, so half of the grid computes dK (and dn, db) and half dV.
+  static constexpr int QS = D <= 64 ? 2 : 1;
+  static constexpr bool ROLES = D >= 256;
+  static constexpr int DKDV_THREADS = 256 * QS;
+  static constexpr int DKDV_STAGE = QS * (2 * BB + 256);  // Q, dO, M[32], Delta[32] per block
+};
+
+template <typename T>
+constexpr int kUnits = sizeof(T) / 2;  // 16-bit units per element (the tile loaders' strides)
+
+// A workgroup's place in a grid of nblk blocks of rows per (sequence, head):
+// XCD-contiguous, the heaviest blocks (rank 0) of a pair of heads first, as
+// FwdPlan and DkdvPlan.
+struct Place {
+  int rank, b, h;
+  __device__ __forceinline__ Place(int block, int grid, int nblk, int B, bool packed) {
+    int hb;
+    dispatch_order(xcd_remap(block, grid), grid / nblk, nblk, packed ? 1 : kOrderGroup, hb, rank);
+    b = hb % B;
+    h = hb / B;
+  }
+};
+
+// Sum (or with `scale` the rescaled sum) of the accumulators of the waves that
+// share owned rows, in the first of them (part == 0): the others leave theirs
+// in LDS, element-major so that every access is contiguous.  Called by every
+// wave; `lds` is free (all waves past their last read of the ring).
+template <int ND, int KW>
+__device__ __forceinline__ void merge_parts(f32x16* acc, float* lds, int group, int part, int lane) {
+  if constexpr (KW > 1) {
+    __syncthreads();
+    float* mine = lds + static_cast<size_t>((group * (KW - 1) + part - 1) * ND * 16 * 64) + lane;
+    if (part > 0) {
+#pragma unroll
+      for (int i = 0; i < ND * 16; ++i) mine[i * 64] = acc[i >> 4][i & 15];
+    }
+    __syncthreads();
+    if (part == 0) {
+#pragma unroll
+      for (int w = 1; w < KW; ++w) {
+        const float* src = lds + static_cast<size_t>((group * (KW - 1) + w - 1) * ND * 16 * 64) + lane;
+#pragma unroll
+        for (int i = 0; i < ND * 16; ++i) acc[i >> 4][i & 15] += src[i * 64];
+      }
+    }
+  }
+}
+
+// The lane's share of its own row: columns 32 db + 8 g + 4 hh + (0..3).
+template <typename T, int D>
+__device__ __forceinline__ void store_own(const f32x16* acc, float scale, T* row, int hh) {
+#pragma unroll
+  for (int db = 0; db < (D + 31) / 32; ++db) {
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      if (32 * db + 8 * g >= D) break;  // head dim 16
+      st4(row + 32 * db + 8 * g + 4 * hh,
+          f32x4{acc[db][4 * g], acc[db][4 * g + 1], acc[db][4 * g + 2], acc[db][4 * g + 3]} * scale);
+    }
+  }
+}
+
+// ---------------------------------------------------------------------------
+// Forward: BM queries of one (batch, q-head), K / V streamed BN keys a stage.
+// Exact running max per tile (online softmax in base 2); the waves that share
+// queries merge (m, l, acc) at the end.
+template <typename T, int D, bool CAUSAL>
+__global__ __launch_bounds__(256) void ssa_fwd_f32_kernel(FwdParams p) {
+  using M = Mat<T, D>;
+  using C = Cfg<T, D>;
+  constexpr int KW = C::KW, BM = C::BM, BN = C::BN, BB = C::BB, ND = M::ND;
+  __shared__ __attribute__((aligned(1024))) char smem[C::LDS_BYTES];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int l32 = lane & 31, hh = lane >> 5;
+  const int kw = wave % KW, qw = wave / KW;
+  const int nqb = (p.N + BM - 1) / BM, grid = nqb * p.B * p.Hq;
+  const int block = blockIdx.y * gridDim.x + blockIdx.x;
+  if (block >= grid) return;
+  const Place pl(block, grid, nqb, p.B, p.cu_seqlens != nullptr);
+  const int b = pl.b, h = pl.h, hk = h / (p.Hq / p.Hkv);
+  const SeqView sv(p.cu_seqlens, p.T, p.N, b);
+  const int N = sv.N;
+  const int q0 = (nqb - 1 - pl.rank) * BM;
+  if (q0 >= N) return;  // packed: past the end of a shorter document
+  const int wq0 = q0 + 32 * qw, qrow = wq0 + l32;
+  const T* qg = static_cast<const T*>(p.q.ptr) + sv.off(p.q, b) + h * p.q.sh;
+  const T* kg = static_cast<const T*>(p.k.ptr) + sv.off(p.k, b) + hk * p.k.sh;
+  const T* vg = static_cast<const T*>(p.v.ptr) + sv.off(p.v, b) + hk * p.v.sh;
+  const float n = *p.n_ptr, c = p.scale * *p.b_ptr;
+  const uint32_t lds0 = lds_addr(smem);
+  const int64_t kss = p.k.ss * kUnits<T>, vss = p.v.ss * kUnits<T>;
+  const LoadLane llk(lane, wave, kss), llv(lane, wave, vss);
+  auto k_at = [&](int st, int i) { return lds0 + ((st & 1) * KW + i) * 2 * BB; };
+  auto load_stage = [&](int st) {
+#pragma unroll
+    for (int i = 0; i < KW; ++i) {
+      tile_load_async<M::LD, 32, 4>(kg, kss, st * BN + 32 * i, N, k_at(st, i), wave, llk);
+      tile_load_async<M::LD, 32, 4>(vg, vss, st * BN + 32 * i, N, k_at(st, i) + BB, wave, llv);
+    }
+  };
+  load_stage(0);
+  const M mat(lane);
+  typename M::frag qf[M::NF];
+#pragma unroll
+  for (int f = 0; f < M::NF; ++f)
+    qf[f] = qrow < N ? M::load(qg + qrow * p.q.ss, f, hh) : typename M::frag{};
+  f32x16 acc[ND];
+#pragma unroll
+  for (int d = 0; d < ND; ++d) acc[d] = f32x16{};
+  float m = -INFINITY, l = 0.f;
+  const int kv_end = CAUSAL ? min(N, q0 + BM) : N;
+  const int nst = (kv_end + BN - 1) / BN;
+  for (int st = 0; st < nst; ++st) {
+    __builtin_amdgcn_s_waitcnt(0);
+    __syncthreads();  // stage st has landed, stage st - 1 is consumed
+    if (st + 1 < nst) load_stage(st + 1);
+    const int k0 = st * BN + 32 * kw;
+    if (k0 >= N || wq0 >= N || (CAUSAL && k0 > wq0 + 31)) continue;
+    const f32x16 s = mat.scores(k_at(st, kw), qf);
+    float t[16];
+    float mx = -INFINITY;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) t[r] = n * ssa_sl(s[r], fmaf(c, fabsf(s[r]), 1.f));
+    if (k0 + 32 > N || (CAUSAL && k0 + 31 > wq0)) {
+      const int last = CAUSAL ? min(qrow, N - 1) : N - 1;
+#pragma unroll
+      for (int r = 0; r < 16; ++r)
+        if (k0 + crow(r, hh) > last) t[r] = -INFINITY;
+    }
+#pragma unroll
+    for (int r = 0; r < 16; ++r) mx = fmaxf(mx, t[r]);
+    mx = fmaxf(m, pair_max(mx));
+    const float base = mx == -INFINITY ? 0.f : mx;  // no key of this row yet: p = 0
+    if (__any(mx > m)) {                            // the running max moves: rescale what is summed so far
+      const float alpha = fast_exp2(m - base);
+      l *= alpha;
+#pragma unroll
+      for (int d = 0; d < ND; ++d) acc[d] *= alpha;
+      m = mx;
+    }
+    float sum = 0.f;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      t[r] = fast_exp2(t[r] - base + M::P_SHIFT);
+      sum += t[r];
+    }
+    l += sum;
+    mat.outer(k_at(st, kw) + BB, t, acc);
+  }
+  l = pair_sum(l);
+  if constexpr (KW > 1) {
+    __syncthreads();  // every wave is past the ring (no load in flight)
+    float* ml = reinterpret_cast<float*>(smem);  // [4 waves][m, l][32]
+    if (hh == 0) {
+      ml[(2 * wave) * 32 + l32] = m;
+      ml[(2 * wave + 1) * 32 + l32] = l;
+    }
+    __syncthreads();
+    const float own = m;
+    l = 0.f;
+#pragma unroll
+    for (int i = 0; i < KW; ++i) m = fmaxf(m, ml[2 * (qw * KW + i) * 32 + l32]);
+    const float base = m == -INFINITY ? 0.f : m;
+#pragma unroll
+    for (int i = 0; i < KW; ++i)
+      l += ml[(2 * (qw * KW + i) + 1) * 32 + l32] * fast_exp2(ml[2 * (qw * KW + i) * 32 + l32] - base);
+    const float alpha = fast_exp2(own - base);
+#pragma unroll
+    for (int d = 0; d < ND; ++d) acc[d] *= alpha;
+    merge_parts<ND, KW>(acc, reinterpret_cast<float*>(smem), qw, kw, lane);
+  }
+  if (kw == 0 && qrow < N) {
+    T* og = static_cast<T*>(const_cast<void*>(p.o.ptr)) + sv.off(p.o, b) + h * p.o.sh;
+    store_own<T, D>(acc, 1.f / l, og + qrow * p.o.ss, hh);  // every row has a key (causal: itself)
+    if (hh == 0) p.m[sv.mrow(b, h, p.Hq, p.T, p.N) + qrow] = m + (log2f(l) - M::P_SHIFT);
   }
 }
 
@@ -196,211 +423,292 @@ __global__ __launch_bounds__(256) void ssa_bwd_preprocess_f32_kernel(BwdParams p
 }
 
 // ---------------------------------------------------------------------------
-// dK, dV (+ dn / db partials) for 128 keys of one (batch, kv-head), in passes
-// of bwd_rows<D>() keys: P lanes per key, each holding its share of k, v, dK,
-// dV; Q / dO tiles of 32 rows,
-// with M and Delta, in LDS, over every q-head of the GQA group.  Per valid
-// pair, as in ssa_bwd.hip: P = exp2(n sL - M), dT = P (dP - Delta),
-// dS' = dT / (1 + c|x|), dV += P dO, dK += dS' q (scaled by scale n b at the
-// end), dn += ln2 dT sL, db += n scale dS' x.
-template <typename T, int D, bool CAUSAL>
-__global__ __launch_bounds__(bwd_threads<D>()) void ssa_bwd_dkdv_f32_kernel(BwdParams p) {
-  constexpr int P = bwd_parts<D>(), C4 = D / 4, CP = C4 / P, NT = bwd_threads<D>(), NWV = NT / 64;
-  constexpr int ROWS = bwd_rows<D>();
-  __shared__ f32x4 qs[kF32Tile * C4], dos[kF32Tile * C4];
-  __shared__ float ms[kF32Tile], dls[kF32Tile];
-  __shared__ float red[2][NWV];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, part = tid % P;
+// dK, dV (+ dn / db partials) for 128 keys of one (batch, kv-head): four
+// groups of 32 keys, QS waves each on alternate 32-query blocks; Q / dO blocks
+// with their M and Delta stream through LDS over every q-head of the GQA
+// group.  Per valid pair, as in ssa_bwd.hip: P = exp2(n sL - M), dT = P (dP -
+// Delta), dS' = dT / (1 + c|x|), dV += P dO, dK += dS' q (scaled by scale n b
+// at the end), dn += ln2 dT sL, db += n scale dS' x.
+template <typename T, int D, bool CAUSAL, bool DO_DK, bool DO_DV>
+__device__ __forceinline__ void dkdv_f32_body(const BwdParams& p, char* smem, float (*red)[8], int block, int grid) {
+  using M = Mat<T, D>;
+  using C = Cfg<T, D>;
+  constexpr int QS = C::QS, NWV = 4 * QS, BB = C::BB, ND = M::ND, STEP = 32 * QS;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int l32 = lane & 31, hh = lane >> 5;
+  const int qs = wave % QS, kg4 = wave / QS;
   const int nkb = dkdv_key_blocks(p.N);
-  const int kb = blockIdx.x % nkb, bhk = blockIdx.x / nkb;
-  const int b = bhk % p.B, hk = bhk / p.B;
+  const Place pl(block, grid, nkb, p.B, p.cu_seqlens != nullptr);
+  const int kb = pl.rank, b = pl.b, hk = pl.h, bhk = hk * p.B + b;
   const int G = p.Hq / p.Hkv;
   const SeqView sv(p.cu_seqlens, p.T, p.N, b);
   const int N = sv.N;
   const int64_t PP = static_cast<int64_t>(p.B) * p.Hkv * nkb;
-  if (kb * kF32Pair >= N) {  // packed: past the end of a shorter document
-    if (tid == 0) {
+  const int k0 = kb * 128;
+  if (k0 >= N) {  // packed: past the end of a shorter document
+    if (DO_DK && tid == 0) {
       p.partials[static_cast<int64_t>(bhk) * nkb + kb] = 0.f;
       p.partials[PP + static_cast<int64_t>(bhk) * nkb + kb] = 0.f;
     }
     return;
   }
+  const int k0w = k0 + 32 * kg4, key = k0w + l32;
   const T* kg = static_cast<const T*>(p.k.ptr) + sv.off(p.k, b) + hk * p.k.sh;
   const T* vg = static_cast<const T*>(p.v.ptr) + sv.off(p.v, b) + hk * p.v.sh;
   const float n = *p.n_ptr, bv = *p.b_ptr, c = p.scale * bv;
-  float dn_acc = 0.f, dn_c = 0.f, db_acc = 0.f, db_c = 0.f;  // Kahan sums (lanes with part == 0)
-  // ROWS keys at a time (one pass up to head dim 128, two at 256)
-  const int kend = min(N, kb * kF32Pair + kF32Pair);
-  for (int k0 = kb * kF32Pair; k0 < kend; k0 += ROWS) {
-    const int key = k0 + tid / P;
-    f32x4 kh[CP], vh[CP], dkh[CP], dvh[CP];
+  const uint32_t lds0 = lds_addr(smem);
+  const int64_t qss = p.q.ss * kUnits<T>, doss = p.dout.ss * kUnits<T>;
+  const LoadLane llq(lane, wave, qss), lld(lane, wave, doss);
+  const int qstart = CAUSAL ? k0 : 0;
+  const int nqs = (N - qstart + STEP - 1) / STEP, nst = G * nqs;
+  auto blk_at = [&](int st, int i) { return lds0 + (st & 1) * C::DKDV_STAGE + i * (2 * BB + 256); };
+  auto load_stage = [&](int st, int g, int q0) {
+    const int h = hk * G + g;
+    const T* qg = static_cast<const T*>(p.q.ptr) + sv.off(p.q, b) + h * p.q.sh;
+    const T* dog = static_cast<const T*>(p.dout.ptr) + sv.off(p.dout, b) + h * p.dout.sh;
+    const int64_t mr = sv.mrow(b, h, p.Hq, p.T, p.N);
 #pragma unroll
-    for (int c4 = 0; c4 < CP; ++c4) {
-      const int col = 4 * (part * CP + c4);
-      kh[c4] = key < N ? ld4(kg + key * p.k.ss + col) : f32x4{0.f, 0.f, 0.f, 0.f};
-      vh[c4] = key < N ? ld4(vg + key * p.v.ss + col) : f32x4{0.f, 0.f, 0.f, 0.f};
-      dkh[c4] = dvh[c4] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int i = 0; i < QS; ++i) {
+      const uint32_t at = blk_at(st, i);
+      tile_load_async<M::LD, 32, NWV>(qg, qss, q0 + 32 * i, N, at, wave, llq);
+      tile_load_async<M::LD, 32, NWV>(dog, doss, q0 + 32 * i, N, at + BB, wave, lld);
+      if (wave == NWV - 1 - i) pair32_load_async(p.m + mr, p.delta + mr, q0 + 32 * i, N, at + 2 * BB, lane);
     }
-    const int qstart = CAUSAL ? k0 : 0;
-    for (int g = 0; g < G; ++g) {
-      const int h = hk * G + g;
-      const T* qg = static_cast<const T*>(p.q.ptr) + sv.off(p.q, b) + h * p.q.sh;
-      const T* dog = static_cast<const T*>(p.dout.ptr) + sv.off(p.dout, b) + h * p.dout.sh;
-      const int64_t mr = sv.mrow(b, h, p.Hq, p.T, p.N);
-      for (int q0 = qstart; q0 < N; q0 += kF32Tile) {
-        __syncthreads();  // the previous tile is consumed
-        for (int idx = tid; idx < kF32Tile * C4; idx += NT) {
-          const int row = min(q0 + idx / C4, N - 1), c4 = idx % C4;
-          qs[idx] = ld4(qg + row * p.q.ss + 4 * c4);
-          dos[idx] = ld4(dog + row * p.dout.ss + 4 * c4);
-        }
-        if (tid < kF32Tile) {
-          const int row = min(q0 + tid, N - 1);
-          ms[tid] = p.m[mr + row];
-          dls[tid] = p.delta[mr + row];
-        }
-        __syncthreads();
-        const int qn = min(kF32Tile, N - q0);
-        for (int r = 0; r < qn; ++r) {
-          const int qi = q0 + r;
-          const f32x4* qrow = qs + r * C4 + part * CP;
-          const f32x4* drow = dos + r * C4 + part * CP;
-          const float s = sum_parts<P>(part_dot<CP>(kh, qrow));
-          const float dp = sum_parts<P>(part_dot<CP>(vh, drow));
-          if (key < N && (!CAUSAL || key <= qi)) {
-            const float u1 = fmaf(c, fabsf(s), 1.f);
-            const float sl = ssa_sl(s, u1);
-            const float pv = fast_exp2(fmaf(n, sl, -ms[r]));
-            const float dt = pv * (dp - dls[r]);
-            const float dsp = dt * fast_rcp(u1);
+  };
+  load_stage(0, 0, qstart);
+  const M mat(lane);
+  typename M::frag kf[M::NF], vf[M::NF];
 #pragma unroll
-            for (int c4 = 0; c4 < CP; ++c4) {
-              dvh[c4] += pv * drow[c4];
-              dkh[c4] += dsp * qrow[c4];
-            }
-            if (part == 0) {
-              const float y = dt * sl - dn_c, t = dn_acc + y;
-              dn_c = (t - dn_acc) - y;
-              dn_acc = t;
-              const float y2 = dsp * s - db_c, t2 = db_acc + y2;
-              db_c = (t2 - db_acc) - y2;
-              db_acc = t2;
-            }
-          }
+  for (int f = 0; f < M::NF; ++f) {
+    kf[f] = key < N ? M::load(kg + key * p.k.ss, f, hh) : typename M::frag{};
+    if constexpr (DO_DK) vf[f] = key < N ? M::load(vg + key * p.v.ss, f, hh) : typename M::frag{};
+  }
+  f32x16 dk[ND], dv[ND];
+#pragma unroll
+  for (int d = 0; d < ND; ++d) dk[d] = dv[d] = f32x16{};
+  float dn_acc = 0.f, dn_c = 0.f, db_acc = 0.f, db_c = 0.f;  // Kahan sums over the blocks' sums
+  WeightScale<M> ws;
+  int g = 0, q0 = qstart;  // of stage st
+  for (int st = 0; st < nst; ++st) {
+    __builtin_amdgcn_s_waitcnt(0);
+    __syncthreads();  // stage st has landed, stage st - 1 is consumed
+    const int qi0 = q0 + 32 * qs;
+    q0 += STEP;
+    if (q0 >= N) {
+      q0 = qstart;
+      ++g;
+    }
+    if (st + 1 < nst) load_stage(st + 1, g, q0);
+    if (qi0 >= N || k0w >= N || (CAUSAL && qi0 + 31 < k0w)) continue;
+    const uint32_t at = blk_at(st, qs);
+    const f32x16 s = mat.scores(at, kf);
+    f32x16 dp = f32x16{};
+    if constexpr (DO_DK) dp = mat.scores(at + BB, vf);
+    float pv[16], ds[16];
+    float tdn = 0.f, tdb = 0.f;
+    const bool masked = qi0 + 32 > N || k0w + 32 > N || (CAUSAL && k0w + 31 > qi0);  // wave-uniform
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const f32x4_t mv = lds_read_f4(at + 2 * BB + (8 * j + 4 * hh) * 4);
+      const f32x4_t dl = lds_read_f4(at + 2 * BB + 128 + (8 * j + 4 * hh) * 4);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int r = 4 * j + e;
+        const float x = s[r];
+        const float u1 = fmaf(c, fabsf(x), 1.f);
+        const float sl = ssa_sl(x, u1);
+        float w = fast_exp2(fmaf(n, sl, -mv[e]));
+        if (masked) {
+          const int qi = qi0 + crow(r, hh);
+          if (qi >= N || key >= N || (CAUSAL && key > qi)) w = 0.f;
+        }
+        pv[r] = w;
+        if constexpr (DO_DK) {
+          const float dt = w * (dp[r] - dl[e]);
+          ds[r] = dt * fast_rcp(u1);
+          tdn = fmaf(dt, sl, tdn);
+          tdb = fmaf(ds[r], x, tdb);
         }
       }
     }
-    if (key < N) {
-      const float ks_ = p.scale * n * bv;
+    if constexpr (DO_DV) {
+      if constexpr (M::F16) {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) pv[r] *= exp2f(M::P_SHIFT);
+      }
+      mat.outer(at + BB, pv, dv);
+    }
+    if constexpr (DO_DK) {
+      const float y = tdn - dn_c, t = dn_acc + y;
+      dn_c = (t - dn_acc) - y;
+      dn_acc = t;
+      const float y2 = tdb - db_c, t2 = db_acc + y2;
+      db_c = (t2 - db_acc) - y2;
+      db_acc = t2;
+      ws.apply(ds, dk);
+      mat.outer(at, ds, dk);
+    }
+  }
+  if constexpr (QS > 1) static_assert(!M::F16, "one weight scale per accumulator");
+  if constexpr (DO_DK) merge_parts<ND, QS>(dk, reinterpret_cast<float*>(smem), kg4, qs, lane);
+  if constexpr (DO_DV) merge_parts<ND, QS>(dv, reinterpret_cast<float*>(smem), kg4, qs, lane);
+  if (qs == 0 && key < N) {
+    if constexpr (DO_DK) {
       T* dkr = static_cast<T*>(const_cast<void*>(p.dk.ptr)) + sv.off(p.dk, b) + hk * p.dk.sh + key * p.dk.ss;
+      store_own<T, D>(dk, p.scale * n * bv * ws.inverse(), dkr, hh);
+    }
+    if constexpr (DO_DV) {
       T* dvr = static_cast<T*>(const_cast<void*>(p.dv.ptr)) + sv.off(p.dv, b) + hk * p.dv.sh + key * p.dv.ss;
+      store_own<T, D>(dv, exp2f(-M::P_SHIFT), dvr, hh);
+    }
+  }
+  if constexpr (DO_DK) {
+    // dn / db partial of this key block: lane butterfly, then the waves in order
+    float pdn = dn_acc - dn_c, pdb = db_acc - db_c;
 #pragma unroll
-      for (int c4 = 0; c4 < CP; ++c4) {
-        const int col = 4 * (part * CP + c4);
-        st4(dkr + col, dkh[c4] * ks_);
-        st4(dvr + col, dvh[c4]);
+    for (int off = 32; off > 0; off >>= 1) {
+      pdn += __shfl_xor(pdn, off, 64);
+      pdb += __shfl_xor(pdb, off, 64);
+    }
+    if (lane == 0) {
+      red[0][wave] = pdn;
+      red[1][wave] = pdb;
+    }
+    __syncthreads();
+    if (tid == 0) {
+      float sdn = 0.f, sdb = 0.f;
+#pragma unroll
+      for (int w = 0; w < NWV; ++w) {
+        sdn += red[0][w];
+        sdb += red[1][w];
       }
+      p.partials[static_cast<int64_t>(bhk) * nkb + kb] = kLn2 * sdn;
+      p.partials[PP + static_cast<int64_t>(bhk) * nkb + kb] = n * p.scale * sdb;
     }
   }
-  // dn / db partial of this key block: lane butterfly, then the waves in order
-  float pdn = dn_acc - dn_c, pdb = db_acc - db_c;
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) {
-    pdn += __shfl_xor(pdn, off, 64);
-    pdb += __shfl_xor(pdb, off, 64);
-  }
-  if (lane == 0) {
-    red[0][wave] = pdn;
-    red[1][wave] = pdb;
-  }
-  __syncthreads();
-  if (tid == 0) {
-    float sdn = 0.f, sdb = 0.f;
-#pragma unroll
-    for (int w = 0; w < NWV; ++w) {
-      sdn += red[0][w];
-      sdb += red[1][w];
-    }
-    p.partials[static_cast<int64_t>(bhk) * nkb + kb] = kLn2 * sdn;
-    p.partials[PP + static_cast<int64_t>(bhk) * nkb + kb] = n * p.scale * sdb;
+}
+
+template <typename T, int D, bool CAUSAL>
+__global__ __launch_bounds__((Cfg<T, D>::DKDV_THREADS)) void ssa_bwd_dkdv_f32_kernel(BwdParams p) {
+  using C = Cfg<T, D>;
+  __shared__ __attribute__((aligned(1024))) char smem[2 * C::DKDV_STAGE];
+  __shared__ float red[2][8];
+  if constexpr (C::ROLES) {
+    // dK workgroups (three products per block) before the lighter dV ones
+    const int half = gridDim.x / 2;
+    if (static_cast<int>(blockIdx.x) < half)
+      dkdv_f32_body<T, D, CAUSAL, true, false>(p, smem, red, blockIdx.x, half);
+    else
+      dkdv_f32_body<T, D, CAUSAL, false, true>(p, smem, red, blockIdx.x - half, half);
+  } else {
+    dkdv_f32_body<T, D, CAUSAL, true, true>(p, smem, red, blockIdx.x, gridDim.x);
   }
 }
 
 // ---------------------------------------------------------------------------
-// dQ for 128 query rows of one (batch, q-head), in passes of bwd_rows<D>()
-// rows: P lanes per row, each holding its share of q, dO and dQ; K / V tiles of 32 keys in LDS; the scores and dP
-// are recomputed (dQ += scale n b dS' k).
+// dQ for BM query rows of one (batch, q-head): K / V streamed BN keys a stage;
+// the scores and dP are recomputed (dQ += scale n b dS' k).
 template <typename T, int D, bool CAUSAL>
-__global__ __launch_bounds__(bwd_threads<D>()) void ssa_bwd_dq_f32_kernel(BwdParams p) {
-  constexpr int P = bwd_parts<D>(), C4 = D / 4, CP = C4 / P, NT = bwd_threads<D>(), ROWS = bwd_rows<D>();
-  __shared__ f32x4 ks[kF32Tile * C4], vs[kF32Tile * C4];
-  const int tid = threadIdx.x, part = tid % P;
-  const int nqb = (p.N + kF32Pair - 1) / kF32Pair;
-  const int qb = blockIdx.x % nqb, bh = blockIdx.x / nqb;
-  const int b = bh % p.B, h = bh / p.B, hk = h / (p.Hq / p.Hkv);
+__global__ __launch_bounds__(256) void ssa_bwd_dq_f32_kernel(BwdParams p) {
+  using M = Mat<T, D>;
+  using C = Cfg<T, D>;
+  constexpr int KW = C::KW, BM = C::BM, BN = C::BN, BB = C::BB, ND = M::ND;
+  __shared__ __attribute__((aligned(1024))) char smem[C::LDS_BYTES];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int l32 = lane & 31, hh = lane >> 5;
+  const int kw = wave % KW, qw = wave / KW;
+  const int nqb = (p.N + BM - 1) / BM, grid = nqb * p.B * p.Hq;
+  const int block = blockIdx.y * gridDim.x + blockIdx.x;
+  if (block >= grid) return;
+  const Place pl(block, grid, nqb, p.B, p.cu_seqlens != nullptr);
+  const int b = pl.b, h = pl.h, hk = h / (p.Hq / p.Hkv);
   const SeqView sv(p.cu_seqlens, p.T, p.N, b);
   const int N = sv.N;
-  if (qb * kF32Pair >= N) return;
+  const int q0 = (nqb - 1 - pl.rank) * BM;
+  if (q0 >= N) return;
+  const int wq0 = q0 + 32 * qw, qrow = wq0 + l32;
   const T* qg = static_cast<const T*>(p.q.ptr) + sv.off(p.q, b) + h * p.q.sh;
   const T* dog = static_cast<const T*>(p.dout.ptr) + sv.off(p.dout, b) + h * p.dout.sh;
   const T* kg = static_cast<const T*>(p.k.ptr) + sv.off(p.k, b) + hk * p.k.sh;
   const T* vg = static_cast<const T*>(p.v.ptr) + sv.off(p.v, b) + hk * p.v.sh;
   const int64_t mr = sv.mrow(b, h, p.Hq, p.T, p.N);
   const float n = *p.n_ptr, bv = *p.b_ptr, c = p.scale * bv;
-  // ROWS query rows at a time (one pass up to head dim 128, two at 256)
-  const int qend = min(N, qb * kF32Pair + kF32Pair);
-  for (int q0 = qb * kF32Pair; q0 < qend; q0 += ROWS) {
-    const int i = q0 + tid / P;
-    f32x4 qh[CP], doh[CP], dqh[CP];
+  const uint32_t lds0 = lds_addr(smem);
+  const int64_t kss = p.k.ss * kUnits<T>, vss = p.v.ss * kUnits<T>;
+  const LoadLane llk(lane, wave, kss), llv(lane, wave, vss);
+  auto k_at = [&](int st, int i) { return lds0 + ((st & 1) * KW + i) * 2 * BB; };
+  auto load_stage = [&](int st) {
 #pragma unroll
-    for (int c4 = 0; c4 < CP; ++c4) {
-      const int col = 4 * (part * CP + c4);
-      qh[c4] = i < N ? ld4(qg + i * p.q.ss + col) : f32x4{0.f, 0.f, 0.f, 0.f};
-      doh[c4] = i < N ? ld4(dog + i * p.dout.ss + col) : f32x4{0.f, 0.f, 0.f, 0.f};
-      dqh[c4] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int i = 0; i < KW; ++i) {
+      tile_load_async<M::LD, 32, 4>(kg, kss, st * BN + 32 * i, N, k_at(st, i), wave, llk);
+      tile_load_async<M::LD, 32, 4>(vg, vss, st * BN + 32 * i, N, k_at(st, i) + BB, wave, llv);
     }
-    const float mi = i < N ? p.m[mr + i] : 0.f, di = i < N ? p.delta[mr + i] : 0.f;
-    const int kv_end = CAUSAL ? min(N, q0 + ROWS) : N;
-    for (int k0 = 0; k0 < kv_end; k0 += kF32Tile) {
-      __syncthreads();  // the previous tile is consumed
-      for (int idx = tid; idx < kF32Tile * C4; idx += NT) {
-        const int row = min(k0 + idx / C4, N - 1), c4 = idx % C4;
-        ks[idx] = ld4(kg + row * p.k.ss + 4 * c4);
-        vs[idx] = ld4(vg + row * p.v.ss + 4 * c4);
-      }
-      __syncthreads();
-      const int kn = min(kF32Tile, kv_end - k0);
-      for (int j = 0; j < kn; ++j) {
-        const f32x4* krow = ks + j * C4 + part * CP;
-        const float s = sum_parts<P>(part_dot<CP>(qh, krow));
-        const float dp = sum_parts<P>(part_dot<CP>(doh, vs + j * C4 + part * CP));
-        if (i < N && (!CAUSAL || k0 + j <= i)) {
-          const float u1 = fmaf(c, fabsf(s), 1.f);
-          const float pv = fast_exp2(fmaf(n, ssa_sl(s, u1), -mi));
-          const float dsp = pv * (dp - di) * fast_rcp(u1);
+  };
+  load_stage(0);
+  const M mat(lane);
+  typename M::frag qf[M::NF], dof[M::NF];
 #pragma unroll
-          for (int c4 = 0; c4 < CP; ++c4) dqh[c4] += dsp * krow[c4];
-        }
-      }
-    }
-    if (i < N) {
-      const float qs_ = p.scale * n * bv;
-      T* dqr = static_cast<T*>(const_cast<void*>(p.dq.ptr)) + sv.off(p.dq, b) + h * p.dq.sh + i * p.dq.ss;
+  for (int f = 0; f < M::NF; ++f) {
+    qf[f] = qrow < N ? M::load(qg + qrow * p.q.ss, f, hh) : typename M::frag{};
+    dof[f] = qrow < N ? M::load(dog + qrow * p.dout.ss, f, hh) : typename M::frag{};
+  }
+  const float mi = qrow < N ? p.m[mr + qrow] : 0.f, di = qrow < N ? p.delta[mr + qrow] : 0.f;
+  f32x16 dq[ND];
 #pragma unroll
-      for (int c4 = 0; c4 < CP; ++c4) st4(dqr + 4 * (part * CP + c4), dqh[c4] * qs_);
+  for (int d = 0; d < ND; ++d) dq[d] = f32x16{};
+  WeightScale<M> ws;
+  const int kv_end = CAUSAL ? min(N, q0 + BM) : N;
+  const int nst = (kv_end + BN - 1) / BN;
+  for (int st = 0; st < nst; ++st) {
+    __builtin_amdgcn_s_waitcnt(0);
+    __syncthreads();  // stage st has landed, stage st - 1 is consumed
+    if (st + 1 < nst) load_stage(st + 1);
+    const int k0 = st * BN + 32 * kw;
+    if (k0 >= N || wq0 >= N || (CAUSAL && k0 > wq0 + 31)) continue;
+    const uint32_t at = k_at(st, kw);
+    const f32x16 s = mat.scores(at, qf), dp = mat.scores(at + BB, dof);
+    float ds[16];
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      const float x = s[r];
+      const float u1 = fmaf(c, fabsf(x), 1.f);
+      const float pv = fast_exp2(fmaf(n, ssa_sl(x, u1), -mi));
+      ds[r] = pv * (dp[r] - di) * fast_rcp(u1);
     }
+    if (k0 + 32 > N || wq0 + 32 > N || (CAUSAL && k0 + 31 > wq0)) {
+      const int last = qrow >= N ? -1 : (CAUSAL ? min(qrow, N - 1) : N - 1);
+#pragma unroll
+      for (int r = 0; r < 16; ++r)
+        if (k0 + crow(r, hh) > last) ds[r] = 0.f;
+    }
+    ws.apply(ds, dq);
+    mat.outer(at, ds, dq);
+  }
+  if constexpr (KW > 1) {
+    if constexpr (M::F16) {  // bring the sharing waves' sums to true scale first
+      const float inv = ws.inverse();
+#pragma unroll
+      for (int d = 0; d < ND; ++d) dq[d] *= inv;
+    }
+    merge_parts<ND, KW>(dq, reinterpret_cast<float*>(smem), qw, kw, lane);
+  }
+  if (kw == 0 && qrow < N) {
+    T* dqr = static_cast<T*>(const_cast<void*>(p.dq.ptr)) + sv.off(p.dq, b) + h * p.dq.sh + qrow * p.dq.ss;
+    store_own<T, D>(dq, p.scale * n * bv * (KW > 1 ? 1.f : ws.inverse()), dqr, hh);
   }
 }
 
-// One launch of KERNEL<T, DD, CAUSAL> with THREADS<DD>() threads.
-#define SSA_F32_LAUNCH(KERNEL, THREADS, T, DD, GRID, P, CAUSAL, S)                                 \
-  do {                                                                                             \
-    if (CAUSAL) hipLaunchKernelGGL((KERNEL<T, DD, true>), dim3(GRID), dim3(THREADS<DD>()), 0, S, P); \
-    else hipLaunchKernelGGL((KERNEL<T, DD, false>), dim3(GRID), dim3(THREADS<DD>()), 0, S, P);      \
+// One launch of KERNEL<T, DD, CAUSAL>.
+#define SSA_F32_LAUNCH(KERNEL, THREADS, T, DD, GRID, P, CAUSAL, S)                                     \
+  do {                                                                                                 \
+    if (CAUSAL) hipLaunchKernelGGL((KERNEL<T, DD, true>), GRID(T, DD), dim3(THREADS(T, DD)), 0, S, P); \
+    else hipLaunchKernelGGL((KERNEL<T, DD, false>), GRID(T, DD), dim3(THREADS(T, DD)), 0, S, P); \
   } while (0)
 
 // The head dims of each element type: fp32 at 16-256, bf16 / fp16 at 256
-// (their other head dims run on the matrix-core kernels).
+// (their other head dims run on the 16-bit kernels).
 #define SSA_F32_DISPATCH(KERNEL, THREADS, GRID, P, DTYPE, D, CAUSAL, S)                         \
   if (DTYPE == kDtypeF32) {                                                                     \
     switch (D) {                                                                                \
@@ -428,9 +736,19 @@ static void launch_pre(const BwdParams& p, hipStream_t s) {
 
 }  // namespace
 
+// A launch takes fewer than 2^32 threads along x: larger row grids (from 2^23
+// workgroups) fold over y.
+static dim3 row_grid(int n) {
+  const int y = (n + (1 << 23) - 1) >> 23;
+  return dim3((n + y - 1) / y, y);
+}
+#define SSA_F32_ROW_GRID(T, DD) row_grid((p.N + Cfg<T, DD>::BM - 1) / Cfg<T, DD>::BM * p.B * p.Hq)
+#define SSA_F32_KEY_GRID(T, DD) dim3(dkdv_key_blocks(p.N) * p.B * p.Hkv * (Cfg<T, DD>::ROLES ? 2 : 1))
+#define SSA_F32_THREADS(T, DD) 256
+#define SSA_F32_KEY_THREADS(T, DD) (Cfg<T, DD>::DKDV_THREADS)
+
 hipError_t launch_fwd_f32(const FwdParams& p, int dtype, int D, bool causal, hipStream_t s) {
-  const int grid = (p.N + kF32Rows - 1) / kF32Rows * p.B * p.Hq;
-  SSA_F32_DISPATCH(ssa_fwd_f32_kernel, fwd_threads, grid, p, dtype, D, causal, s)
+  SSA_F32_DISPATCH(ssa_fwd_f32_kernel, SSA_F32_THREADS, SSA_F32_ROW_GRID, p, dtype, D, causal, s)
   return hipGetLastError();
 }
 
@@ -456,14 +774,12 @@ hipError_t launch_bwd_preprocess_f32(const BwdParams& p, int dtype, int D, hipSt
 }
 
 hipError_t launch_bwd_dkdv_f32(const BwdParams& p, int dtype, int D, bool causal, hipStream_t s) {
-  const int grid = dkdv_key_blocks(p.N) * p.B * p.Hkv;
-  SSA_F32_DISPATCH(ssa_bwd_dkdv_f32_kernel, bwd_threads, grid, p, dtype, D, causal, s)
+  SSA_F32_DISPATCH(ssa_bwd_dkdv_f32_kernel, SSA_F32_KEY_THREADS, SSA_F32_KEY_GRID, p, dtype, D, causal, s)
   return hipGetLastError();
 }
 
 hipError_t launch_bwd_dq_f32(const BwdParams& p, int dtype, int D, bool causal, hipStream_t s) {
-  const int grid = (p.N + kF32Pair - 1) / kF32Pair * p.B * p.Hq;
-  SSA_F32_DISPATCH(ssa_bwd_dq_f32_kernel, bwd_threads, grid, p, dtype, D, causal, s)
+  SSA_F32_DISPATCH(ssa_bwd_dq_f32_kernel, SSA_F32_THREADS, SSA_F32_ROW_GRID, p, dtype, D, causal, s)
   return hipGetLastError();
 }
 

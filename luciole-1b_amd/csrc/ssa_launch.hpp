@@ -21,10 +21,10 @@ hipError_t launch_reduce_partials(const BwdParams& p, hipStream_t stream);
 
 hipError_t launch_decode(const DecodeParams& p, int dtype, int D, hipStream_t stream);
 
-// The fp32-arithmetic vector-ALU kernels (ssa_f32.hip) run fp32 inputs at
-// every head dim and bf16 / fp16 inputs at head dim 256; the matrix-core
-// kernels run bf16 / fp16 at 32, 64 and 128.  The vector-ALU backward does
-// not use the dS' workspace (its dQ recomputes).
+// The fp32-precision kernels (ssa_f32.hip) run fp32 inputs at every head dim
+// and bf16 / fp16 inputs at head dim 256; the 16-bit kernels run bf16 / fp16
+// at 32, 64 and 128.  The fp32-precision backward does not use the dS'
+// workspace (its dQ recomputes).
 constexpr int kDtypeF32 = 2;
 inline bool use_f32(int dtype, int D) { return dtype == kDtypeF32 || D == 256; }
 hipError_t launch_fwd_f32(const FwdParams& p, int dtype, int D, bool causal, hipStream_t stream);
