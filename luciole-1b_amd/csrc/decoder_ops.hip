@@ -85,8 +85,14 @@ bool aligned(const void* p, uintptr_t n) { return (reinterpret_cast<uintptr_t>(p
 // RMSNorm over rows of H fp32 values: r = (mean(x^2) + eps)^-1/2,
 // y = (x r) w in the output dtype.  Backward, with g = dy w and xh = x r:
 //   dx = r (g - xh sum(g xh) / H),  dw = sum over rows of dy xh.
+//
+// Both directions are HBM streams.  Forward: one workgroup per row (2048 x 2048
+// to bf16: 6.5 us; 25 MB, 5 us at the rate of a large copy).
 constexpr int kNormThreads = 256;
-constexpr int kNormBwdRows = 64;  // rows per backward workgroup (one dw partial each)
+constexpr int kNormMaxHidden = 4096;
+constexpr int kNormBwdRows = 64;  // rows per dw partial
+
+typedef float f4 __attribute__((ext_vector_type(4)));
 
 __device__ __forceinline__ float block_sum(float v, float* red) {
 #pragma unroll
@@ -123,74 +129,162 @@ __global__ __launch_bounds__(kNormThreads) void rmsnorm_fwd_kernel(const float* 
   if (threadIdx.x == 0) rstd[row] = r;
 }
 
-template <typename TG>
-__global__ __launch_bounds__(kNormThreads) void rmsnorm_bwd_kernel(const float* __restrict__ x,
-                                                                   const float* __restrict__ w,
-                                                                   const TG* __restrict__ dy,
-                                                                   const float* __restrict__ rstd,
-                                                                   float* __restrict__ dx, float* __restrict__ dw_part,
-                                                                   int T, int H) {
+// Backward in two kernels.  dx: a wave holds a whole row (lane l: columns
+// 4 (l + 64 k) .. + 3, k < K; K = 4, 8 or 16 covers hidden sizes up to 1024,
+// 2048 and 4096), so a row needs wave reductions only.  dw: a workgroup sums 64
+// rows of 256 columns (each wave 16 rows, all its loads in flight), one partial
+// per 64 rows.  One kernel that walked 64 rows per workgroup for both, a row at
+// a time with a block reduction between the halves of its work, filled 32 CUs
+// at 2048 rows and waited at its barriers.  bf16 dy, hidden 2048, the whole
+// backward: 2048 rows 89 -> 20 us (dx 11, dw partials 5, their sum 3.5; 42 MB
+// are 8 us at the rate of a large copy), 16384 rows 193 -> 102 us.  At 16384
+// rows one kernel for both that keeps a row per wave and the dw sums in
+// registers measured 73 us, at 2048 rows 37.
+// The row's dot product keeps the summation tree of 256 threads with columns
+// 4 (t + 256 j): four partial sums per lane (k % 4), a butterfly each, then
+// (d0 + d1) + (d2 + d3).
+constexpr int kNormDxWaves = 4;
+
+template <typename TG, int K>
+__global__ __launch_bounds__(kNormDxWaves * 64) void rmsnorm_dx_kernel(const float* __restrict__ x,
+                                                                       const float* __restrict__ w,
+                                                                       const TG* __restrict__ dy,
+                                                                       const float* __restrict__ rstd,
+                                                                       float* __restrict__ dx, int64_t row0, int T,
+                                                                       int H) {
   typedef float f4 __attribute__((ext_vector_type(4)));
-  constexpr int MAXC = 4;  // column groups of 4 per thread: H <= 4 * 4 * 256
-  __shared__ float red[4];
-  f4 acc[MAXC];
+  typedef typename Pack4<TG>::type g4;
+  const int lane = threadIdx.x & 63;
+  const int64_t row = static_cast<int64_t>(blockIdx.x) * kNormDxWaves + (threadIdx.x >> 6) + row0;
+  if (row >= T) return;
+  const float r = rstd[row];
+  const float* xr = x + row * H;
+  const TG* gr = dy + row * H;
+  f4 xv[K];
+  g4 gv[K];
 #pragma unroll
-  for (int k = 0; k < MAXC; ++k) acc[k] = f4{0.f, 0.f, 0.f, 0.f};
-  const int r0 = blockIdx.x * kNormBwdRows;
-  const int r1 = min(T, r0 + kNormBwdRows);
-  for (int row = r0; row < r1; ++row) {
-    const float* xr = x + static_cast<int64_t>(row) * H;
-    const TG* gr = dy + static_cast<int64_t>(row) * H;
-    const float r = rstd[row];
-    f4 xh[MAXC], g[MAXC], gy[MAXC];
-    float dot = 0.f;
+  for (int k = 0; k < K; ++k) {
+    const int c = 4 * (lane + 64 * k);
+    xv[k] = c < H ? *reinterpret_cast<const f4*>(xr + c) : f4{0.f, 0.f, 0.f, 0.f};
+    gv[k] = c < H ? *reinterpret_cast<const g4*>(gr + c) : g4{};
+  }
+  float dot[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int k = 0; k < MAXC; ++k) {
-      const int c = (threadIdx.x + k * kNormThreads) * 4;
-      if (c < H) {
-        const f4 v = *reinterpret_cast<const f4*>(xr + c);
-        const f4 wv = *reinterpret_cast<const f4*>(w + c);
+  for (int k = 0; k < K; ++k) {
+    const int c = 4 * (lane + 64 * k);
+    if (c < H) {
+      const f4 wv = *reinterpret_cast<const f4*>(w + c);
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          gy[k][e] = static_cast<float>(gr[c + e]);
-          xh[k][e] = v[e] * r;
-          g[k][e] = gy[k][e] * wv[e];
-          dot += g[k][e] * xh[k][e];
-        }
-      }
-    }
-    const float m = block_sum(dot, red) / H;
-    float* dxr = dx + static_cast<int64_t>(row) * H;
-#pragma unroll
-    for (int k = 0; k < MAXC; ++k) {
-      const int c = (threadIdx.x + k * kNormThreads) * 4;
-      if (c < H) {
-        f4 o;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          o[e] = r * (g[k][e] - xh[k][e] * m);
-          acc[k][e] += gy[k][e] * xh[k][e];
-        }
-        *reinterpret_cast<f4*>(dxr + c) = o;
-      }
+      for (int e = 0; e < 4; ++e)
+        dot[k & 3] = fmaf(static_cast<float>(gv[k][e]) * wv[e], xv[k][e] * r, dot[k & 3]);
     }
   }
-  float* part = dw_part + static_cast<int64_t>(blockIdx.x) * H;
 #pragma unroll
-  for (int k = 0; k < MAXC; ++k) {
-    const int c = (threadIdx.x + k * kNormThreads) * 4;
-    if (c < H) *reinterpret_cast<f4*>(part + c) = acc[k];
+  for (int off = 32; off > 0; off >>= 1) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) dot[i] += __shfl_xor(dot[i], off, 64);
+  }
+  const float m = ((dot[0] + dot[1]) + (dot[2] + dot[3])) / H;
+  float* dxr = dx + row * H;
+#pragma unroll
+  for (int k = 0; k < K; ++k) {
+    const int c = 4 * (lane + 64 * k);
+    if (c < H) {
+      const f4 wv = *reinterpret_cast<const f4*>(w + c);
+      f4 o;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) o[e] = r * fmaf(-(xv[k][e] * r), m, static_cast<float>(gv[k][e]) * wv[e]);
+      *reinterpret_cast<f4*>(dxr + c) = o;
+    }
   }
 }
 
-// dw[c] = sum over partials b (in order) of dw_part[b][c]
-__global__ __launch_bounds__(256) void rmsnorm_dw_kernel(const float* __restrict__ dw_part, float* __restrict__ dw,
-                                                         int nparts, int H) {
-  const int c = blockIdx.x * 256 + threadIdx.x;
-  if (c >= H) return;
+template <typename TG>
+__global__ __launch_bounds__(256) void rmsnorm_dw_part_kernel(const float* __restrict__ x,
+                                                              const TG* __restrict__ dy,
+                                                              const float* __restrict__ rstd,
+                                                              float* __restrict__ dw_part, int T, int H) {
+  typedef float f4 __attribute__((ext_vector_type(4)));
+  typedef typename Pack4<TG>::type g4;
+  __shared__ f4 part[4][64];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int ncol = (H + 255) / 256, group = blockIdx.x / ncol;  // 64 rows; the column blocks of a group together
+  const int c = 256 * (blockIdx.x % ncol) + 4 * lane;
+  const int64_t r0 = static_cast<int64_t>(group) * kNormBwdRows + wave * 16;
+  f4 acc = f4{0.f, 0.f, 0.f, 0.f};
+  if (c < H) {
+    f4 xv[16];
+    g4 gv[16];
+    float rs[16];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      const int64_t row = r0 + i < T ? r0 + i : T - 1;
+      xv[i] = *reinterpret_cast<const f4*>(x + row * H + c);
+      gv[i] = *reinterpret_cast<const g4*>(dy + row * H + c);
+      rs[i] = r0 + i < T ? rstd[row] : 0.f;
+    }
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (r0 + i < T) acc[e] = fmaf(static_cast<float>(gv[i][e]), xv[i][e] * rs[i], acc[e]);
+    }
+  }
+  part[wave][lane] = acc;
+  __syncthreads();
+  if (wave == 0 && c < H) {
+    f4 s = part[0][lane];
+#pragma unroll
+    for (int v = 1; v < 4; ++v) s += part[v][lane];
+    *reinterpret_cast<f4*>(dw_part + static_cast<int64_t>(group) * H + c) = s;
+  }
+}
+
+// dw[c] = sum over partials of dw_part[b][c]: 64 columns per workgroup, 16
+// waves on every 16th partial, their sums added in order (one thread per
+// column walked up to 256 partials one after another: 9 us at 32 of them).
+__global__ __launch_bounds__(1024) void rmsnorm_dw_kernel(const float* __restrict__ dw_part, float* __restrict__ dw,
+                                                          int nparts, int H) {
+  __shared__ float sum[16][64];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int c = blockIdx.x * 64 + lane;
   float s = 0.f;
-  for (int b = 0; b < nparts; ++b) s += dw_part[static_cast<int64_t>(b) * H + c];
+  if (c < H)
+    for (int b = wave; b < nparts; b += 16) s += dw_part[static_cast<int64_t>(b) * H + c];
+  sum[wave][lane] = s;
+  __syncthreads();
+  if (wave != 0 || c >= H) return;
+  s = 0.f;
+#pragma unroll
+  for (int v = 0; v < 16; ++v) s += sum[v][lane];
   dw[c] = s;
+}
+
+template <typename TG, int K>
+void launch_norm_dx(const ssa_rmsnorm_bwd_args* a, hipStream_t s) {
+  constexpr int kMaxRows = 1 << 25;  // 2^31 threads a launch
+  for (int64_t row0 = 0; row0 < a->rows; row0 += kMaxRows) {
+    const int n = static_cast<int>(a->rows - row0 < kMaxRows ? a->rows - row0 : kMaxRows);
+    hipLaunchKernelGGL((rmsnorm_dx_kernel<TG, K>), dim3((n + kNormDxWaves - 1) / kNormDxWaves),
+                       dim3(kNormDxWaves * 64), 0, s, static_cast<const float*>(a->x),
+                       static_cast<const float*>(a->weight), static_cast<const TG*>(a->dy), a->rstd, a->dx, row0,
+                       a->rows, a->hidden);
+  }
+}
+
+// dx, then the dw partials (their reads of x and dy find what dx's left in the
+// caches); K the smallest whose 256 K columns hold a row
+template <typename TG>
+void launch_norm_bwd(const ssa_rmsnorm_bwd_args* a, int nparts, hipStream_t s) {
+  if (a->hidden <= 1024)
+    launch_norm_dx<TG, 4>(a, s);
+  else if (a->hidden <= 2048)
+    launch_norm_dx<TG, 8>(a, s);
+  else
+    launch_norm_dx<TG, 16>(a, s);
+  hipLaunchKernelGGL((rmsnorm_dw_part_kernel<TG>), dim3((a->hidden + 255) / 256 * nparts), dim3(256), 0, s,
+                     static_cast<const float*>(a->x), static_cast<const TG*>(a->dy), a->rstd, a->workspace, a->rows,
+                     a->hidden);
 }
 
 // ---------------------------------------------------------------------------
@@ -301,7 +395,7 @@ __global__ __launch_bounds__(256) void xent_bwd_kernel(const T* __restrict__ log
 
 int32_t check_norm(const void* x, const void* w, const void* a, const void* b, int32_t T, int32_t H, int32_t dtype) {
   if (x == nullptr || w == nullptr || a == nullptr || b == nullptr) return SSA_OPS_ERR_NULL_POINTER;
-  if (T <= 0 || H <= 0 || H % 4 != 0 || H > 4 * 4 * kNormThreads) return SSA_OPS_ERR_SHAPE;
+  if (T <= 0 || H <= 0 || H % 4 != 0 || H > kNormMaxHidden) return SSA_OPS_ERR_SHAPE;
   if (dtype != 0 && dtype != 1 && dtype != 2) return SSA_OPS_ERR_DTYPE;
   if (!aligned(x, 16) || !aligned(w, 16)) return SSA_OPS_ERR_ALIGNMENT;
   return SSA_OPS_OK;
@@ -360,21 +454,13 @@ extern "C" int32_t ssa_rmsnorm_bwd(const ssa_rmsnorm_bwd_args* a, void* stream) 
   if (!aligned(a->dx, 16) || !aligned(a->workspace, 16) || !aligned(a->dy, 8)) return SSA_OPS_ERR_ALIGNMENT;
   hipStream_t s = static_cast<hipStream_t>(stream);
   const int nparts = static_cast<int>((static_cast<int64_t>(a->rows) + kNormBwdRows - 1) / kNormBwdRows);
-  const float* x = static_cast<const float*>(a->x);
-  const float* w = static_cast<const float*>(a->weight);
   switch (a->dy_dtype) {
-    case 0: hipLaunchKernelGGL(rmsnorm_bwd_kernel<__bf16>, dim3(nparts), dim3(kNormThreads), 0, s, x, w,
-                               static_cast<const __bf16*>(a->dy), a->rstd, a->dx, a->workspace, a->rows,
-                               a->hidden); break;
-    case 1: hipLaunchKernelGGL(rmsnorm_bwd_kernel<_Float16>, dim3(nparts), dim3(kNormThreads), 0, s, x, w,
-                               static_cast<const _Float16*>(a->dy), a->rstd, a->dx, a->workspace, a->rows,
-                               a->hidden); break;
-    default: hipLaunchKernelGGL(rmsnorm_bwd_kernel<float>, dim3(nparts), dim3(kNormThreads), 0, s, x, w,
-                                static_cast<const float*>(a->dy), a->rstd, a->dx, a->workspace, a->rows,
-                                a->hidden); break;
+    case 0: launch_norm_bwd<__bf16>(a, nparts, s); break;
+    case 1: launch_norm_bwd<_Float16>(a, nparts, s); break;
+    default: launch_norm_bwd<float>(a, nparts, s); break;
   }
   if (hipGetLastError() != hipSuccess) return SSA_OPS_ERR_LAUNCH;
-  hipLaunchKernelGGL(rmsnorm_dw_kernel, dim3((a->hidden + 255) / 256), dim3(256), 0, s, a->workspace, a->dweight,
+  hipLaunchKernelGGL(rmsnorm_dw_kernel, dim3((a->hidden + 63) / 64), dim3(1024), 0, s, a->workspace, a->dweight,
                      nparts, a->hidden);
   return hipGetLastError() == hipSuccess ? SSA_OPS_OK : SSA_OPS_ERR_LAUNCH;
 }
