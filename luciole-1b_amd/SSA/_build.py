@@ -1,7 +1,9 @@
-"""Build libssa_mi355x.so (gfx950) in-tree with hipcc.
+"""Build libssa_mi355x.so (gfx950) and the _ssa_native extension in-tree.
 
-Every ``csrc/*.hip`` file is compiled to an object in ``luciole-1b_amd/_build``
-(in parallel), then linked into ``luciole-1b_amd/SSA/libssa_mi355x.so``.  Run as
+Every ``csrc/*.hip`` file is compiled with hipcc to an object in
+``luciole-1b_amd/_build`` (in parallel), then linked into
+``luciole-1b_amd/SSA/libssa_mi355x.so``; ``csrc/torch_native.cpp`` (host code
+against PyTorch's headers) becomes ``SSA/_ssa_native.so``.  Run as
 ``python luciole-1b_amd/SSA/_build.py`` or through ``__graft_entry__.build()``.
 """
 
@@ -20,6 +22,8 @@ CSRC = ROOT_DIR / "csrc"
 BUILD_DIR = ROOT_DIR / "_build"
 LIB_NAME = "libssa_mi355x.so"
 LIB_PATH = PKG_DIR / LIB_NAME
+NATIVE_SRC = CSRC / "torch_native.cpp"
+NATIVE_PATH = PKG_DIR / "_ssa_native.so"
 ARCH = "gfx950"
 
 # -packed-fp32-ops: packed fp32 VALU forms are kept out of the generated code.
@@ -73,6 +77,29 @@ def _device_asm(src: Path, out: Path, extra: list[str]) -> None:
         raise RuntimeError(f"hipcc -S failed for {src.name}:\n{' '.join(cmd)}\n{res.stdout}\n{res.stderr}")
 
 
+def build_native() -> Path:
+    """Compile the launch layer's extension module against the installed PyTorch."""
+    import sysconfig
+
+    import torch
+    from torch.utils import cpp_extension
+
+    cxx = os.environ.get("CXX") or shutil.which("g++") or shutil.which("c++")
+    if cxx is None:
+        raise RuntimeError("no C++ compiler: the SSA launch extension cannot be built")
+    tmp = NATIVE_PATH.with_suffix(".so.tmp")
+    cmd = [cxx, "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-fvisibility=hidden",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}"]
+    cmd += [f"-isystem{d}" for d in cpp_extension.include_paths()] + [f"-isystem{sysconfig.get_path('include')}"]
+    cmd += [str(NATIVE_SRC), "-o", str(tmp)]
+    cmd += [f"-L{d}" for d in cpp_extension.library_paths()] + ["-ltorch_python", "-ltorch_cpu", "-lc10"]
+    res = subprocess.run(cmd, capture_output=True, text=True)
+    if res.returncode != 0:
+        raise RuntimeError(f"{cxx} failed for {NATIVE_SRC.name}:\n{' '.join(cmd)}\n{res.stdout}\n{res.stderr}")
+    os.replace(tmp, NATIVE_PATH)
+    return NATIVE_PATH
+
+
 def build_library(extra_flags: list[str] | None = None, jobs: int | None = None) -> Path:
     """Compile every HIP source, check the device assembly's wait states
     (SSA/_hazards.py) and link the shared library.  Returns its path."""
@@ -89,6 +116,7 @@ def build_library(extra_flags: list[str] | None = None, jobs: int | None = None)
     with cf.ThreadPoolExecutor(max_workers=jobs) as ex:
         futs = [ex.submit(_compile, s, o, extra) for s, o in zip(sources, objs)]
         futs += [ex.submit(_device_asm, s, a, extra) for s, a in zip(sources, asms)]
+        futs.append(ex.submit(build_native))
         for f in futs:
             f.result()
     sites = _hazards.check_files(asms)

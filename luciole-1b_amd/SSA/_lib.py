@@ -287,6 +287,40 @@ def lib() -> ctypes.CDLL:
     return _lib
 
 
+# The launch layer's extension module (csrc/torch_native.cpp), and the C ABI
+# entry points it calls, in the order its bind() takes them.
+NATIVE_PATH = Path(__file__).resolve().parent / "_ssa_native.so"
+_NATIVE_ENTRIES = ("ssa_fwd", "ssa_bwd", "ssa_varlen_fwd", "ssa_varlen_bwd", "ssa_decode", "ssa_bwd_partials_count",
+                   "ssa_bwd_ds_workspace_bytes", "ssa_varlen_bwd_ds_workspace_bytes", "ssa_decode_workspace_bytes")
+_native = None
+
+
+def native():
+    """Load (once) and return the extension module, bound to the library; raises
+    if it has not been built."""
+    global _native
+    if _native is not None:
+        return _native
+    handle = lib()
+    with _lock:
+        if _native is None:
+            if not NATIVE_PATH.exists():
+                raise RuntimeError(
+                    f"SSA launch extension not found at {NATIVE_PATH}; build it with "
+                    "`python luciole-1b_amd/SSA/_build.py` (or __graft_entry__.build())."
+                )
+            import importlib.util
+
+            import torch  # noqa: F401  (its libraries resolve the extension's symbols)
+
+            spec = importlib.util.spec_from_file_location("_ssa_native", NATIVE_PATH)
+            mod = importlib.util.module_from_spec(spec)
+            spec.loader.exec_module(mod)
+            mod.bind(*(ctypes.cast(getattr(handle, name), ctypes.c_void_p).value for name in _NATIVE_ENTRIES))
+            _native = mod
+    return _native
+
+
 def status_text(status: int) -> str:
     return lib().ssa_status_string(int(status)).decode()
 

@@ -96,6 +96,23 @@ def _pad_cols(t: torch.Tensor, width: int) -> torch.Tensor:
     return torch.nn.functional.pad(t, (0, width - t.shape[-1]))
 
 
+# Calls that the kernels can take as they are go through the extension module
+# (csrc/torch_native.cpp): it checks, allocates and launches in one step and
+# returns None for everything else, which then takes the Python path below.
+
+
+def _current():
+    """The current device and its current raw stream."""
+    dev = torch._C._cuda_getDevice()
+    return dev, torch._C._cuda_getCurrentRawStream(dev)
+
+
+def _native_result(r, what: str):
+    if type(r) is int:  # a library status
+        _lib.check(r, what)
+    return r
+
+
 def _check_inputs(q, k, v):
     if q.dim() != 4 or k.dim() != 4 or v.dim() != 4:
         raise ValueError("q, k, v must be 4-D [B, H, N, D] tensors")
@@ -121,6 +138,10 @@ def _padded_width(D: int, dtype: torch.dtype) -> int:
 
 def ssa_flash_attn_forward(q, k, v, softmax_scale, ssa_n, ssa_b, causal=True):
     """SSA attention forward.  Returns ``(out [B,Hq,N,D], m [B,Hq,N] fp32)``."""
+    if q.is_cuda:
+        r = _lib.native().fwd(q, k, v, softmax_scale, ssa_n, ssa_b, bool(causal), *_current())
+        if r is not None:
+            return _native_result(r, "ssa_fwd")
     B, Hq, Hkv, N, D = _check_inputs(q, k, v)
     w = _padded_width(D, q.dtype)
     if w:
@@ -151,6 +172,32 @@ def _has_ds_path(dtype: torch.dtype, head_dim: int) -> bool:
     return dtype != torch.float32 and head_dim <= 128
 
 
+# Workspaces up to this size are taken without asking for the device's
+# headroom: the allocator's statistics and the driver's free memory take about
+# 90 us, more than the kernels of a small problem, and this is a thousandth of
+# the card.  It is the call's last allocation, is free again when the call
+# returns, and where it fails dq recomputes the scores.
+_DS_UNASKED_BYTES = 256 << 20
+
+
+def _ds_mode(ds):
+    """The dS' policy of a call: 0 (never), -1 (always), or the byte cap."""
+    if ds is not None:
+        return -1 if ds else 0
+    mode = os.environ.get("SSA_BWD_DS", "auto").strip().lower()
+    if mode in ("0", "off", "false", "no"):
+        return 0
+    if mode in ("1", "on", "true", "yes"):
+        return -1
+    return max(0, int(os.environ.get("SSA_BWD_DS_MAX_BYTES", str(16 << 30))))
+
+
+def _ds_unasked(ds):
+    """The largest dS' workspace the extension module may take for this call."""
+    mode = _ds_mode(ds)
+    return min(mode, _DS_UNASKED_BYTES)
+
+
 def _device_headroom(device) -> int | None:
     """Bytes a new allocation on ``device`` can take without the caching
     allocator asking the driver for more than it has: the driver's free memory
@@ -171,18 +218,27 @@ def _use_ds_workspace(nbytes: int, head_dim: int, ds, device=None) -> bool:
     memory a training step needs; above either bound dq recomputes the scores
     instead).  ``head_dim`` is kept for callers; every head dim measured faster
     with the workspace."""
-    if ds is not None:
-        return bool(ds)
-    mode = os.environ.get("SSA_BWD_DS", "auto").strip().lower()
-    if mode in ("0", "off", "false", "no"):
-        return False
-    if mode in ("1", "on", "true", "yes"):
+    limit = _ds_mode(ds)
+    if limit < 0:
         return True
-    limit = int(os.environ.get("SSA_BWD_DS_MAX_BYTES", str(16 << 30)))
     if not 0 < nbytes <= limit:
         return False
+    if nbytes <= _DS_UNASKED_BYTES:
+        return True
     room = _device_headroom(device) if device is not None else None
     return room is None or nbytes <= room // 2
+
+
+def _ds_workspace(nbytes: int, head_dim: int, ds, device):
+    """The dS' workspace tensor of a backward, or None to recompute."""
+    if not _use_ds_workspace(nbytes, head_dim, ds, device):
+        return None
+    try:
+        return torch.empty(nbytes, device=device, dtype=torch.uint8)
+    except torch.OutOfMemoryError:
+        if _ds_mode(ds) < 0:
+            raise
+        return None
 
 
 class BackwardLaunch:
@@ -221,8 +277,7 @@ class BackwardLaunch:
         self.dn = torch.empty((), device=dev, dtype=torch.float32)
         self.db = torch.empty((), device=dev, dtype=torch.float32)
         ds_bytes = int(self.lib.ssa_bwd_ds_workspace_bytes(B, Hq, N, int(bool(causal))))
-        self.ds = (torch.empty(ds_bytes, device=dev, dtype=torch.uint8)
-                   if _has_ds_path(q.dtype, D) and _use_ds_workspace(ds_bytes, D, ds, dev) else None)
+        self.ds = _ds_workspace(ds_bytes, D, ds, dev) if _has_ds_path(q.dtype, D) else None
         self.device = dev
         self.args = _lib.BwdArgs(
             _t4(self.q), _t4(self.k), _t4(self.v), _t4(self.out), _t4(self.dout),
@@ -255,6 +310,11 @@ class BackwardLaunch:
 def ssa_flash_attn_backward(q, k, v, out, dout, m, softmax_scale, ssa_n, ssa_b, causal=True, ds=None):
     """SSA attention backward.  Returns ``(dq, dk, dv, dn, db)``; dn/db are 0-d fp32 tensors.
     ``ds``: keep dS' in a workspace (True / False; None: the ``SSA_BWD_DS`` policy)."""
+    if q.is_cuda:
+        r = _lib.native().bwd(q, k, v, out, dout, m, softmax_scale, ssa_n, ssa_b, bool(causal), _ds_unasked(ds),
+                              *_current())
+        if r is not None:
+            return _native_result(r, "ssa_bwd")
     D = q.shape[-1] if q.dim() == 4 else 0
     w = _padded_width(D, q.dtype)
     if w and tuple(out.shape) == tuple(q.shape) and tuple(dout.shape) == tuple(q.shape):
@@ -340,6 +400,11 @@ def ssa_flash_attn_varlen_forward(q, k, v, cu_seqlens, max_seqlen, softmax_scale
     """Packed-sequence forward.  q [T,Hq,D], k/v [T,Hkv,D], cu_seqlens [docs+1]
     (int32, on the device), max_seqlen = longest document.  Returns
     ``(out [T,Hq,D], m [Hq,T] fp32)``."""
+    if q.is_cuda:
+        r = _lib.native().varlen_fwd(q, k, v, cu_seqlens, max_seqlen, softmax_scale, ssa_n, ssa_b, bool(causal),
+                                     *_current())
+        if r is not None:
+            return _native_result(r, "ssa_varlen_fwd")
     cu, docs, T, Hq, Hkv, D, max_seqlen = _check_varlen_inputs(q, k, v, cu_seqlens, max_seqlen)
     w = _padded_width(D, q.dtype)
     if w:
@@ -367,6 +432,11 @@ def ssa_flash_attn_varlen_backward(q, k, v, out, dout, m, cu_seqlens, max_seqlen
                                    causal=True, ds=None):
     """Packed-sequence backward.  Returns ``(dq, dk, dv, dn, db)``; dn/db are 0-d fp32 tensors.
     ``ds``: keep dS' in a workspace (True / False; None: the ``SSA_BWD_DS`` policy)."""
+    if q.is_cuda:
+        r = _lib.native().varlen_bwd(q, k, v, out, dout, m, cu_seqlens, max_seqlen, softmax_scale, ssa_n, ssa_b,
+                                     bool(causal), _ds_unasked(ds), *_current())
+        if r is not None:
+            return _native_result(r, "ssa_varlen_bwd")
     cu, docs, T, Hq, Hkv, D, max_seqlen = _check_varlen_inputs(q, k, v, cu_seqlens, max_seqlen)
     if tuple(out.shape) != tuple(q.shape) or tuple(dout.shape) != tuple(q.shape) or out.dtype != q.dtype:
         raise ValueError("out and dout must have the shape (and out the dtype) of q")
@@ -394,8 +464,7 @@ def ssa_flash_attn_varlen_backward(q, k, v, out, dout, m, cu_seqlens, max_seqlen
     dn = torch.empty((), device=dev, dtype=torch.float32)
     db = torch.empty((), device=dev, dtype=torch.float32)
     ds_bytes = int(lib.ssa_varlen_bwd_ds_workspace_bytes(docs, Hq, max_seqlen, T, int(bool(causal))))
-    ds_ws = (torch.empty(ds_bytes, device=dev, dtype=torch.uint8)
-             if ds_bytes > 0 and _has_ds_path(q.dtype, D) and _use_ds_workspace(ds_bytes, D, ds, dev) else None)
+    ds_ws = _ds_workspace(ds_bytes, D, ds, dev) if ds_bytes > 0 and _has_ds_path(q.dtype, D) else None
     dense = _lib.BwdArgs(
         _t3(q), _t3(k), _t3(v), _t3(out), _t3(dout), _t3(dq), _t3(dk), _t3(dv),
         m.data_ptr(), delta.data_ptr(), partials.data_ptr(), dn.data_ptr(), db.data_ptr(),
@@ -466,6 +535,11 @@ def ssa_decode_attention(q, k_cache, v_cache, cache_seqlens, softmax_scale, ssa_
     (training/train/train_ssa_triton/generate_triton.py:315-331).
     """
     squeeze = q.dim() == 3
+    if squeeze and q.is_cuda and not return_m:
+        r = _lib.native().decode(q, k_cache, v_cache, cache_seqlens, softmax_scale, ssa_n, ssa_b, num_splits,
+                                 *_current())
+        if r is not None:
+            return _native_result(r, "ssa_decode")[0]
     q4 = q.unsqueeze(2) if squeeze else q
     if q4.dim() != 4 or q4.shape[2] != 1:
         raise ValueError("q must be [B, Hq, D] or [B, Hq, 1, D]")
