@@ -3,10 +3,10 @@
 // Replaces _ssa_attn_fwd / _ssa_attn_fwd_inner
 // (training/train/train_ssa_triton/SSA/ssa_triton_kernel.py:40-260).
 //
-// One workgroup = 8 waves = 256 query rows of one (batch, q-head); each wave
-// owns 32 query rows, two waves share a SIMD.  K/V tiles of 64 keys live in
-// four LDS buffers filled by direct-to-LDS loads two tiles ahead and shared by
-// the 8 waves (one barrier per tile).  Everything is computed transposed so
+// One workgroup = 4 or 8 waves = 128 or 256 query rows of one (batch, q-head);
+// each wave owns 32 query rows, two waves share a SIMD.  K/V tiles of 64 keys
+// live in four LDS buffers filled by direct-to-LDS loads two tiles ahead and
+// shared by the waves (one barrier per tile).  Everything is computed transposed so
 // that a query row lives in a single lane pair (l, l+32):
 //   S^T = K Q^T      (A = K rows from LDS, B = Q^T fragment held in registers)
 //   O^T += V^T P^T   (A = V^T via LDS transpose reads, B = P^T straight from S^T)
@@ -75,9 +75,9 @@ struct FwdTile {
 };
 
 // ---------------------------------------------------------------------------
-// Software-pipelined forward.  One workgroup = 8 waves = 256 query rows (32
-// per wave), two waves per SIMD; K/V tiles of 64 keys in NB = 4 LDS buffers
-// shared by all 8 waves, one barrier per tile.  Iteration i of a wave issues
+// Software-pipelined forward.  One workgroup = NW waves = 32 NW query rows, two
+// waves per SIMD; K/V tiles of 64 keys in NB = 4 LDS buffers shared by the
+// waves, one barrier per tile.  Iteration i of a wave issues
 //   MFMA : S_{i+1} = K_{i+1} Q^T   and   O^T += V_{i-1}^T P_{i-1}^T
 //   VALU : SSA transform, online max / sum and P_i = exp2(...) of S_i
 // with no dependence between the two streams inside the iteration, so each
@@ -87,11 +87,10 @@ struct FwdTile {
 // has been added at the old scale).  Tile t is loaded at the start of
 // iteration t - 2 (its buffer last held tile t - 4, whose V was last read in
 // iteration t - 3) and must be complete at the start of iteration t - 1.
-template <typename T, int D, bool CAUSAL, bool NPOS>
-__device__ __forceinline__ void fwd_sp_body(const FwdParams& p, const FwdPlan<D, CAUSAL>& pl, char* smem) {
+template <typename T, int D, bool CAUSAL, bool NPOS, class Plan>
+__device__ __forceinline__ void fwd_sp_body(const FwdParams& p, const Plan& pl, char* smem) {
   typedef FwdTile<T, D> FT;
   typedef typename FT::v8 v8;
-  using Plan = FwdPlan<D, CAUSAL>;
   constexpr int BM = Plan::BM, BN = Plan::BN, NW = Plan::NW, NB = Plan::NB;
   constexpr int TILE = Plan::TILE, BUF = Plan::BUF;
   constexpr int ND16 = D / 16, ND32 = D / 32;
@@ -428,23 +427,44 @@ __device__ __forceinline__ void fwd_sp_body(const FwdParams& p, const FwdPlan<D,
 
 }  // namespace
 
-template <typename T, int D, bool CAUSAL>
-__global__ __launch_bounds__(512) void ssa_fwd_kernel(FwdParams p) {
-  using Plan = FwdPlan<D, CAUSAL>;
+template <typename T, int D, bool CAUSAL, int NW>
+__global__ __launch_bounds__(NW * 64, D < 128 || NW == 8 ? 2 : 1) void ssa_fwd_kernel(FwdParams p) {
+  using Plan = FwdPlan<D, CAUSAL, NW>;
   __shared__ __attribute__((aligned(1024))) char smem[Plan::LDS_BYTES];
   const Plan pl(p, blockIdx.x, gridDim.x);
   if (pl.empty()) return;  // packed: past the end of a shorter document
   if (*p.n_ptr >= 0.f)
-    fwd_sp_body<T, D, CAUSAL, true>(p, pl, smem);
+    fwd_sp_body<T, D, CAUSAL, true, Plan>(p, pl, smem);
   else
-    fwd_sp_body<T, D, CAUSAL, false>(p, pl, smem);
+    fwd_sp_body<T, D, CAUSAL, false, Plan>(p, pl, smem);
 }
 
+template <typename T, int D, bool CAUSAL, int NW>
+static hipError_t launch_fwd_nw(const FwdParams& p, hipStream_t stream) {
+  const int grid = FwdPlan<D, CAUSAL, NW>::grid(p);
+  hipLaunchKernelGGL((ssa_fwd_kernel<T, D, CAUSAL, NW>), dim3(grid), dim3(NW * 64), 0, stream, p);
+  return hipGetLastError();
+}
+
+// Waves per workgroup.  Each wave's tiles, and so its results, are the same
+// either way.  Up to head dim 64 the four buffers of a 4-wave workgroup take at
+// most 64 KB and two or three workgroups share a CU: their barriers are
+// independent, grids below one 256-row workgroup per CU spread over twice the
+// CUs, and the finer blocks balance (us, 8 -> 4 waves: 4 x 32/8 x 4096 x 64
+// causal 458 -> 427, full 778 -> 752; 2 x 16 x 1000 x 64 full 32 -> 23; 1 x 32/8
+// x 777 x 64 25.0 -> 19.2; 4 x 16 x 4096 x 32 204 -> 185; of 50 shapes the worst
+// is +4 %, 47 -> 48 at 1 x 28/4 x 2048 x 32).  At head dim 128 a workgroup has
+// the CU's LDS for itself, so four waves pay only while every 128-row
+// workgroup gets a CU of its own (256): 1 x 16 x 2048 61.7 -> 46.1, 1 x 32/8 x
+// 777 30.5 -> 24.2; at 288 to 512 workgroups they measured -25 to +18 %, above
+// 1024 +24 % (4 x 16 x 4096 308 -> 384).
+constexpr int kFwdCus = 256;
 template <typename T, int D, bool CAUSAL>
 static hipError_t launch_fwd_t(const FwdParams& p, hipStream_t stream) {
-  const int grid = FwdPlan<D, CAUSAL>::grid(p);
-  hipLaunchKernelGGL((ssa_fwd_kernel<T, D, CAUSAL>), dim3(grid), dim3(512), 0, stream, p);
-  return hipGetLastError();
+  if constexpr (D >= 128) {
+    if (FwdPlan<D, CAUSAL, 4>::grid(p) > kFwdCus) return launch_fwd_nw<T, D, CAUSAL, 8>(p, stream);
+  }
+  return launch_fwd_nw<T, D, CAUSAL, 4>(p, stream);
 }
 
 template <typename T>

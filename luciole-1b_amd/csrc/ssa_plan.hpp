@@ -50,12 +50,12 @@ struct StepWalk {
 };
 
 // ----------------------------------------------------------------------------
-// Forward (ssa_fwd.hip): a workgroup of 8 waves on 256 queries of (b, h); K
-// and V tiles of 64 rows in a ring of NB buffers (tile t: K at buf(t), V at
-// buf(t) + TILE).
-template <int D, bool CAUSAL>
+// Forward (ssa_fwd.hip): a workgroup of 4 or 8 waves on 32 queries each of
+// (b, h); K and V tiles of 64 rows in a ring of NB buffers (tile t: K at
+// buf(t), V at buf(t) + TILE).
+template <int D, bool CAUSAL, int WAVES = 8>
 struct FwdPlan {
-  static constexpr int BM = 256, BN = 64, NW = 8, NB = 4;
+  static constexpr int NW = WAVES, BM = 32 * NW, BN = 64, NB = 4;
   static constexpr int TILE = BN * D * 2;  // one K (or V) tile
   static constexpr int BUF = 2 * TILE;     // K_t then V_t
   static constexpr int LDS_BYTES = NB * BUF;

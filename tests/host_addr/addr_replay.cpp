@@ -469,9 +469,9 @@ bool replay_block(const Case& c, int block, int grid) {
 }
 
 // ---------------------------------------------------------------------------
-template <int D, bool CAUSAL>
+template <int D, bool CAUSAL, int NW>
 void run_fwd(Problem& P) {
-  using Plan = FwdPlan<D, CAUSAL>;
+  using Plan = FwdPlan<D, CAUSAL, NW>;
   const FwdParams& p = P.fp;
   const int grid = Plan::grid(p);
   Replay R;
@@ -817,7 +817,8 @@ void run_decode(int B, int Hq, int Hkv, int cap, int splits_req, const std::vect
 template <int D, bool CAUSAL>
 void run_case_dc(Problem& P) {
   const bool sampled = P.c.sample > 0;
-  run_fwd<D, CAUSAL>(P);
+  run_fwd<D, CAUSAL, 8>(P);
+  run_fwd<D, CAUSAL, 4>(P);
   run_dq<D, CAUSAL>(P);
   // dK/dV in both address forms (the launcher picks OFF32 when dkdv_off32
   // holds), each followed by the dS' K pass on its workspace
