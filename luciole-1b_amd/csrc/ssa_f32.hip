@@ -1,7 +1,6 @@
-// SSA attention forward and backward with every product and sum kept in fp32
-// precision, on the matrix cores: the kernels of fp32 inputs at every head
-// dim, and of bf16 / fp16 inputs at head dim 256 (the kernels of ssa_fwd.hip
-// and ssa_bwd*.hip cover bf16 / fp16 at 32, 64 and 128).
+// SSA attention forward and backward of fp32 inputs at every head dim, on the
+// matrix cores, with every product and sum in fp32 (bf16 / fp16: ssa_fwd.hip,
+// ssa_bwd*.hip and, at head dim 256, ssa_d256.hip).
 //
 // The reference runs its Triton kernels on fp32 tensors with fp32 operands in
 // the dot products (MATMUL_PRECISION = tl.float32,
@@ -24,11 +23,7 @@
 //           rows crow(r, hh);
 //   outer:  acc^T += X_streamed^T w, w the 16 weights (P or dS') of the lane's
 //           own row, straight from the accumulator they were computed in.
-// fp32: v_mfma_f32_32x32x2_f32, whose products and sums are fp32.  bf16 / fp16
-// at head dim 256: the score products take the inputs as they are (exact in
-// fp32), and the weights, which are fp32, go in as the sum of two 16-bit
-// halves (w = hi + lo, relative error 2^-17 in bf16, 2^-22 in fp16), each
-// multiplied on the matrix cores, so no probability is rounded to 16 bits.
+// Both run on v_mfma_f32_32x32x2_f32, whose products and sums are fp32.
 //
 // What bounds it: an fp32 MFMA takes 64 cycles for 4096 FLOPs, so the fp32
 // kernels run at the rate of the matrix cores' fp32 form (138 TFLOP/s in a
@@ -37,98 +32,19 @@
 // at a time) up to head dim 128, so that a workgroup owns 32 or 64 rows: a
 // grid of one sequence then fills the chip, and causal blocks balance.
 // Measured (us, the earlier vector-ALU kernels -> these): fp32, B = 1, H = 16,
-// N = 1024, D = 64 causal: forward 376 -> 42, dK/dV 498 -> 144, dQ 380 -> 51;
-// bf16, B = 1, H = 16, N = 2048, D = 256 causal: 3792 -> 126, 4622 -> 252,
-// 4332 -> 126.
-#include "ssa_common.hpp"
-#include "ssa_launch.hpp"
-#include "ssa_tile.hpp"
+// N = 1024, D = 64 causal: forward 376 -> 42, dK/dV 498 -> 144, dQ 380 -> 51.
+#include "ssa_rows.hpp"
 
 namespace ssa {
 
 namespace {
 
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-
-// Four consecutive elements of T as fp32 (16-byte or 8-byte aligned: columns
-// are multiples of 4, rows 16-byte aligned), and back.
-__device__ __forceinline__ f32x4 ld4(const float* p) { return *reinterpret_cast<const f32x4*>(p); }
-__device__ __forceinline__ void st4(float* p, f32x4 v) { *reinterpret_cast<f32x4*>(p) = v; }
-template <typename T>
-__device__ __forceinline__ f32x4 ld4(const T* p) {
-  typedef T t4 __attribute__((ext_vector_type(4)));
-  const t4 x = *reinterpret_cast<const t4*>(p);
-  return f32x4{static_cast<float>(x[0]), static_cast<float>(x[1]), static_cast<float>(x[2]),
-               static_cast<float>(x[3])};
-}
-template <typename T>
-__device__ __forceinline__ void st4(T* p, f32x4 v) {
-  typedef T t4 __attribute__((ext_vector_type(4)));
-  *reinterpret_cast<t4*>(p) = t4{static_cast<T>(v[0]), static_cast<T>(v[1]), static_cast<T>(v[2]),
-                                 static_cast<T>(v[3])};
-}
-
-// sL = sign(x) log2(1 + c|x|) for a raw score x = q.k, c = scale b; u1 = 1 + c|x|
-__device__ __forceinline__ float ssa_sl(float x, float u1) { return copysignf(fast_log2(u1), x); }
-
 // The two matrix operations on a streamed block of 32 rows x D in LDS, stored
 // in the block-chunk-major layout of ssa_tile.hpp (LD: its width in 16-bit
 // columns, so fp32 blocks are 2 D wide and the same loaders move them).
-template <typename T, int D>
-struct Mat {  // bf16 / fp16
-  static constexpr int LD = D, BLOCK = BlockLayout<LD>::BLOCK, ND = D / 32, NF = D / 16;
-  // fp16 holds 2^-24 .. 65504: probabilities (at most 1) are scaled up so that
-  // the halves of all that matter stay normal; bf16 has fp32's range.
-  static constexpr bool F16 = sizeof(T) == 2 && !__is_same(T, __bf16);
-  static constexpr float P_SHIFT = F16 ? 12.f : 0.f;
-  typedef typename Vec8<T>::type frag;
-  typedef T v4 __attribute__((ext_vector_type(4)));
-  RowBase<LD> rb;
-  TrBase<LD> tb;
-  __device__ __forceinline__ explicit Mat(int lane) : rb(lane & 31, lane >> 5), tb(lane) {}
-  // fragment f of the row at `row`: columns 16 f + 8 hh + (0..7)
-  __device__ static __forceinline__ frag load(const T* row, int f, int hh) {
-    return load16<frag>(row + 16 * f + 8 * hh);
-  }
-  __device__ __forceinline__ f32x16 scores(uint32_t lds, const frag* own) const {
-    const RowBase<LD> r = at_tile(rb, lds);
-    f32x16 s = f32x16{};
-#pragma unroll
-    for (int f = 0; f < NF; ++f) s = mfma32(tile_read_row<LD, frag>(r, 0, f), own[f], s);
-    return s;
-  }
-  __device__ __forceinline__ void outer(uint32_t lds, const float* w, f32x16* acc) const {
-    const TrBase<LD> t = at_tile(tb, lds);
-    frag hi[2], lo[2];
-#pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      const T h = static_cast<T>(w[r]);
-      hi[r >> 3][r & 7] = h;
-      lo[r >> 3][r & 7] = static_cast<T>(w[r] - static_cast<float>(h));
-    }
-#pragma unroll
-    for (int ks = 0; ks < 2; ++ks) {
-#pragma unroll
-      for (int d0 = 0; d0 < ND; d0 += 2) {
-        frag a[2];
-#pragma unroll
-        for (int i = 0; i < 2; ++i)
-          a[i] = __builtin_shufflevector(tile_read_tr<LD, v4>(t, 0, ks, 0, d0 + i),
-                                         tile_read_tr<LD, v4>(t, 0, ks, 1, d0 + i), 0, 1, 2, 3, 4, 5, 6, 7);
-#pragma unroll
-        for (int i = 0; i < 2; ++i) acc[d0 + i] = mfma32(a[i], hi[ks], acc[d0 + i]);
-#pragma unroll
-        for (int i = 0; i < 2; ++i) acc[d0 + i] = mfma32(a[i], lo[ks], acc[d0 + i]);
-      }
-    }
-  }
-};
-
 template <int D>
-struct Mat<float, D> {
+struct Mat {
   static constexpr int LD = 2 * D, BLOCK = BlockLayout<LD>::BLOCK, ND = D >= 32 ? D / 32 : 1, NF = D / 8;
-  static constexpr bool F16 = false;
-  static constexpr float P_SHIFT = 0.f;
   typedef f32x4 frag;
   RowBase<LD> rb;
   uint32_t ob[2];
@@ -172,49 +88,13 @@ struct Mat<float, D> {
   }
 };
 
-// Weights (dS') of any size on the fp16 halves: a power of two per wave, set by
-// the first block with a nonzero weight and lowered (exactly) whenever a larger
-// one comes, keeps the largest weight seen below 2^15; the accumulators hold
-// the scaled sums.  Nothing on bf16 and fp32.
-template <typename M>
-struct WeightScale {
-  float s = 0.f;
-  __device__ __forceinline__ void apply(float* w, f32x16* acc) {
-    if constexpr (M::F16) {
-      float a = 0.f;
-#pragma unroll
-      for (int r = 0; r < 16; ++r) a = fmaxf(a, fabsf(w[r]));
-      if (__any(a * s > 32768.f || (s == 0.f && a > 0.f))) {  // wave-uniform
-#pragma unroll
-        for (int off = 32; off > 0; off >>= 1) a = fmaxf(a, __shfl_xor(a, off, 64));
-        // 2^14 / 2^floor(log2 a), at most 2^60
-        int ex = 0;
-        (void)frexpf(a, &ex);
-        const float sn = ldexpf(1.f, min(15 - ex, 60));
-        if (s != 0.f) {
-          const float f = sn / s;
-#pragma unroll
-          for (int d = 0; d < M::ND; ++d) acc[d] *= f;
-        }
-        s = sn;
-      }
-#pragma unroll
-      for (int r = 0; r < 16; ++r) w[r] *= s;
-    }
-  }
-  __device__ __forceinline__ float inverse() const {
-    if constexpr (M::F16) return s != 0.f ? 1.f / s : 0.f;
-    return 1.f;
-  }
-};
-
 // Streamed blocks per stage (= waves that share 32 owned rows) of the forward
 // and dQ, and of dK/dV (whose workgroups own 128 keys, the unit of the dn / db
 // partials).  A stage holds two blocks (K and V, or Q and dO) per kw, twice
 // buffered, in at most 128 KB of LDS.
-template <typename T, int D>
+template <int D>
 struct Cfg {
-  static constexpr int BB = Mat<T, D>::BLOCK;
+  static constexpr int BB = Mat<D>::BLOCK;
   static constexpr int KW = 4 * BB <= 32768 ? 4 : (BB <= 16384 ? 2 : 1);
   static constexpr int QW = 4 / KW;  // waves on different rows (forward, dQ): 32 QW rows per workgroup
   static constexpr int BM = 32 * QW, BN = 32 * KW;
@@ -228,69 +108,15 @@ struct Cfg {
   static constexpr int DKDV_STAGE = QS * (2 * BB + 256);  // Q, dO, M[32], Delta[32] per block
 };
 
-template <typename T>
-constexpr int kUnits = sizeof(T) / 2;  // 16-bit units per element (the tile loaders' strides)
-
-// A workgroup's place in a grid of nblk blocks of rows per (sequence, head):
-// XCD-contiguous, the heaviest blocks (rank 0) of a pair of heads first, as
-// FwdPlan and DkdvPlan.
-struct Place {
-  int rank, b, h;
-  __device__ __forceinline__ Place(int block, int grid, int nblk, int B, bool packed) {
-    int hb;
-    dispatch_order(xcd_remap(block, grid), grid / nblk, nblk, packed ? 1 : kOrderGroup, hb, rank);
-    b = hb % B;
-    h = hb / B;
-  }
-};
-
-// Sum (or with `scale` the rescaled sum) of the accumulators of the waves that
-// share owned rows, in the first of them (part == 0): the others leave theirs
-// in LDS, element-major so that every access is contiguous.  Called by every
-// wave; `lds` is free (all waves past their last read of the ring).
-template <int ND, int KW>
-__device__ __forceinline__ void merge_parts(f32x16* acc, float* lds, int group, int part, int lane) {
-  if constexpr (KW > 1) {
-    __syncthreads();
-    float* mine = lds + static_cast<size_t>((group * (KW - 1) + part - 1) * ND * 16 * 64) + lane;
-    if (part > 0) {
-#pragma unroll
-      for (int i = 0; i < ND * 16; ++i) mine[i * 64] = acc[i >> 4][i & 15];
-    }
-    __syncthreads();
-    if (part == 0) {
-#pragma unroll
-      for (int w = 1; w < KW; ++w) {
-        const float* src = lds + static_cast<size_t>((group * (KW - 1) + w - 1) * ND * 16 * 64) + lane;
-#pragma unroll
-        for (int i = 0; i < ND * 16; ++i) acc[i >> 4][i & 15] += src[i * 64];
-      }
-    }
-  }
-}
-
-// The lane's share of its own row: columns 32 db + 8 g + 4 hh + (0..3).
-template <typename T, int D>
-__device__ __forceinline__ void store_own(const f32x16* acc, float scale, T* row, int hh) {
-#pragma unroll
-  for (int db = 0; db < (D + 31) / 32; ++db) {
-#pragma unroll
-    for (int g = 0; g < 4; ++g) {
-      if (32 * db + 8 * g >= D) break;  // head dim 16
-      st4(row + 32 * db + 8 * g + 4 * hh,
-          f32x4{acc[db][4 * g], acc[db][4 * g + 1], acc[db][4 * g + 2], acc[db][4 * g + 3]} * scale);
-    }
-  }
-}
-
 // ---------------------------------------------------------------------------
 // Forward: BM queries of one (batch, q-head), K / V streamed BN keys a stage.
-// Exact running max per tile (online softmax in base 2); the waves that share
-// queries merge (m, l, acc) at the end.
-template <typename T, int D, bool CAUSAL>
+// Online softmax in base 2 with the running max moved lazily (kRescaleTau; of 32
+// rows some exact max moves in most tiles; M is exact either way); the waves
+// that share queries merge (m, l, acc) at the end.
+template <int D, bool CAUSAL>
 __global__ __launch_bounds__(256) void ssa_fwd_f32_kernel(FwdParams p) {
-  using M = Mat<T, D>;
-  using C = Cfg<T, D>;
+  using M = Mat<D>;
+  using C = Cfg<D>;
   constexpr int KW = C::KW, BM = C::BM, BN = C::BN, BB = C::BB, ND = M::ND;
   __shared__ __attribute__((aligned(1024))) char smem[C::LDS_BYTES];
   const int tid = threadIdx.x, lane = tid & 63;
@@ -307,12 +133,12 @@ __global__ __launch_bounds__(256) void ssa_fwd_f32_kernel(FwdParams p) {
   const int q0 = (nqb - 1 - pl.rank) * BM;
   if (q0 >= N) return;  // packed: past the end of a shorter document
   const int wq0 = q0 + 32 * qw, qrow = wq0 + l32;
-  const T* qg = static_cast<const T*>(p.q.ptr) + sv.off(p.q, b) + h * p.q.sh;
-  const T* kg = static_cast<const T*>(p.k.ptr) + sv.off(p.k, b) + hk * p.k.sh;
-  const T* vg = static_cast<const T*>(p.v.ptr) + sv.off(p.v, b) + hk * p.v.sh;
+  const float* qg = static_cast<const float*>(p.q.ptr) + sv.off(p.q, b) + h * p.q.sh;
+  const float* kg = static_cast<const float*>(p.k.ptr) + sv.off(p.k, b) + hk * p.k.sh;
+  const float* vg = static_cast<const float*>(p.v.ptr) + sv.off(p.v, b) + hk * p.v.sh;
   const float n = *p.n_ptr, c = p.scale * *p.b_ptr;
   const uint32_t lds0 = lds_addr(smem);
-  const int64_t kss = p.k.ss * kUnits<T>, vss = p.v.ss * kUnits<T>;
+  const int64_t kss = p.k.ss * 2, vss = p.v.ss * 2;
   const LoadLane llk(lane, wave, kss), llv(lane, wave, vss);
   auto k_at = [&](int st, int i) { return lds0 + ((st & 1) * KW + i) * 2 * BB; };
   auto load_stage = [&](int st) {
@@ -354,18 +180,18 @@ __global__ __launch_bounds__(256) void ssa_fwd_f32_kernel(FwdParams p) {
 #pragma unroll
     for (int r = 0; r < 16; ++r) mx = fmaxf(mx, t[r]);
     mx = fmaxf(m, pair_max(mx));
-    const float base = mx == -INFINITY ? 0.f : mx;  // no key of this row yet: p = 0
-    if (__any(mx > m)) {                            // the running max moves: rescale what is summed so far
-      const float alpha = fast_exp2(m - base);
+    if (__any(mx > m + kRescaleTau)) {  // rare: the running max moves, and with it what is summed so far
+      const float alpha = fast_exp2(m - (mx == -INFINITY ? 0.f : mx));
       l *= alpha;
 #pragma unroll
       for (int d = 0; d < ND; ++d) acc[d] *= alpha;
       m = mx;
     }
+    const float base = m == -INFINITY ? 0.f : m;  // no key of this row yet: p = 0
     float sum = 0.f;
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
-      t[r] = fast_exp2(t[r] - base + M::P_SHIFT);
+      t[r] = fast_exp2(t[r] - base);
       sum += t[r];
     }
     l += sum;
@@ -394,9 +220,9 @@ __global__ __launch_bounds__(256) void ssa_fwd_f32_kernel(FwdParams p) {
     merge_parts<ND, KW>(acc, reinterpret_cast<float*>(smem), qw, kw, lane);
   }
   if (kw == 0 && qrow < N) {
-    T* og = static_cast<T*>(const_cast<void*>(p.o.ptr)) + sv.off(p.o, b) + h * p.o.sh;
-    store_own<T, D>(acc, 1.f / l, og + qrow * p.o.ss, hh);  // every row has a key (causal: itself)
-    if (hh == 0) p.m[sv.mrow(b, h, p.Hq, p.T, p.N) + qrow] = m + (log2f(l) - M::P_SHIFT);
+    float* og = static_cast<float*>(const_cast<void*>(p.o.ptr)) + sv.off(p.o, b) + h * p.o.sh;
+    store_own<float, D>(acc, 1.f / l, og + qrow * p.o.ss, hh);  // every row has a key (causal: itself)
+    if (hh == 0) p.m[sv.mrow(b, h, p.Hq, p.T, p.N) + qrow] = m + log2f(l);
   }
 }
 
@@ -429,10 +255,10 @@ __global__ __launch_bounds__(256) void ssa_bwd_preprocess_f32_kernel(BwdParams p
 // group.  Per valid pair, as in ssa_bwd.hip: P = exp2(n sL - M), dT = P (dP -
 // Delta), dS' = dT / (1 + c|x|), dV += P dO, dK += dS' q (scaled by scale n b
 // at the end), dn += ln2 dT sL, db += n scale dS' x.
-template <typename T, int D, bool CAUSAL, bool DO_DK, bool DO_DV>
+template <int D, bool CAUSAL, bool DO_DK, bool DO_DV>
 __device__ __forceinline__ void dkdv_f32_body(const BwdParams& p, char* smem, float (*red)[8], int block, int grid) {
-  using M = Mat<T, D>;
-  using C = Cfg<T, D>;
+  using M = Mat<D>;
+  using C = Cfg<D>;
   constexpr int QS = C::QS, NWV = 4 * QS, BB = C::BB, ND = M::ND, STEP = 32 * QS;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -454,19 +280,19 @@ __device__ __forceinline__ void dkdv_f32_body(const BwdParams& p, char* smem, fl
     return;
   }
   const int k0w = k0 + 32 * kg4, key = k0w + l32;
-  const T* kg = static_cast<const T*>(p.k.ptr) + sv.off(p.k, b) + hk * p.k.sh;
-  const T* vg = static_cast<const T*>(p.v.ptr) + sv.off(p.v, b) + hk * p.v.sh;
+  const float* kg = static_cast<const float*>(p.k.ptr) + sv.off(p.k, b) + hk * p.k.sh;
+  const float* vg = static_cast<const float*>(p.v.ptr) + sv.off(p.v, b) + hk * p.v.sh;
   const float n = *p.n_ptr, bv = *p.b_ptr, c = p.scale * bv;
   const uint32_t lds0 = lds_addr(smem);
-  const int64_t qss = p.q.ss * kUnits<T>, doss = p.dout.ss * kUnits<T>;
+  const int64_t qss = p.q.ss * 2, doss = p.dout.ss * 2;
   const LoadLane llq(lane, wave, qss), lld(lane, wave, doss);
   const int qstart = CAUSAL ? k0 : 0;
   const int nqs = (N - qstart + STEP - 1) / STEP, nst = G * nqs;
   auto blk_at = [&](int st, int i) { return lds0 + (st & 1) * C::DKDV_STAGE + i * (2 * BB + 256); };
   auto load_stage = [&](int st, int g, int q0) {
     const int h = hk * G + g;
-    const T* qg = static_cast<const T*>(p.q.ptr) + sv.off(p.q, b) + h * p.q.sh;
-    const T* dog = static_cast<const T*>(p.dout.ptr) + sv.off(p.dout, b) + h * p.dout.sh;
+    const float* qg = static_cast<const float*>(p.q.ptr) + sv.off(p.q, b) + h * p.q.sh;
+    const float* dog = static_cast<const float*>(p.dout.ptr) + sv.off(p.dout, b) + h * p.dout.sh;
     const int64_t mr = sv.mrow(b, h, p.Hq, p.T, p.N);
 #pragma unroll
     for (int i = 0; i < QS; ++i) {
@@ -488,7 +314,6 @@ __device__ __forceinline__ void dkdv_f32_body(const BwdParams& p, char* smem, fl
 #pragma unroll
   for (int d = 0; d < ND; ++d) dk[d] = dv[d] = f32x16{};
   float dn_acc = 0.f, dn_c = 0.f, db_acc = 0.f, db_c = 0.f;  // Kahan sums over the blocks' sums
-  WeightScale<M> ws;
   int g = 0, q0 = qstart;  // of stage st
   for (int st = 0; st < nst; ++st) {
     __builtin_amdgcn_s_waitcnt(0);
@@ -532,13 +357,7 @@ __device__ __forceinline__ void dkdv_f32_body(const BwdParams& p, char* smem, fl
         }
       }
     }
-    if constexpr (DO_DV) {
-      if constexpr (M::F16) {
-#pragma unroll
-        for (int r = 0; r < 16; ++r) pv[r] *= exp2f(M::P_SHIFT);
-      }
-      mat.outer(at + BB, pv, dv);
-    }
+    if constexpr (DO_DV) mat.outer(at + BB, pv, dv);
     if constexpr (DO_DK) {
       const float y = tdn - dn_c, t = dn_acc + y;
       dn_c = (t - dn_acc) - y;
@@ -546,21 +365,19 @@ __device__ __forceinline__ void dkdv_f32_body(const BwdParams& p, char* smem, fl
       const float y2 = tdb - db_c, t2 = db_acc + y2;
       db_c = (t2 - db_acc) - y2;
       db_acc = t2;
-      ws.apply(ds, dk);
       mat.outer(at, ds, dk);
     }
   }
-  if constexpr (QS > 1) static_assert(!M::F16, "one weight scale per accumulator");
   if constexpr (DO_DK) merge_parts<ND, QS>(dk, reinterpret_cast<float*>(smem), kg4, qs, lane);
   if constexpr (DO_DV) merge_parts<ND, QS>(dv, reinterpret_cast<float*>(smem), kg4, qs, lane);
   if (qs == 0 && key < N) {
     if constexpr (DO_DK) {
-      T* dkr = static_cast<T*>(const_cast<void*>(p.dk.ptr)) + sv.off(p.dk, b) + hk * p.dk.sh + key * p.dk.ss;
-      store_own<T, D>(dk, p.scale * n * bv * ws.inverse(), dkr, hh);
+      float* dkr = static_cast<float*>(const_cast<void*>(p.dk.ptr)) + sv.off(p.dk, b) + hk * p.dk.sh + key * p.dk.ss;
+      store_own<float, D>(dk, p.scale * n * bv, dkr, hh);
     }
     if constexpr (DO_DV) {
-      T* dvr = static_cast<T*>(const_cast<void*>(p.dv.ptr)) + sv.off(p.dv, b) + hk * p.dv.sh + key * p.dv.ss;
-      store_own<T, D>(dv, exp2f(-M::P_SHIFT), dvr, hh);
+      float* dvr = static_cast<float*>(const_cast<void*>(p.dv.ptr)) + sv.off(p.dv, b) + hk * p.dv.sh + key * p.dv.ss;
+      store_own<float, D>(dv, 1.f, dvr, hh);
     }
   }
   if constexpr (DO_DK) {
@@ -589,30 +406,30 @@ __device__ __forceinline__ void dkdv_f32_body(const BwdParams& p, char* smem, fl
   }
 }
 
-template <typename T, int D, bool CAUSAL>
-__global__ __launch_bounds__((Cfg<T, D>::DKDV_THREADS)) void ssa_bwd_dkdv_f32_kernel(BwdParams p) {
-  using C = Cfg<T, D>;
+template <int D, bool CAUSAL>
+__global__ __launch_bounds__((Cfg<D>::DKDV_THREADS)) void ssa_bwd_dkdv_f32_kernel(BwdParams p) {
+  using C = Cfg<D>;
   __shared__ __attribute__((aligned(1024))) char smem[2 * C::DKDV_STAGE];
   __shared__ float red[2][8];
   if constexpr (C::ROLES) {
     // dK workgroups (three products per block) before the lighter dV ones
     const int half = gridDim.x / 2;
     if (static_cast<int>(blockIdx.x) < half)
-      dkdv_f32_body<T, D, CAUSAL, true, false>(p, smem, red, blockIdx.x, half);
+      dkdv_f32_body<D, CAUSAL, true, false>(p, smem, red, blockIdx.x, half);
     else
-      dkdv_f32_body<T, D, CAUSAL, false, true>(p, smem, red, blockIdx.x - half, half);
+      dkdv_f32_body<D, CAUSAL, false, true>(p, smem, red, blockIdx.x - half, half);
   } else {
-    dkdv_f32_body<T, D, CAUSAL, true, true>(p, smem, red, blockIdx.x, gridDim.x);
+    dkdv_f32_body<D, CAUSAL, true, true>(p, smem, red, blockIdx.x, gridDim.x);
   }
 }
 
 // ---------------------------------------------------------------------------
 // dQ for BM query rows of one (batch, q-head): K / V streamed BN keys a stage;
 // the scores and dP are recomputed (dQ += scale n b dS' k).
-template <typename T, int D, bool CAUSAL>
+template <int D, bool CAUSAL>
 __global__ __launch_bounds__(256) void ssa_bwd_dq_f32_kernel(BwdParams p) {
-  using M = Mat<T, D>;
-  using C = Cfg<T, D>;
+  using M = Mat<D>;
+  using C = Cfg<D>;
   constexpr int KW = C::KW, BM = C::BM, BN = C::BN, BB = C::BB, ND = M::ND;
   __shared__ __attribute__((aligned(1024))) char smem[C::LDS_BYTES];
   const int tid = threadIdx.x, lane = tid & 63;
@@ -629,14 +446,14 @@ __global__ __launch_bounds__(256) void ssa_bwd_dq_f32_kernel(BwdParams p) {
   const int q0 = (nqb - 1 - pl.rank) * BM;
   if (q0 >= N) return;
   const int wq0 = q0 + 32 * qw, qrow = wq0 + l32;
-  const T* qg = static_cast<const T*>(p.q.ptr) + sv.off(p.q, b) + h * p.q.sh;
-  const T* dog = static_cast<const T*>(p.dout.ptr) + sv.off(p.dout, b) + h * p.dout.sh;
-  const T* kg = static_cast<const T*>(p.k.ptr) + sv.off(p.k, b) + hk * p.k.sh;
-  const T* vg = static_cast<const T*>(p.v.ptr) + sv.off(p.v, b) + hk * p.v.sh;
+  const float* qg = static_cast<const float*>(p.q.ptr) + sv.off(p.q, b) + h * p.q.sh;
+  const float* dog = static_cast<const float*>(p.dout.ptr) + sv.off(p.dout, b) + h * p.dout.sh;
+  const float* kg = static_cast<const float*>(p.k.ptr) + sv.off(p.k, b) + hk * p.k.sh;
+  const float* vg = static_cast<const float*>(p.v.ptr) + sv.off(p.v, b) + hk * p.v.sh;
   const int64_t mr = sv.mrow(b, h, p.Hq, p.T, p.N);
   const float n = *p.n_ptr, bv = *p.b_ptr, c = p.scale * bv;
   const uint32_t lds0 = lds_addr(smem);
-  const int64_t kss = p.k.ss * kUnits<T>, vss = p.v.ss * kUnits<T>;
+  const int64_t kss = p.k.ss * 2, vss = p.v.ss * 2;
   const LoadLane llk(lane, wave, kss), llv(lane, wave, vss);
   auto k_at = [&](int st, int i) { return lds0 + ((st & 1) * KW + i) * 2 * BB; };
   auto load_stage = [&](int st) {
@@ -658,7 +475,6 @@ __global__ __launch_bounds__(256) void ssa_bwd_dq_f32_kernel(BwdParams p) {
   f32x16 dq[ND];
 #pragma unroll
   for (int d = 0; d < ND; ++d) dq[d] = f32x16{};
-  WeightScale<M> ws;
   const int kv_end = CAUSAL ? min(N, q0 + BM) : N;
   const int nst = (kv_end + BN - 1) / BN;
   for (int st = 0; st < nst; ++st) {
@@ -683,47 +499,29 @@ __global__ __launch_bounds__(256) void ssa_bwd_dq_f32_kernel(BwdParams p) {
       for (int r = 0; r < 16; ++r)
         if (k0 + crow(r, hh) > last) ds[r] = 0.f;
     }
-    ws.apply(ds, dq);
     mat.outer(at, ds, dq);
   }
-  if constexpr (KW > 1) {
-    if constexpr (M::F16) {  // bring the sharing waves' sums to true scale first
-      const float inv = ws.inverse();
-#pragma unroll
-      for (int d = 0; d < ND; ++d) dq[d] *= inv;
-    }
-    merge_parts<ND, KW>(dq, reinterpret_cast<float*>(smem), qw, kw, lane);
-  }
+  merge_parts<ND, KW>(dq, reinterpret_cast<float*>(smem), qw, kw, lane);
   if (kw == 0 && qrow < N) {
-    T* dqr = static_cast<T*>(const_cast<void*>(p.dq.ptr)) + sv.off(p.dq, b) + h * p.dq.sh + qrow * p.dq.ss;
-    store_own<T, D>(dq, p.scale * n * bv * (KW > 1 ? 1.f : ws.inverse()), dqr, hh);
+    float* dqr = static_cast<float*>(const_cast<void*>(p.dq.ptr)) + sv.off(p.dq, b) + h * p.dq.sh + qrow * p.dq.ss;
+    store_own<float, D>(dq, p.scale * n * bv, dqr, hh);
   }
 }
 
-// One launch of KERNEL<T, DD, CAUSAL>.
-#define SSA_F32_LAUNCH(KERNEL, THREADS, T, DD, GRID, P, CAUSAL, S)                                     \
-  do {                                                                                                 \
-    if (CAUSAL) hipLaunchKernelGGL((KERNEL<T, DD, true>), GRID(T, DD), dim3(THREADS(T, DD)), 0, S, P); \
-    else hipLaunchKernelGGL((KERNEL<T, DD, false>), GRID(T, DD), dim3(THREADS(T, DD)), 0, S, P); \
+// One launch of KERNEL<DD, CAUSAL>, and the head dims.
+#define SSA_F32_LAUNCH(KERNEL, THREADS, DD, GRID, P, CAUSAL, S)                                     \
+  do {                                                                                              \
+    if (CAUSAL) hipLaunchKernelGGL((KERNEL<DD, true>), GRID(DD), dim3(THREADS(DD)), 0, S, P);        \
+    else hipLaunchKernelGGL((KERNEL<DD, false>), GRID(DD), dim3(THREADS(DD)), 0, S, P);              \
   } while (0)
-
-// The head dims of each element type: fp32 at 16-256, bf16 / fp16 at 256
-// (their other head dims run on the 16-bit kernels).
-#define SSA_F32_DISPATCH(KERNEL, THREADS, GRID, P, DTYPE, D, CAUSAL, S)                         \
-  if (DTYPE == kDtypeF32) {                                                                     \
-    switch (D) {                                                                                \
-      case 16: SSA_F32_LAUNCH(KERNEL, THREADS, float, 16, GRID, P, CAUSAL, S); break;           \
-      case 32: SSA_F32_LAUNCH(KERNEL, THREADS, float, 32, GRID, P, CAUSAL, S); break;           \
-      case 64: SSA_F32_LAUNCH(KERNEL, THREADS, float, 64, GRID, P, CAUSAL, S); break;           \
-      case 128: SSA_F32_LAUNCH(KERNEL, THREADS, float, 128, GRID, P, CAUSAL, S); break;         \
-      case 256: SSA_F32_LAUNCH(KERNEL, THREADS, float, 256, GRID, P, CAUSAL, S); break;         \
-      default: return hipErrorInvalidValue;                                                     \
-    }                                                                                           \
-  } else if (D == 256) {                                                                        \
-    if (DTYPE == 0) SSA_F32_LAUNCH(KERNEL, THREADS, __bf16, 256, GRID, P, CAUSAL, S);           \
-    else SSA_F32_LAUNCH(KERNEL, THREADS, _Float16, 256, GRID, P, CAUSAL, S);                    \
-  } else {                                                                                      \
-    return hipErrorInvalidValue;                                                                \
+#define SSA_F32_DISPATCH(KERNEL, THREADS, GRID, P, D, CAUSAL, S)                 \
+  switch (D) {                                                                   \
+    case 16: SSA_F32_LAUNCH(KERNEL, THREADS, 16, GRID, P, CAUSAL, S); break;     \
+    case 32: SSA_F32_LAUNCH(KERNEL, THREADS, 32, GRID, P, CAUSAL, S); break;     \
+    case 64: SSA_F32_LAUNCH(KERNEL, THREADS, 64, GRID, P, CAUSAL, S); break;     \
+    case 128: SSA_F32_LAUNCH(KERNEL, THREADS, 128, GRID, P, CAUSAL, S); break;   \
+    case 256: SSA_F32_LAUNCH(KERNEL, THREADS, 256, GRID, P, CAUSAL, S); break;   \
+    default: return hipErrorInvalidValue;                                        \
   }
 
 template <typename T, int D>
@@ -736,19 +534,14 @@ static void launch_pre(const BwdParams& p, hipStream_t s) {
 
 }  // namespace
 
-// A launch takes fewer than 2^32 threads along x: larger row grids (from 2^23
-// workgroups) fold over y.
-static dim3 row_grid(int n) {
-  const int y = (n + (1 << 23) - 1) >> 23;
-  return dim3((n + y - 1) / y, y);
-}
-#define SSA_F32_ROW_GRID(T, DD) row_grid((p.N + Cfg<T, DD>::BM - 1) / Cfg<T, DD>::BM * p.B * p.Hq)
-#define SSA_F32_KEY_GRID(T, DD) dim3(dkdv_key_blocks(p.N) * p.B * p.Hkv * (Cfg<T, DD>::ROLES ? 2 : 1))
-#define SSA_F32_THREADS(T, DD) 256
-#define SSA_F32_KEY_THREADS(T, DD) (Cfg<T, DD>::DKDV_THREADS)
+#define SSA_F32_ROW_GRID(DD) row_grid((p.N + Cfg<DD>::BM - 1) / Cfg<DD>::BM * p.B * p.Hq)
+#define SSA_F32_KEY_GRID(DD) dim3(dkdv_key_blocks(p.N) * p.B * p.Hkv * (Cfg<DD>::ROLES ? 2 : 1))
+#define SSA_F32_THREADS(DD) 256
+#define SSA_F32_KEY_THREADS(DD) (Cfg<DD>::DKDV_THREADS)
 
 hipError_t launch_fwd_f32(const FwdParams& p, int dtype, int D, bool causal, hipStream_t s) {
-  SSA_F32_DISPATCH(ssa_fwd_f32_kernel, SSA_F32_THREADS, SSA_F32_ROW_GRID, p, dtype, D, causal, s)
+  if (dtype != kDtypeF32) return launch_fwd_d256(p, dtype, D, causal, s);
+  SSA_F32_DISPATCH(ssa_fwd_f32_kernel, SSA_F32_THREADS, SSA_F32_ROW_GRID, p, D, causal, s)
   return hipGetLastError();
 }
 
@@ -774,12 +567,14 @@ hipError_t launch_bwd_preprocess_f32(const BwdParams& p, int dtype, int D, hipSt
 }
 
 hipError_t launch_bwd_dkdv_f32(const BwdParams& p, int dtype, int D, bool causal, hipStream_t s) {
-  SSA_F32_DISPATCH(ssa_bwd_dkdv_f32_kernel, SSA_F32_KEY_THREADS, SSA_F32_KEY_GRID, p, dtype, D, causal, s)
+  if (dtype != kDtypeF32) return launch_bwd_dkdv_d256(p, dtype, D, causal, s);
+  SSA_F32_DISPATCH(ssa_bwd_dkdv_f32_kernel, SSA_F32_KEY_THREADS, SSA_F32_KEY_GRID, p, D, causal, s)
   return hipGetLastError();
 }
 
 hipError_t launch_bwd_dq_f32(const BwdParams& p, int dtype, int D, bool causal, hipStream_t s) {
-  SSA_F32_DISPATCH(ssa_bwd_dq_f32_kernel, SSA_F32_THREADS, SSA_F32_ROW_GRID, p, dtype, D, causal, s)
+  if (dtype != kDtypeF32) return launch_bwd_dq_d256(p, dtype, D, causal, s);
+  SSA_F32_DISPATCH(ssa_bwd_dq_f32_kernel, SSA_F32_THREADS, SSA_F32_ROW_GRID, p, D, causal, s)
   return hipGetLastError();
 }
 

@@ -21,7 +21,7 @@ hipError_t launch_reduce_partials(const BwdParams& p, hipStream_t stream);
 
 hipError_t launch_decode(const DecodeParams& p, int dtype, int D, hipStream_t stream);
 
-// The fp32-precision kernels (ssa_f32.hip) run fp32 inputs at every head dim
+// The fp32-precision kernels (ssa_f32.hip, ssa_d256.hip) run fp32 inputs at every head dim
 // and bf16 / fp16 inputs at head dim 256; the 16-bit kernels run bf16 / fp16
 // at 32, 64 and 128.  The fp32-precision backward does not use the dS'
 // workspace (its dQ recomputes).
@@ -31,6 +31,10 @@ hipError_t launch_fwd_f32(const FwdParams& p, int dtype, int D, bool causal, hip
 hipError_t launch_bwd_preprocess_f32(const BwdParams& p, int dtype, int D, hipStream_t stream);
 hipError_t launch_bwd_dkdv_f32(const BwdParams& p, int dtype, int D, bool causal, hipStream_t stream);
 hipError_t launch_bwd_dq_f32(const BwdParams& p, int dtype, int D, bool causal, hipStream_t stream);
+// ... bf16 / fp16 at head dim 256 (ssa_d256.hip)
+hipError_t launch_fwd_d256(const FwdParams& p, int dtype, int D, bool causal, hipStream_t stream);
+hipError_t launch_bwd_dkdv_d256(const BwdParams& p, int dtype, int D, bool causal, hipStream_t stream);
+hipError_t launch_bwd_dq_d256(const BwdParams& p, int dtype, int D, bool causal, hipStream_t stream);
 
 }  // namespace ssa
 
