@@ -174,14 +174,12 @@ int32_t fill_bwd_params(const ssa_bwd_args* a, BwdParams* p, bool preprocess_onl
   return SSA_OK;
 }
 
-// dQ then the dn / db reduction: on the workspace path (the matrix-core
-// kernels with a dS' workspace) the dQ pass's first workgroup does the
-// reduction, so it needs no launch of its own.
+// dQ and the dn / db reduction, which the dQ kernel's first workgroup does, so
+// it needs no launch of its own.
 int32_t run_dq_and_reduce(const BwdParams& p, int dtype, int D, bool causal, hipStream_t s) {
   BwdParams pq = p;
-  pq.fuse_reduce = p.ds != nullptr && !use_f32(dtype, D);
-  SSA_TRY(launch_status(launch_bwd_dq(pq, dtype, D, causal, s)));
-  return pq.fuse_reduce ? SSA_OK : launch_status(launch_reduce_partials(p, s));
+  pq.fuse_reduce = 1;
+  return launch_status(launch_bwd_dq(pq, dtype, D, causal, s));
 }
 
 // The whole backward on one stream: preprocess, dK/dV, dQ, reduction.

@@ -613,6 +613,11 @@ __global__ __launch_bounds__(256, 2) void ssa_bwd_dq_kernel(BwdParams p) {
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int l32 = lane & 31, hh = lane >> 5;
+  if (p.fuse_reduce && blockIdx.x == 0) {  // the backward's dn / db sums, before the first load
+    reduce_partials_body(p.partials, static_cast<int64_t>(p.B) * p.Hkv * dkdv_key_blocks(p.N), p.dn, p.db,
+                         reinterpret_cast<float(*)[256]>(smem), threadIdx.x);
+    __syncthreads();
+  }
   // dispatch and K / V tile loads (ssa_plan.hpp)
   const Plan pl(p, blockIdx.x, gridDim.x);
   if (pl.empty()) return;  // packed: past the end of a shorter document

@@ -172,9 +172,9 @@ struct BwdParams {
   // Optional dS' workspace (dense batches): when set, dK/dV writes the
   // gradient tiles there and dQ is a product with K instead of a recompute.
   void* ds;
-  // Workspace dQ pass only: its workgroup 0 also sums the dn / db partials
-  // (the reduction of ssa_reduce_partials_kernel, bit for bit), so the whole
-  // backward needs no separate reduction launch.
+  // dQ: its workgroup 0 also sums the dn / db partials (the reduction of
+  // ssa_reduce_partials_kernel, bit for bit), so the whole backward needs no
+  // separate reduction launch (4 us).
   int fuse_reduce;
 };
 

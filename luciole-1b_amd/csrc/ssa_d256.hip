@@ -558,6 +558,11 @@ __global__ __launch_bounds__(256) void ssa_bwd_dq_d256_kernel(BwdParams p) {
   const int nqb = (p.N + kBM - 1) / kBM, grid = nqb * p.B * p.Hq;
   const int block = blockIdx.y * gridDim.x + blockIdx.x;
   if (block >= grid) return;
+  if (p.fuse_reduce && block == 0) {  // the backward's dn / db sums, before the first load (reduce_partials_body)
+    reduce_partials_body(p.partials, static_cast<int64_t>(p.B) * p.Hkv * dkdv_key_blocks(p.N), p.dn, p.db,
+                         reinterpret_cast<float(*)[256]>(smem), threadIdx.x);
+    __syncthreads();
+  }
   const Place pl(block, grid, nqb, p.B, p.cu_seqlens != nullptr);
   const int b = pl.b, h = pl.h, hk = h / (p.Hq / p.Hkv);
   const SeqView sv(p.cu_seqlens, p.T, p.N, b);

@@ -32,7 +32,7 @@
 // at a time) up to head dim 128, so that a workgroup owns 32 or 64 rows: a
 // grid of one sequence then fills the chip, and causal blocks balance.
 // Measured (us, the earlier vector-ALU kernels -> these): fp32, B = 1, H = 16,
-// N = 1024, D = 64 causal: forward 376 -> 42, dK/dV 498 -> 144, dQ 380 -> 51.
+// N = 1024, D = 64 causal: forward 376 -> 43, dK/dV 498 -> 124, dQ 380 -> 53.
 #include "ssa_rows.hpp"
 
 namespace ssa {
@@ -99,11 +99,8 @@ struct Cfg {
   static constexpr int QW = 4 / KW;  // waves on different rows (forward, dQ): 32 QW rows per workgroup
   static constexpr int BM = 32 * QW, BN = 32 * KW;
   static constexpr int LDS_BYTES = 2 * KW * 2 * BB;
-  // dK/dV: two waves per 32 keys up to head dim 64 (two waves per SIMD); at
-  // 256 the accumulators of dK and dV do not fit one wave beside the K and V
-  // fragments, so half of the grid computes dK (and dn, db) and half dV.
+  // dK/dV: two waves per 32 keys up to head dim 64 (two waves per SIMD)
   static constexpr int QS = D <= 64 ? 2 : 1;
-  static constexpr bool ROLES = D >= 256;
   static constexpr int DKDV_THREADS = 256 * QS;
   static constexpr int DKDV_STAGE = QS * (2 * BB + 256);  // Q, dO, M[32], Delta[32] per block
 };
@@ -406,12 +403,14 @@ __device__ __forceinline__ void dkdv_f32_body(const BwdParams& p, char* smem, fl
   }
 }
 
-template <int D, bool CAUSAL>
+// ROLES: half of the grid computes dK (and dn, db; three products a block) and
+// half dV (two).
+template <int D, bool CAUSAL, bool ROLES>
 __global__ __launch_bounds__((Cfg<D>::DKDV_THREADS)) void ssa_bwd_dkdv_f32_kernel(BwdParams p) {
   using C = Cfg<D>;
   __shared__ __attribute__((aligned(1024))) char smem[2 * C::DKDV_STAGE];
   __shared__ float red[2][8];
-  if constexpr (C::ROLES) {
+  if constexpr (ROLES) {
     // dK workgroups (three products per block) before the lighter dV ones
     const int half = gridDim.x / 2;
     if (static_cast<int>(blockIdx.x) < half)
@@ -439,12 +438,17 @@ __global__ __launch_bounds__(256) void ssa_bwd_dq_f32_kernel(BwdParams p) {
   const int nqb = (p.N + BM - 1) / BM, grid = nqb * p.B * p.Hq;
   const int block = blockIdx.y * gridDim.x + blockIdx.x;
   if (block >= grid) return;
+  if (p.fuse_reduce && block == 0) {  // the backward's dn / db sums, before the first load (reduce_partials_body)
+    reduce_partials_body(p.partials, static_cast<int64_t>(p.B) * p.Hkv * dkdv_key_blocks(p.N), p.dn, p.db,
+                         reinterpret_cast<float(*)[256]>(smem), threadIdx.x);
+    __syncthreads();
+  }
   const Place pl(block, grid, nqb, p.B, p.cu_seqlens != nullptr);
   const int b = pl.b, h = pl.h, hk = h / (p.Hq / p.Hkv);
   const SeqView sv(p.cu_seqlens, p.T, p.N, b);
   const int N = sv.N;
   const int q0 = (nqb - 1 - pl.rank) * BM;
-  if (q0 >= N) return;
+  if (q0 >= N) return;  // packed: past the end of a shorter document
   const int wq0 = q0 + 32 * qw, qrow = wq0 + l32;
   const float* qg = static_cast<const float*>(p.q.ptr) + sv.off(p.q, b) + h * p.q.sh;
   const float* dog = static_cast<const float*>(p.dout.ptr) + sv.off(p.dout, b) + h * p.dout.sh;
@@ -535,9 +539,30 @@ static void launch_pre(const BwdParams& p, hipStream_t s) {
 }  // namespace
 
 #define SSA_F32_ROW_GRID(DD) row_grid((p.N + Cfg<DD>::BM - 1) / Cfg<DD>::BM * p.B * p.Hq)
-#define SSA_F32_KEY_GRID(DD) dim3(dkdv_key_blocks(p.N) * p.B * p.Hkv * (Cfg<DD>::ROLES ? 2 : 1))
 #define SSA_F32_THREADS(DD) 256
-#define SSA_F32_KEY_THREADS(DD) (Cfg<DD>::DKDV_THREADS)
+
+// dK and dV in one workgroup (four products a block) or in two (three and two).
+// Apart they have twice the workgroups, the longest of them three quarters as
+// long: worth a quarter more work while the grid leaves CUs idle, that is up to
+// 128 workgroups of 128 keys without the mask and, since half of a causal
+// grid's work is in its first quarter, up to 256 with it (us, together -> apart:
+// causal D = 64 1 x 16 x 1024 148 -> 124, 1 x 16 x 2048 (256) 290 -> 252, D = 128
+// 1 x 16 x 1100 318 -> 252; full D = 64 1 x 16 x 1024 151 -> 131, 2 x 16 x 1100
+// (288) 329 -> 327).  At head dim 256 the accumulators of both do not fit one
+// wave beside the K and V fragments.
+constexpr int kRolesGrid = 128;
+template <int D, bool CAUSAL>
+static hipError_t launch_dkdv(const BwdParams& p, hipStream_t s) {
+  const int grid = dkdv_key_blocks(p.N) * p.B * p.Hkv;
+  const dim3 threads(Cfg<D>::DKDV_THREADS);
+  if (D >= 256 || grid <= (CAUSAL ? 2 : 1) * kRolesGrid) {
+    hipLaunchKernelGGL((ssa_bwd_dkdv_f32_kernel<D, CAUSAL, true>), dim3(2 * grid), threads, 0, s, p);
+    return hipGetLastError();
+  }
+  if constexpr (D < 256)
+    hipLaunchKernelGGL((ssa_bwd_dkdv_f32_kernel<D, CAUSAL, false>), dim3(grid), threads, 0, s, p);
+  return hipGetLastError();
+}
 
 hipError_t launch_fwd_f32(const FwdParams& p, int dtype, int D, bool causal, hipStream_t s) {
   if (dtype != kDtypeF32) return launch_fwd_d256(p, dtype, D, causal, s);
@@ -568,8 +593,14 @@ hipError_t launch_bwd_preprocess_f32(const BwdParams& p, int dtype, int D, hipSt
 
 hipError_t launch_bwd_dkdv_f32(const BwdParams& p, int dtype, int D, bool causal, hipStream_t s) {
   if (dtype != kDtypeF32) return launch_bwd_dkdv_d256(p, dtype, D, causal, s);
-  SSA_F32_DISPATCH(ssa_bwd_dkdv_f32_kernel, SSA_F32_KEY_THREADS, SSA_F32_KEY_GRID, p, D, causal, s)
-  return hipGetLastError();
+  switch (D) {
+    case 16: return causal ? launch_dkdv<16, true>(p, s) : launch_dkdv<16, false>(p, s);
+    case 32: return causal ? launch_dkdv<32, true>(p, s) : launch_dkdv<32, false>(p, s);
+    case 64: return causal ? launch_dkdv<64, true>(p, s) : launch_dkdv<64, false>(p, s);
+    case 128: return causal ? launch_dkdv<128, true>(p, s) : launch_dkdv<128, false>(p, s);
+    case 256: return causal ? launch_dkdv<256, true>(p, s) : launch_dkdv<256, false>(p, s);
+    default: return hipErrorInvalidValue;
+  }
 }
 
 hipError_t launch_bwd_dq_f32(const BwdParams& p, int dtype, int D, bool causal, hipStream_t s) {
