@@ -514,7 +514,8 @@ def _check_cache_layout(t: torch.Tensor, name: str) -> None:
 
 
 def ssa_decode_num_splits(B: int, Hq: int, Hkv: int, capacity: int, num_splits: int = 0) -> int:
-    """Key splits the decode kernel uses (``num_splits`` = 0: its own choice)."""
+    """Key splits ``ssa_decode_attention`` uses (``num_splits`` = 0: its own choice)."""
+    num_splits = num_splits or _lib.native().decode_splits(B, Hq, Hkv, capacity)
     return int(_lib.lib().ssa_decode_num_splits(B, Hq, Hkv, capacity, num_splits))
 
 
@@ -566,6 +567,7 @@ def ssa_decode_attention(q, k_cache, v_cache, cache_seqlens, softmax_scale, ssa_
     lens = lens.to(torch.int32).contiguous()
     n32 = _scalar(ssa_n, q.device)
     b32 = _scalar(ssa_b, q.device)
+    num_splits = int(num_splits) or _lib.native().decode_splits(B, Hq, Hkv, cap)
     out = torch.empty((B, Hq, 1, D), dtype=q.dtype, device=q.device)
     m = torch.empty((B, Hq), dtype=torch.float32, device=q.device) if return_m else None
     ws_bytes = int(_lib.lib().ssa_decode_workspace_bytes(B, Hq, Hkv, cap, D, int(num_splits)))

@@ -193,9 +193,12 @@ __global__ __launch_bounds__(DecodeCfg<D>::NW * 64) void ssa_decode_kernel(Decod
 // One thread per output element d of a (sequence, q-head): combine the split
 // partials in split order, out = sum_s acc_s 2^(m_s - M) / sum_s l_s 2^(m_s - M),
 // in one pass with the running maximum (each split's loads are independent of
-// the running state, so they can all be in flight at once).
+// the running state, so they can all be in flight at once).  Up to
+// kMergeFewSplits splits: 8.0 against 8.5 us of a 2-split step (16 x 24/8 x 700 x
+// 32) by the wide form below.
+constexpr int kMergeFewSplits = 4;
 template <typename T, int D>
-__global__ __launch_bounds__(128) void ssa_decode_merge_kernel(DecodeParams p) {
+__global__ __launch_bounds__(128) void ssa_decode_merge_few_kernel(DecodeParams p) {
   const int bh = blockIdx.x, d = threadIdx.x;
   const int b = bh / p.Hq, hq = bh - b * p.Hq;
   const int64_t rec0 = static_cast<int64_t>(bh) * p.splits;
@@ -224,11 +227,63 @@ __global__ __launch_bounds__(128) void ssa_decode_merge_kernel(DecodeParams p) {
   if (d == 0 && p.m != nullptr) p.m[bh] = M + log2f(l_safe);
 }
 
+// More splits: one workgroup per (sequence, q-head), out = sum_s acc_s
+// 2^(m_s - M) / sum_s l_s 2^(m_s - M).  Latency bound (a few KB), so nothing is a
+// chain over the splits: every wave takes the maximum and the sum of l over
+// lanes, one split each, while its own share of acc (every fourth split, in
+// order, independent loads) is on its way, and the four shares meet in LDS.
+// The walk of one thread per element over the splits grew with them (whole
+// step, us: 1 x 4 heads x 8192 x 128, 32 splits 19.1 -> 12.6; 1 x 16 x 2048 x 128,
+// 8 splits 13.4 -> 12.5).
+template <typename T, int D>
+__global__ __launch_bounds__(256) void ssa_decode_merge_kernel(DecodeParams p) {
+  constexpr int CPL = D >= 64 ? D / 64 : 1;  // columns per lane
+  __shared__ float part[4][D];
+  const int bh = blockIdx.x, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int b = bh / p.Hq, hq = bh - b * p.Hq;
+  const int64_t rec0 = static_cast<int64_t>(bh) * p.splits;
+  const float* ml = p.ws_ml + 2 * rec0;
+  float M = -INFINITY;
+  for (int s = lane; s < p.splits; s += 64) M = fmaxf(M, ml[2 * s]);
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) M = fmaxf(M, __shfl_xor(M, off, 64));
+  const float ref = M == -INFINITY ? 0.f : M;  // every split empty: l = 0, acc = 0
+  float Ls = 0.f;
+  for (int s = lane; s < p.splits; s += 64) Ls += ml[2 * s + 1] * fast_exp2(ml[2 * s] - ref);
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) Ls += __shfl_xor(Ls, off, 64);
+  float O[CPL];
+#pragma unroll
+  for (int j = 0; j < CPL; ++j) O[j] = 0.f;
+  const int col = D >= 64 ? lane : (lane & (D - 1));
+  const float* acc = p.ws_acc + rec0 * D + col;
+#pragma unroll 4
+  for (int s = wave; s < p.splits; s += 4) {
+    const float f = fast_exp2(ml[2 * s] - ref);
+#pragma unroll
+    for (int j = 0; j < CPL; ++j) O[j] = fmaf(acc[static_cast<int64_t>(s) * D + 64 * j], f, O[j]);
+  }
+#pragma unroll
+  for (int j = 0; j < CPL; ++j)
+    if (lane < D) part[wave][col + 64 * j] = O[j];
+  __syncthreads();
+  const float l_safe = Ls > 0.f ? Ls : 1.f;
+  const int d = threadIdx.x;
+  if (d < D) {
+    T* o = static_cast<T*>(const_cast<void*>(p.o.ptr)) + b * p.o.sb + hq * p.o.sh;
+    o[d] = static_cast<T>(((part[0][d] + part[1][d]) + (part[2][d] + part[3][d])) * (1.f / l_safe));
+  }
+  if (d == 0 && p.m != nullptr) p.m[bh] = M + log2f(l_safe);
+}
+
 template <typename T, int D>
 static hipError_t launch_decode_t(const DecodeParams& p, hipStream_t s) {
   const int grid = DecodePlan<D>::grid(p);
   hipLaunchKernelGGL((ssa_decode_kernel<T, D>), dim3(grid), dim3(DecodeCfg<D>::NW * 64), 0, s, p);
-  if (p.splits > 1) hipLaunchKernelGGL((ssa_decode_merge_kernel<T, D>), dim3(p.B * p.Hq), dim3(128), 0, s, p);
+  if (p.splits > kMergeFewSplits)
+    hipLaunchKernelGGL((ssa_decode_merge_kernel<T, D>), dim3(p.B * p.Hq), dim3(256), 0, s, p);
+  else if (p.splits > 1)
+    hipLaunchKernelGGL((ssa_decode_merge_few_kernel<T, D>), dim3(p.B * p.Hq), dim3(128), 0, s, p);
   return hipGetLastError();
 }
 

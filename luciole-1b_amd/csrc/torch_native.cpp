@@ -319,6 +319,34 @@ PyObject* backward(PyObject*, PyObject* const* a, Py_ssize_t n) {
   END_HANDLE_TH_ERRORS
 }
 
+// The launch layer's key splits for num_splits = 0: about 256 workgroups (one
+// per CU), as the library's own choice, but down to 128 keys a split (the library
+// stops at 256): a lone short cache is bound by latency, and its splits run side
+// by side (us, 256 -> 128 keys: 1 x 16 x 2048 x 128 12.5 -> 9.4, 1 x 32/8 x 2048 x 64
+// 9.1 -> 8.0, 1 x 4 x 8192 x 128 12.6 -> 10.6).  Caches up to 256 keys stay whole:
+// the merge costs more than they gain (8 x 8 x 150 x 64: 5.2 against 7.4).
+int64_t launch_splits(int64_t B, int64_t Hq, int64_t Hkv, int64_t cap) {
+  if (B <= 0 || Hq <= 0 || Hkv <= 0 || cap <= 256) return 1;
+  const int64_t units = B * Hkv * ((Hq / Hkv + 31) / 32);
+  const int64_t want = (256 + units - 1) / units, most = (cap + 127) / 128;
+  return want < most ? want : most;
+}
+
+// decode_splits(B, Hq, Hkv, capacity): launch_splits
+PyObject* decode_splits(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  if (n != 4) {
+    PyErr_SetString(PyExc_TypeError, "decode_splits: four arguments");
+    return nullptr;
+  }
+  int64_t v[4];
+  for (int i = 0; i < 4; ++i) {
+    v[i] = PyLong_AsLongLong(a[i]);
+    if (v[i] == -1 && PyErr_Occurred()) return nullptr;
+    if (v[i] < 0 || v[i] > INT32_MAX) v[i] = 0;  // the library refuses the call
+  }
+  return PyLong_FromLongLong(launch_splits(v[0], v[1], v[2], v[3]));
+}
+
 // decode(q, k_cache, v_cache, lens, scale, n, b, num_splits, dev, stream)
 //   -> (out [B, Hq, D],) | status | None
 PyObject* decode(PyObject*, PyObject* const* a, Py_ssize_t n) {
@@ -348,7 +376,8 @@ PyObject* decode(PyObject*, PyObject* const* a, Py_ssize_t n) {
   {
     pybind11::gil_scoped_release unlocked;
     const int32_t b32 = static_cast<int32_t>(B), hq = static_cast<int32_t>(Hq), hk = static_cast<int32_t>(Hkv),
-                  c32 = static_cast<int32_t>(cap), d32 = static_cast<int32_t>(D), sp = static_cast<int32_t>(splits);
+                  c32 = static_cast<int32_t>(cap), d32 = static_cast<int32_t>(D),
+                  sp = static_cast<int32_t>(splits != 0 ? splits : launch_splits(B, Hq, Hkv, cap));
     out = at::empty({B, Hq, D}, q->options());
     const int64_t ws_bytes = abi.decode_bytes(b32, hq, hk, c32, d32, sp);
     at::Tensor ws;
@@ -389,6 +418,7 @@ PyMethodDef methods[] = {{"bind", SSA_FAST(&bind)},
                          {"varlen_fwd", SSA_FAST(&forward<true>)},
                          {"varlen_bwd", SSA_FAST(&backward<true>)},
                          {"decode", SSA_FAST(&decode)},
+                         {"decode_splits", SSA_FAST(&decode_splits)},
                          {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_ssa_native", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
 

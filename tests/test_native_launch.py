@@ -11,7 +11,10 @@ import torch
 
 
 class _Declines:
-    """Stands in for the extension module and takes nothing."""
+    """Stands in for the extension module and takes no call."""
+
+    def __init__(self, real):
+        self.decode_splits = real.decode_splits
 
     def __getattr__(self, name):
         return lambda *a: None
@@ -22,7 +25,8 @@ def python_path(monkeypatch):
     from SSA import _lib
 
     def switch():
-        monkeypatch.setattr(_lib, "native", _Declines)
+        stub = _Declines(_lib.native())
+        monkeypatch.setattr(_lib, "native", lambda: stub)
 
     return switch
 
@@ -43,6 +47,19 @@ def test_declines_what_it_cannot_take():
         nat.bind(1, 2)
     with pytest.raises(ValueError):
         nat.bind(*[0] * 9)
+
+
+def test_decode_splits():
+    """256 workgroups, splits of at least 128 keys, short caches whole; the C
+    ABI clamps and rounds the request as any other."""
+    from SSA import _lib, ssa_decode_num_splits
+
+    f = _lib.native().decode_splits
+    assert f(1, 16, 16, 2048) == 16 and f(1, 4, 4, 8192) == 64 and f(1, 32, 8, 500) == 4
+    assert f(16, 32, 8, 4096) == 2 and f(32, 32, 8, 8192) == 1 and f(1, 8, 8, 256) == 1
+    assert f(1, 64, 1, 100000) == 128  # two groups of 32 heads
+    assert f(0, 8, 8, 1000) == 1 and f(-1, 8, 8, 2**40) == 1
+    assert ssa_decode_num_splits(1, 16, 16, 2048) == 16 and ssa_decode_num_splits(1, 16, 16, 2048, 3) == 3
 
 
 def _views(t):
