@@ -142,6 +142,23 @@ typedef struct {
 
 int32_t ssa_cross_entropy(const ssa_cross_entropy_args* args, void* stream);
 
+/*
+ * Gradient of a token embedding's fp32 table (the word embedding ahead of the
+ * reference's decoder layers): grad [vocab, hidden] fp32, every row written,
+ * = the sum of dy's rows over the tokens that name it, in a fixed order.
+ * ids int64 [tokens] (one outside [0, vocab) adds nothing), dy [tokens,
+ * hidden] fp32, both contiguous, dy and grad 16-byte aligned, hidden a
+ * multiple of 4.
+ */
+typedef struct {
+  const void* ids;
+  const float* dy;
+  float* grad;
+  int32_t tokens, vocab, hidden;
+} ssa_embedding_bwd_args;
+
+int32_t ssa_embedding_bwd(const ssa_embedding_bwd_args* args, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -53,6 +53,7 @@ EXPORTED_SYMBOLS = (
     "ssa_rmsnorm_bwd",
     "ssa_swiglu",
     "ssa_cross_entropy",
+    "ssa_embedding_bwd",
 )
 
 ABI_VERSION = 6
@@ -199,6 +200,19 @@ class CrossEntropyArgs(ctypes.Structure):
     ]
 
 
+class EmbeddingBwdArgs(ctypes.Structure):
+    """ssa_embedding_bwd_args of include/ssa_decoder_ops.h."""
+
+    _fields_ = [
+        ("ids", ctypes.c_void_p),
+        ("dy", ctypes.c_void_p),
+        ("grad", ctypes.c_void_p),
+        ("tokens", ctypes.c_int32),
+        ("vocab", ctypes.c_int32),
+        ("hidden", ctypes.c_int32),
+    ]
+
+
 class VarlenFwdArgs(ctypes.Structure):
     _fields_ = [("dense", FwdArgs), ("cu_seqlens", ctypes.c_void_p), ("total_tokens", ctypes.c_int32)]
 
@@ -253,7 +267,7 @@ def _declare(lib: ctypes.CDLL) -> None:
     for name, argt in (("ssa_varlen_fwd", VarlenFwdArgs), ("ssa_varlen_bwd", VarlenBwdArgs),
                        ("ssa_decode", DecodeArgs), ("ssa_rope", RopeArgs), ("ssa_rmsnorm_fwd", RmsNormFwdArgs),
                        ("ssa_rmsnorm_bwd", RmsNormBwdArgs), ("ssa_swiglu", SwigluArgs),
-                       ("ssa_cross_entropy", CrossEntropyArgs)):
+                       ("ssa_cross_entropy", CrossEntropyArgs), ("ssa_embedding_bwd", EmbeddingBwdArgs)):
         fn = getattr(lib, name)
         fn.restype = ctypes.c_int32
         fn.argtypes = [ctypes.POINTER(argt), ctypes.c_void_p]

@@ -423,6 +423,186 @@ __global__ __launch_bounds__(256) void xent_bwd_kernel(const T* __restrict__ log
   }
 }
 
+// ---------------------------------------------------------------------------
+// Gradient of an fp32 embedding table: one workgroup per 64 table rows and 256
+// columns, one float4 of columns per lane.  It walks the token ids (L2 hits),
+// keeps its own tokens in LDS in token order, sorts them by row (stable) and
+// writes each of its rows once: the sum of the named dy rows, or zero.  The four
+// waves share the sorted list evenly, sixteen loads in flight each whatever rows
+// they belong to, so frequent tokens that sit together do not make a chain; a row
+// cut by a wave's end is put together in LDS.  A list that may not hold another
+// chunk is added to the rows and started again.  All sums in a fixed order.
+// Bound by the table's write.  Against PyTorch's fill and add, us by tokens (drawn
+// evenly; all the same): 65536 x 2048 table (537 MB) 2048: 254 -> 99; 300 -> 148,
+// 3072: 338 -> 106; 410 -> 190; 32000 x 1024 1000: 80 -> 28; 116 -> 49.
+typedef float emb4 __attribute__((ext_vector_type(4)));
+constexpr int kEmbRows = 64, kEmbCols = 256, kEmbChunk = 1024, kEmbList = 2 * kEmbChunk, kEmbLoads = 16;
+constexpr int kEmbMaxTokens = 1 << 26;  // a list entry: token << 6 | row
+
+__global__ __launch_bounds__(256) void embedding_bwd_kernel(const int64_t* __restrict__ ids,
+                                                            const float* __restrict__ dy, float* __restrict__ grad,
+                                                            int T, int V, int H, int slabs) {
+  __shared__ uint32_t list[kEmbList], sorted[kEmbList];
+  __shared__ volatile int hist[4][kEmbRows];
+  __shared__ int place[4][kEmbRows];
+  __shared__ int wave_count[4], head_row[4];
+  __shared__ emb4 part[4][64];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const uint64_t below = (1ull << lane) - 1;
+  const int r0 = static_cast<int>(blockIdx.x / slabs) * kEmbRows;
+  const int nrows = min(kEmbRows, V - r0);
+  const int col = static_cast<int>(blockIdx.x % slabs) * kEmbCols + lane * 4;
+  const bool on = col < H;
+
+  constexpr int PER = kEmbChunk / 256;
+  int64_t id[PER];
+  auto load_ids = [&](int base) {
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+      const int t = base + wave * (kEmbChunk / 4) + i * 64 + lane;
+      id[i] = t < T ? ids[t] : -1;
+    }
+  };
+  load_ids(0);
+  int n = 0;
+  bool first = true;
+  for (int base = 0; base < T; base += kEmbChunk) {
+    // this chunk's tokens of these rows, in token order
+    bool hit[PER];
+    uint32_t entry[PER];
+    uint64_t mask[PER];
+    int count = 0;
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+      hit[i] = id[i] >= r0 && id[i] < r0 + nrows;
+      entry[i] = static_cast<uint32_t>(base + wave * (kEmbChunk / 4) + i * 64 + lane) << 6 |
+                 static_cast<uint32_t>(id[i] - r0);
+      mask[i] = __ballot(hit[i]);
+      count += __popcll(mask[i]);
+    }
+    load_ids(base + kEmbChunk);
+    if (lane == 0) wave_count[wave] = count;
+    __syncthreads();
+    int pos = n;
+    for (int w = 0; w < wave; ++w) pos += wave_count[w];
+    n += (wave_count[0] + wave_count[1]) + (wave_count[2] + wave_count[3]);
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+      if (hit[i]) list[pos + __popcll(mask[i] & below)] = entry[i];
+      pos += __popcll(mask[i]);
+    }
+    __syncthreads();
+    if (n <= kEmbList - kEmbChunk && base + kEmbChunk < T) continue;
+
+    // Stable sort by row: rank of each entry among its wave's earlier ones of the
+    // row, then the row's and the wave's place.  (The next chunk writes `list`
+    // after its first barrier, which every wave reaches after all of this.)
+    hist[wave][lane] = 0;
+    const int quarter = ((n + 255) / 256) * 64;
+    constexpr int GR = kEmbList / 256;
+    uint32_t ent[GR];
+    int rank[GR];
+#pragma unroll
+    for (int i = 0; i < GR; ++i) {
+      if (i * 64 >= quarter) break;
+      const int k = wave * quarter + i * 64 + lane;
+      const bool have = k < n;
+      ent[i] = have ? list[k] : 0u;
+      const int r = ent[i] & 63;
+      uint64_t same = __ballot(have);
+#pragma unroll
+      for (int b = 0; b < 6; ++b) {
+        const uint64_t bit = __ballot(r >> b & 1);
+        same &= r >> b & 1 ? bit : ~bit;
+      }
+      const int before = hist[wave][r];
+      rank[i] = before + __popcll(same & below);
+      if (have && (same >> lane) == 1) hist[wave][r] = rank[i] + 1;  // the group's last of the row
+    }
+    __syncthreads();
+    const int h0 = hist[0][lane], h1 = hist[1][lane], h2 = hist[2][lane], h3 = hist[3][lane];
+    int end = h0 + h1 + h2 + h3;  // of row `lane` in the sorted list
+    const uint64_t has = __ballot(end != 0);
+    const int total = end;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+      const int up = __shfl_up(end, off, 64);
+      if (lane >= off) end += up;
+    }
+    const int start = end - total;
+    place[wave][lane] = start + (wave > 0 ? h0 : 0) + (wave > 1 ? h1 : 0) + (wave > 2 ? h2 : 0);
+    if (lane == 0) head_row[wave] = -1;
+#pragma unroll
+    for (int i = 0; i < GR; ++i) {
+      if (i * 64 >= quarter) break;
+      if (wave * quarter + i * 64 + lane < n) sorted[place[wave][ent[i] & 63] + rank[i]] = ent[i];
+    }
+    __syncthreads();
+
+    emb4* const row0 = reinterpret_cast<emb4*>(grad + static_cast<int64_t>(r0) * H + col);
+    auto at = [&](int r) { return row0 + static_cast<int64_t>(r) * (H / 4); };
+    if (first && on)
+      for (int r = wave; r < nrows; r += 4)
+        if (!(has >> r & 1)) *at(r) = emb4{};
+    auto emit = [&](int r, emb4 g) {
+      if (on) *at(r) = first ? g : *at(r) + g;
+    };
+    const int k0 = n * wave / 4, k1 = n * (wave + 1) / 4;
+    int cur = -1;
+    emb4 sum = {}, acc = {};  // of `cur`: whole batches, this batch (shorter chains round less)
+    // `cur` ends: its sum to its row, or (begun in an earlier wave) to that wave
+    auto close = [&]() {
+      if (cur < 0) return;
+      if (__builtin_amdgcn_readlane(start, cur) >= k0) {
+        emit(cur, sum + acc);
+      } else {
+        part[wave][lane] = sum + acc;
+        if (lane == 0) head_row[wave] = cur;
+      }
+    };
+    for (int k = k0; k < k1; k += kEmbLoads) {
+      const int cnt = min(kEmbLoads, k1 - k);
+      const uint32_t mine = sorted[k + min(lane, cnt - 1)];
+      emb4 v[kEmbLoads];
+#pragma unroll
+      for (int j = 0; j < kEmbLoads; ++j) {
+        v[j] = emb4{};
+        if (j < cnt) {
+          const uint32_t e = __builtin_amdgcn_readlane(mine, j);
+          if (on) v[j] = *reinterpret_cast<const emb4*>(dy + static_cast<int64_t>(e >> 6) * H + col);
+        }
+      }
+#pragma unroll
+      for (int j = 0; j < kEmbLoads; ++j) {
+        if (j < cnt) {
+          const int r = __builtin_amdgcn_readlane(mine, j) & 63;
+          if (r != cur) {
+            close();
+            cur = r;
+            sum = emb4{};
+            acc = v[j];
+          } else {
+            acc += v[j];
+          }
+        }
+      }
+      sum += acc;
+      acc = emb4{};
+    }
+    const bool open = cur >= 0 && __builtin_amdgcn_readlane(end, max(cur, 0)) > k1 &&
+                      __builtin_amdgcn_readlane(start, max(cur, 0)) >= k0;
+    if (!open) close();
+    __syncthreads();
+    if (open) {
+      for (int w = wave + 1; w < 4; ++w)
+        if (head_row[w] == cur) sum += part[w][lane];
+      emit(cur, sum);
+    }
+    n = 0;
+    first = false;
+  }
+}
+
 int32_t check_norm(const void* x, const void* w, const void* a, const void* b, int32_t T, int32_t H, int32_t dtype) {
   if (x == nullptr || w == nullptr || a == nullptr || b == nullptr) return SSA_OPS_ERR_NULL_POINTER;
   if (T <= 0 || H <= 0 || H % 4 != 0 || H > kNormMaxHidden) return SSA_OPS_ERR_SHAPE;
@@ -542,5 +722,19 @@ extern "C" int32_t ssa_cross_entropy(const ssa_cross_entropy_args* a, void* stre
                          static_cast<const _Float16*>(a->logits), lab, a->lse, a->scale,
                          static_cast<_Float16*>(a->dlogits), a->vocab);
   }
+  return hipGetLastError() == hipSuccess ? SSA_OPS_OK : SSA_OPS_ERR_LAUNCH;
+}
+
+extern "C" int32_t ssa_embedding_bwd(const ssa_embedding_bwd_args* a, void* stream) {
+  if (a == nullptr || a->ids == nullptr || a->dy == nullptr || a->grad == nullptr) return SSA_OPS_ERR_NULL_POINTER;
+  if (a->tokens <= 0 || a->tokens > kEmbMaxTokens || a->vocab <= 0 || a->hidden <= 0 || a->hidden % 4 != 0)
+    return SSA_OPS_ERR_SHAPE;
+  if (!aligned(a->ids, 8) || !aligned(a->dy, 16) || !aligned(a->grad, 16)) return SSA_OPS_ERR_ALIGNMENT;
+  const int64_t slabs = (static_cast<int64_t>(a->hidden) + kEmbCols - 1) / kEmbCols;
+  const int64_t grid = (static_cast<int64_t>(a->vocab) + kEmbRows - 1) / kEmbRows * slabs;
+  if (grid > INT32_MAX) return SSA_OPS_ERR_SHAPE;
+  hipLaunchKernelGGL(embedding_bwd_kernel, dim3(static_cast<uint32_t>(grid)), dim3(256), 0,
+                     static_cast<hipStream_t>(stream), static_cast<const int64_t*>(a->ids), a->dy, a->grad, a->tokens,
+                     a->vocab, a->hidden, static_cast<int>(slabs));
   return hipGetLastError() == hipSuccess ? SSA_OPS_OK : SSA_OPS_ERR_LAUNCH;
 }
