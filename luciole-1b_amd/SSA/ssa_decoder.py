@@ -278,7 +278,8 @@ class _EmbeddingFn(torch.autograd.Function):
     @staticmethod
     def backward(ctx, dy):
         (ids,) = ctx.saved_tensors
-        if torch.is_grad_enabled() or not _plain(dy):  # a gradient of the gradient, a batch of gradients
+        # a traced call, a gradient of the gradient, a batch of gradients
+        if torch.compiler.is_compiling() or torch.is_grad_enabled() or not _plain(dy):
             return None, torch.ops.aten.embedding_dense_backward(dy, ids, ctx.vocab, -1, False)
         dy2 = dy.reshape(-1, dy.shape[-1]).contiguous()
         if dy2.data_ptr() % 16:
@@ -290,8 +291,7 @@ def _plain(t: torch.Tensor) -> bool:
     """An ordinary tensor outside every transform and tracer."""
     return (type(t) in (torch.Tensor, nn.Parameter) and not torch._C._functorch.is_functorch_wrapped_tensor(t)
             and torch._C._functorch.peek_interpreter_stack() is None and torch._C._len_torch_dispatch_stack() == 0
-            and torch.autograd.forward_ad._current_level < 0 and not torch.compiler.is_compiling()
-            and torch._C._get_tracing_state() is None)
+            and torch.autograd.forward_ad._current_level < 0 and torch._C._get_tracing_state() is None)
 
 
 class TokenEmbedding(nn.Embedding):
@@ -306,10 +306,11 @@ class TokenEmbedding(nn.Embedding):
 
     def forward(self, ids):
         w = self.weight
-        if (torch.is_grad_enabled() and w.requires_grad and w.is_cuda and w.dtype == torch.float32
-                and w.shape[1] % 4 == 0 and ids.is_cuda and self.TOKENS[0] <= ids.numel() <= self.TOKENS[1]
-                and self.padding_idx is None and self.max_norm is None and not self.scale_grad_by_freq
-                and not self.sparse and _plain(w) and _plain(ids)):
+        if (not torch.compiler.is_compiling() and torch.is_grad_enabled() and w.requires_grad and w.is_cuda
+                and w.dtype == torch.float32 and w.shape[1] % 4 == 0 and ids.is_cuda
+                and self.TOKENS[0] <= ids.numel() <= self.TOKENS[1] and self.padding_idx is None
+                and self.max_norm is None and not self.scale_grad_by_freq and not self.sparse
+                and _plain(w) and _plain(ids)):
             return _EmbeddingFn.apply(ids, w)
         return super().forward(ids)
 
