@@ -9,7 +9,8 @@
 // X_streamed^T w on v_mfma_f32_32x32x16.  The scores take the 16-bit inputs as
 // they are (exact in fp32).  The weights w (P or dS') are fp32 and go in as the
 // sum of two 16-bit halves, hi + lo, each multiplied (relative error 2^-17 in
-// bf16, 2^-22 in fp16): no probability is rounded to 16 bits.
+// bf16, 2^-22 of a row's largest weight in fp16): no probability is rounded to 16
+// bits.
 //
 // Schedule.  A wave's fragments and accumulators take 200 to 330 registers, so
 // a SIMD holds one wave, which has to hide its own latencies.  An iteration has
@@ -47,10 +48,10 @@ __device__ __forceinline__ void for_ticks(std::integer_sequence<int, I...>, F f)
 template <typename T>
 struct Mat16 {
   static constexpr bool F16 = !__is_same(T, __bf16);
-  // fp16 holds 2^-24 .. 65504: probabilities are scaled up so that the halves
-  // of all that matter stay normal (against M at most 1; against the forward's
-  // lazily moved running max at most PSUM); bf16 has fp32's range.
-  static constexpr float P_SHIFT = F16 ? 12.f : 0.f, FWD_SHIFT = F16 ? 4.f : 0.f;
+  // fp16 holds 2^-24 .. 65504: the forward's probabilities are scaled up so that
+  // the halves of all that matter in a row stay normal (against the lazily moved
+  // running max at most PSUM); bf16 has fp32's range.
+  static constexpr float FWD_SHIFT = F16 ? 4.f : 0.f;
   static constexpr float PSUM = F16 ? 32768.f : kPsumLimit;
   typedef typename Vec8<T>::type frag;
   typedef T v4 __attribute__((ext_vector_type(4)));
@@ -122,10 +123,14 @@ struct Mat16 {
   }
 };
 
-// dS' of any size on the fp16 halves: a power of two per wave, set by the first
-// block with a nonzero weight and lowered (exactly) whenever a larger one
-// comes, keeps the largest weight seen below 2^15; the accumulators hold the
-// scaled sums.  bf16 needs none.
+// Weights of any size on the fp16 halves: a power of two per owned row (a lane
+// pair), set by its first block with a nonzero weight and lowered (exactly)
+// whenever a larger one comes, keeps the row's largest weight seen below 2^15;
+// the accumulators hold the scaled sums.  Each row keeps 2^-22 of its own
+// weights that way, however large its neighbours' are (one scale for the 32 rows
+// of a wave left a row of 2^-28 of their size 2^-10; the wave-wide maximum
+// also took a shuffle per step: fp16 backward of 2 x 8/2 x 2048 causal 895 ->
+// 718 us).  bf16 has fp32's range and needs none.
 template <typename T>
 struct WeightScale {
   float s = 0.f;
@@ -133,17 +138,15 @@ struct WeightScale {
     float a = 0.f;
 #pragma unroll
     for (int r = 0; r < 16; ++r) a = fmaxf(a, fabsf(w[r]));
-    if (__any(a * s > 32768.f || (s == 0.f && a > 0.f))) {  // wave-uniform
-#pragma unroll
-      for (int off = 32; off > 0; off >>= 1) a = fmaxf(a, __shfl_xor(a, off, 64));
+    a = fminf(pair_max(a), 3.0e38f);
+    const bool move = a * s > 32768.f || (s == 0.f && a > 0.f);
+    if (__any(move)) {
       int ex = 0;  // a = m 2^ex, m in [1/2, 1)
       (void)frexpf(a, &ex);
-      const float sn = ldexpf(1.f, min(15 - ex, 60));
-      if (s != 0.f) {
-        const float f = sn / s;
+      const float sn = move ? ldexpf(1.f, min(15 - ex, 60)) : s;
+      const float f = s != 0.f ? sn / s : 1.f;
 #pragma unroll
-        for (int d = 0; d < kND; ++d) acc[d] *= f;
-      }
+      for (int d = 0; d < kND; ++d) acc[d] *= f;
       s = sn;
     }
 #pragma unroll
@@ -441,7 +444,7 @@ __device__ __forceinline__ void dkdv_d256_body(const BwdParams& p, char* smem, f
         };
         auto B = [&](int e) {
           Lv[e] = copysignf(Lv[e], s[e]);
-          pv[e] = fast_exp2(fmaf(n, Lv[e], (DK ? 0.f : M::P_SHIFT) - mv[e >> 2][e & 3]));
+          pv[e] = fast_exp2(fmaf(n, Lv[e], -mv[e >> 2][e & 3]));
           if constexpr (decltype(masked)::value) {
             const int qi = q0 + crow(e, hh);
             pv[e] = qi < N && key < N && (!CAUSAL || key <= qi) ? pv[e] : 0.f;
@@ -454,10 +457,10 @@ __device__ __forceinline__ void dkdv_d256_body(const BwdParams& p, char* smem, f
             wv[e] = dt * rv[e];
             tdn = fmaf(dt, Lv[e], tdn);
             tdb = fmaf(wv[e], s[e], tdb);
-            if constexpr (!M::F16) w.put(e, wv[e]);
           } else {
-            w.put(e, pv[e]);
+            wv[e] = pv[e];
           }
+          if constexpr (!M::F16) w.put(e, wv[e]);
         };
         if (t < 16) A(t);
         if (t >= 1 && t < 17) B(t - 1);
@@ -482,15 +485,13 @@ __device__ __forceinline__ void dkdv_d256_body(const BwdParams& p, char* smem, f
         const float y2 = tdb - db_c, t2 = db_acc + y2;
         db_c = (t2 - db_acc) - y2;
         db_acc = t2;
-        if constexpr (M::F16) {
-          ws.apply(wv, acc);
-#pragma unroll
-          for (int e = 0; e < 16; ++e) w.put(e, wv[e]);
-        }
-        mat.outer(q_at(qs), w, acc);
-      } else {
-        mat.outer(d_at(ds), w, acc);
       }
+      if constexpr (M::F16) {
+        ws.apply(wv, acc);
+#pragma unroll
+        for (int e = 0; e < 16; ++e) w.put(e, wv[e]);
+      }
+      mat.outer(DK ? q_at(qs) : d_at(ds), w, acc);
     } else if (next) {
       next_scores(qs1, ds1, [](auto) {});
     }
@@ -504,8 +505,8 @@ __device__ __forceinline__ void dkdv_d256_body(const BwdParams& p, char* smem, f
   if (key < N) {
     const Tensor4& o = DK ? p.dk : p.dv;
     T* row = static_cast<T*>(const_cast<void*>(o.ptr)) + sv.off(o, b) + hk * o.sh + key * o.ss;
-    float scale = DK ? p.scale * n * bv : exp2f(-M::P_SHIFT);
-    if constexpr (DK && M::F16) scale *= ws.inverse();
+    float scale = DK ? p.scale * n * bv : 1.f;
+    if constexpr (M::F16) scale *= ws.inverse();
     store_own<T, kD>(acc, scale, row, hh);
   }
   if constexpr (DK) {
