@@ -312,9 +312,15 @@ __global__ __launch_bounds__(256) void ssa_fwd_d256_kernel(FwdParams p) {
   merge_parts<kND, kKW>(acc, reinterpret_cast<float*>(smem), qw, kw, lane);
   __syncthreads();
   if (kw == 0 && wq0 < N) {
+    const bool bad = row_nonfinite<kND>(acc);
     T* og = static_cast<T*>(const_cast<void*>(p.o.ptr)) + sv.off(p.o, b) + h * p.o.sh;
     store_rows_via_lds<T, kD>(acc, 1.f / l, [&](int r) { return lds0 + qw * (32 * kD * 2) + r * (kD * 2); },
                               og + static_cast<int64_t>(wq0) * p.o.ss, p.o.ss, N - wq0, lane);
+    if (SSA_RARE(__any(bad)) && bad && qrow < N) {
+      __builtin_amdgcn_s_waitcnt(0);  // after the row's first store
+      row_fwd<T, kD>(og + qrow * p.o.ss, 1.f / l, qg + qrow * p.q.ss, kg, p.k.ss, vg, p.v.ss, CAUSAL ? qrow : N - 1, n,
+                     c, ref - M::FWD_SHIFT, hh);
+    }
     if (hh == 0 && qrow < N) p.m[sv.mrow(b, h, p.Hq, p.T, p.N) + qrow] = m + (log2f(l) - M::FWD_SHIFT);
   }
 }
@@ -506,8 +512,16 @@ __device__ __forceinline__ void dkdv_d256_body(const BwdParams& p, char* smem, f
     const Tensor4& o = DK ? p.dk : p.dv;
     T* row = static_cast<T*>(const_cast<void*>(o.ptr)) + sv.off(o, b) + hk * o.sh + key * o.ss;
     float scale = DK ? p.scale * n * bv : 1.f;
+    const float whole = scale;
     if constexpr (M::F16) scale *= ws.inverse();
-    store_own<T, kD>(acc, scale, row, hh);
+    const bool bad = row_nonfinite<kND>(acc, DK ? dn_acc + db_acc : 0.f);
+    if (!bad) store_own<T, kD>(acc, scale, row, hh);
+    if (SSA_RARE(__any(bad)) && bad) {
+      dn_c = db_c = 0.f;
+      row_dkdv<T, kD, CAUSAL>(p, sv, b, hk, key, n, c, DK ? row : nullptr, whole, DK ? nullptr : row, dn_acc, db_acc,
+                              hh);
+      if (hh != 0) dn_acc = db_acc = 0.f;  // both lanes of the pair have the whole sums
+    }
   }
   if constexpr (DK) {
     // dn / db partial of this key block: lane butterfly, then the waves in order
@@ -677,9 +691,15 @@ __global__ __launch_bounds__(256) void ssa_bwd_dq_d256_kernel(BwdParams p) {
   merge_parts<kND, kKW>(dq, reinterpret_cast<float*>(smem), qw, kw, lane);
   __syncthreads();
   if (kw == 0 && wq0 < N) {
+    const bool bad = row_nonfinite<kND>(dq);
     T* dqg = static_cast<T*>(const_cast<void*>(p.dq.ptr)) + sv.off(p.dq, b) + h * p.dq.sh;
     store_rows_via_lds<T, kD>(dq, p.scale * n * bv, [&](int r) { return lds0 + qw * (32 * kD * 2) + r * (kD * 2); },
                               dqg + static_cast<int64_t>(wq0) * p.dq.ss, p.dq.ss, N - wq0, lane);
+    if (SSA_RARE(__any(bad)) && bad && qrow < N) {
+      __builtin_amdgcn_s_waitcnt(0);  // after the row's first store
+      row_dq<T, kD>(dqg + qrow * p.dq.ss, p.scale * n * bv, qg + qrow * p.q.ss, dog + qrow * p.dout.ss, kg, p.k.ss, vg,
+                    p.v.ss, CAUSAL ? qrow : N - 1, n, c, mi, di, hh);
+    }
   }
 }
 

@@ -218,7 +218,12 @@ __global__ __launch_bounds__(256) void ssa_fwd_f32_kernel(FwdParams p) {
   }
   if (kw == 0 && qrow < N) {
     float* og = static_cast<float*>(const_cast<void*>(p.o.ptr)) + sv.off(p.o, b) + h * p.o.sh;
-    store_own<float, D>(acc, 1.f / l, og + qrow * p.o.ss, hh);  // every row has a key (causal: itself)
+    const bool bad = row_nonfinite<ND>(acc);
+    if (!bad)
+      store_own<float, D>(acc, 1.f / l, og + qrow * p.o.ss, hh);  // every row has a key (causal: itself)
+    if (SSA_RARE(__any(bad)) && bad)
+      row_fwd<float, D>(og + qrow * p.o.ss, 1.f / l, qg + qrow * p.q.ss, kg, p.k.ss, vg, p.v.ss, CAUSAL ? qrow : N - 1,
+                        n, c, m == -INFINITY ? 0.f : m, hh);
     if (hh == 0) p.m[sv.mrow(b, h, p.Hq, p.T, p.N) + qrow] = m + log2f(l);
   }
 }
@@ -367,14 +372,40 @@ __device__ __forceinline__ void dkdv_f32_body(const BwdParams& p, char* smem, fl
   }
   if constexpr (DO_DK) merge_parts<ND, QS>(dk, reinterpret_cast<float*>(smem), kg4, qs, lane);
   if constexpr (DO_DV) merge_parts<ND, QS>(dv, reinterpret_cast<float*>(smem), kg4, qs, lane);
-  if (qs == 0 && key < N) {
-    if constexpr (DO_DK) {
-      float* dkr = static_cast<float*>(const_cast<void*>(p.dk.ptr)) + sv.off(p.dk, b) + hk * p.dk.sh + key * p.dk.ss;
-      store_own<float, D>(dk, p.scale * n * bv, dkr, hh);
+  // keys with non-finite sums in any of their waves (ssa_rows.hpp): the first of these waves sums them again
+  bool bad = DO_DK && row_nonfinite<ND>(dk, dn_acc + db_acc);
+  if constexpr (DO_DV) bad = bad || row_nonfinite<ND>(dv);
+  if (QS > 1) {
+    if (lane == 0) red[2][wave] = __any(bad) ? 1.f : 0.f;
+    __syncthreads();
+    float any_bad = 0.f;
+#pragma unroll
+    for (int w = 0; w < NWV; ++w) any_bad += red[2][w];
+    if (SSA_RARE(any_bad != 0.f)) {
+      int* rows = reinterpret_cast<int*>(smem);  // [QS][4][32]
+      if (hh == 0) rows[(qs * 4 + kg4) * 32 + l32] = bad;
+      __syncthreads();
+#pragma unroll
+      for (int i = 0; i < QS; ++i) bad = bad || rows[(i * 4 + kg4) * 32 + l32] != 0;
     }
-    if constexpr (DO_DV) {
-      float* dvr = static_cast<float*>(const_cast<void*>(p.dv.ptr)) + sv.off(p.dv, b) + hk * p.dv.sh + key * p.dv.ss;
-      store_own<float, D>(dv, 1.f, dvr, hh);
+  }
+  if (key < N) {
+    float *dkr = nullptr, *dvr = nullptr;
+    if constexpr (DO_DK)
+      dkr = static_cast<float*>(const_cast<void*>(p.dk.ptr)) + sv.off(p.dk, b) + hk * p.dk.sh + key * p.dk.ss;
+    if constexpr (DO_DV)
+      dvr = static_cast<float*>(const_cast<void*>(p.dv.ptr)) + sv.off(p.dv, b) + hk * p.dv.sh + key * p.dv.ss;
+    if (!bad) {
+      if constexpr (DO_DK)
+        if (qs == 0) store_own<float, D>(dk, p.scale * n * bv, dkr, hh);
+      if constexpr (DO_DV)
+        if (qs == 0) store_own<float, D>(dv, 1.f, dvr, hh);
+    }
+    if (SSA_RARE(__any(bad)) && bad) {
+      dn_acc = dn_c = db_acc = db_c = 0.f;
+      if (qs == 0)
+        row_dkdv<float, D, CAUSAL>(p, sv, b, hk, key, n, c, dkr, p.scale * n * bv, dvr, dn_acc, db_acc, hh);
+      if (hh != 0) dn_acc = db_acc = 0.f;  // both lanes of the pair have the whole sums
     }
   }
   if constexpr (DO_DK) {
@@ -409,7 +440,7 @@ template <int D, bool CAUSAL, bool ROLES>
 __global__ __launch_bounds__((Cfg<D>::DKDV_THREADS)) void ssa_bwd_dkdv_f32_kernel(BwdParams p) {
   using C = Cfg<D>;
   __shared__ __attribute__((aligned(1024))) char smem[2 * C::DKDV_STAGE];
-  __shared__ float red[2][8];
+  __shared__ float red[3][8];
   if constexpr (ROLES) {
     // dK workgroups (three products per block) before the lighter dV ones
     const int half = gridDim.x / 2;
@@ -508,7 +539,12 @@ __global__ __launch_bounds__(256) void ssa_bwd_dq_f32_kernel(BwdParams p) {
   merge_parts<ND, KW>(dq, reinterpret_cast<float*>(smem), qw, kw, lane);
   if (kw == 0 && qrow < N) {
     float* dqr = static_cast<float*>(const_cast<void*>(p.dq.ptr)) + sv.off(p.dq, b) + h * p.dq.sh + qrow * p.dq.ss;
-    store_own<float, D>(dq, p.scale * n * bv, dqr, hh);
+    const bool bad = row_nonfinite<ND>(dq);
+    if (!bad)
+      store_own<float, D>(dq, p.scale * n * bv, dqr, hh);
+    if (SSA_RARE(__any(bad)) && bad)
+      row_dq<float, D>(dqr, p.scale * n * bv, qg + qrow * p.q.ss, dog + qrow * p.dout.ss, kg, p.k.ss, vg, p.v.ss,
+                       CAUSAL ? qrow : N - 1, n, c, mi, di, hh);
   }
 }
 
