@@ -45,12 +45,14 @@ HIPCC_FLAGS = [
 # VALU reads S and dP there without copies); the dK/dV accumulators are held in
 # AGPRs by the inline assembly of ssa_common.hpp (mfma32_acc / acc_fence).
 # ssa_fwd.hip: the same for its 4-wave head-dim-128 workgroups (one wave per
-# SIMD); ssa_d256.hip: score results in VGPRs (dK/dV 424 -> 195 us, no spills).
+# SIMD); ssa_d256.hip: score results in VGPRs (dK/dV 424 -> 195 us, no spills);
+# ssa_f32.hip: the same (head dim 256 causal forward 751 -> 614 us at 16 x 2048).
 SOURCE_FLAGS = {
     "ssa_bwd.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
     "ssa_bwd_dkdv2w.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
     "ssa_fwd.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
     "ssa_d256.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
+    "ssa_f32.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
 }
 
 

@@ -33,6 +33,11 @@
 // grid of one sequence then fills the chip, and causal blocks balance.
 // Measured (us, the earlier vector-ALU kernels -> these): fp32, B = 1, H = 16,
 // N = 1024, D = 64 causal: forward 376 -> 43, dK/dV 498 -> 124, dQ 380 -> 53.
+// Head dim 256 (K, V, Q or dO fragments and accumulators of 128 registers each):
+// 16 x 2048 causal forward 3800 -> 614, backward 8920 -> 1950; 16 x 4096 14700 ->
+// 1310 and 35500 -> 5440.  It fits one wave's registers with the scores in VGPRs
+// (_build.py) and LDS reads kept near their use, but for 91 spills of the causal
+// dQ; without either it spilled up to 340 (751 and 2350 at 2048).
 #include "ssa_rows.hpp"
 
 namespace ssa {
@@ -62,21 +67,36 @@ struct Mat {
   }
   // fragment f: columns 8 f + 4 hh + (0..3), one MFMA step each
   __device__ static __forceinline__ frag load(const float* row, int f, int hh) { return ld4(row + 8 * f + 4 * hh); }
-  __device__ __forceinline__ f32x16 scores(uint32_t lds, const frag* own) const {
-    const RowBase<LD> r = at_tile(rb, lds);
-    f32x16 s = f32x16{};
+  // Chains of 32 columns added in a tree: one chain over the row was off by more
+  // than the vector-ALU kernels' partial sums (against 64 bits, N = 64 causal, of
+  // the norm: dq at head dim 128 3.4e-7 and 256 4.4e-7 in one chain, 2.5e-7 and
+  // 2.7e-7 so, 2.6e-7 and 2.8e-7 there).
+  template <int F0, int N>
+  __device__ __forceinline__ f32x16 chain(const RowBase<LD>& r, const frag* own) const {
+    if constexpr (N > 4) {
+      const f32x16 a = chain<F0, N / 2>(r, own);
+      // head dim 256 fills the registers: no LDS reads ahead over a chain or an outer step
+      if constexpr (D >= 256) __builtin_amdgcn_sched_barrier(0);
+      return a + chain<F0 + N / 2, N / 2>(r, own);
+    } else {
+      f32x16 s = f32x16{};
 #pragma unroll
-    for (int f = 0; f < NF; ++f) {
-      const f32x4 a = tile_read_row<LD, f32x4>(r, 0, f);
+      for (int f = F0; f < F0 + N; ++f) {
+        const f32x4 a = tile_read_row<LD, f32x4>(r, 0, f);
 #pragma unroll
-      for (int e = 0; e < 4; ++e) s = __builtin_amdgcn_mfma_f32_32x32x2f32(a[e], own[f][e], s, 0, 0, 0);
+        for (int e = 0; e < 4; ++e) s = __builtin_amdgcn_mfma_f32_32x32x2f32(a[e], own[f][e], s, 0, 0, 0);
+      }
+      return s;
     }
-    return s;
+  }
+  __device__ __forceinline__ f32x16 scores(uint32_t lds, const frag* own) const {
+    return chain<0, NF>(at_tile(rb, lds), own);
   }
   __device__ __forceinline__ void outer(uint32_t lds, const float* w, f32x16* acc) const {
     const uint32_t b[2] = {opaque(ob[0] + lds), opaque(ob[1] + lds)};
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
+      if constexpr (D >= 256) __builtin_amdgcn_sched_barrier(0);
       const uint32_t imm = (r >> 3) * 256 + (r & 3) * 16;
 #pragma unroll
       for (int db = 0; db < ND; ++db) {
