@@ -62,7 +62,8 @@ int32_t ssa_rope(const ssa_rope_args* args, void* stream);
  * contiguous, 16-byte aligned; hidden a multiple of 4, at most 4096.  y is
  * written in out_dtype (0 bf16, 1 fp16, 2 fp32: the dtype of the next GEMM's
  * input), rstd [rows] fp32 is kept for the backward.  The backward reads dy
- * in dy_dtype, writes dx fp32 [rows, hidden] and dweight fp32 [hidden]; its
+ * in dy_dtype (8-byte aligned), writes dx fp32 [rows, hidden] (16-byte aligned;
+ * it may be x, or dy if that is fp32) and dweight fp32 [hidden]; its
  * workspace holds ssa_rmsnorm_workspace_floats(rows, hidden) fp32 partial
  * weight gradients, summed in a fixed order (deterministic).
  */
