@@ -27,7 +27,8 @@ int32_t check_tensor(const ssa_tensor4& t, bool required) {
 
 // Sizes every launcher can take with int32 arithmetic: sequence lengths up
 // to 2^30 (so N + tile - 1 fits), at most 2^28 units of 128 rows per grid
-// (the smallest workgroup covers 64 rows, so every grid size fits), and --
+// (the smallest workgroup covers 32 rows, so every grid has at most 2^30; the
+// fp32-precision launchers fold theirs, folded_grid()), and --
 // checked separately -- at most INT32_MAX query rows per launch over dense
 // batches (B * Hq * N) and packed streams (Hq * T), the rows the Delta kernels
 // cover.

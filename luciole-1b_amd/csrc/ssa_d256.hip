@@ -175,7 +175,7 @@ __global__ __launch_bounds__(256) void ssa_fwd_d256_kernel(FwdParams p) {
   const int l32 = lane & 31, hh = lane >> 5;
   const int kw = wave % kKW, qw = wave / kKW;
   const int nqb = (p.N + kBM - 1) / kBM, grid = nqb * p.B * p.Hq;
-  const int block = blockIdx.y * gridDim.x + blockIdx.x;
+  const int block = folded_block();
   if (block >= grid) return;
   const Place pl(block, grid, nqb, p.B, p.cu_seqlens != nullptr);
   const int b = pl.b, h = pl.h, hk = h / (p.Hq / p.Hkv);
@@ -550,11 +550,11 @@ __global__ __launch_bounds__(256) void ssa_bwd_dkdv_d256_kernel(BwdParams p) {
   __shared__ __attribute__((aligned(1024))) char smem[kDkdvLds];
   __shared__ float red[2][4];
   // the dK workgroups (three products per block) before the lighter dV ones
-  const int half = gridDim.x / 2, block = blockIdx.x;
-  if (block < half)
-    dkdv_d256_body<T, CAUSAL, true>(p, smem, red, block, half);
-  else
-    dkdv_d256_body<T, CAUSAL, false>(p, smem, red, block - half, half);
+  const int grid = dkdv_key_blocks(p.N) * p.B * p.Hkv, block = folded_block();
+  if (block < grid)
+    dkdv_d256_body<T, CAUSAL, true>(p, smem, red, block, grid);
+  else if (block < 2 * grid)
+    dkdv_d256_body<T, CAUSAL, false>(p, smem, red, block - grid, grid);
 }
 
 // ---------------------------------------------------------------------------
@@ -571,7 +571,7 @@ __global__ __launch_bounds__(256) void ssa_bwd_dq_d256_kernel(BwdParams p) {
   const int l32 = lane & 31, hh = lane >> 5;
   const int kw = wave % kKW, qw = wave / kKW;
   const int nqb = (p.N + kBM - 1) / kBM, grid = nqb * p.B * p.Hq;
-  const int block = blockIdx.y * gridDim.x + blockIdx.x;
+  const int block = folded_block();
   if (block >= grid) return;
   if (p.fuse_reduce && block == 0) {  // the backward's dn / db sums, before the first load (reduce_partials_body)
     reduce_partials_body(p.partials, static_cast<int64_t>(p.B) * p.Hkv * dkdv_key_blocks(p.N), p.dn, p.db,
@@ -716,15 +716,15 @@ __global__ __launch_bounds__(256) void ssa_bwd_dq_d256_kernel(BwdParams p) {
   } while (0)
 
 hipError_t launch_fwd_d256(const FwdParams& p, int dtype, int D, bool causal, hipStream_t s) {
-  SSA_D256_LAUNCH(ssa_fwd_d256_kernel, row_grid((p.N + kBM - 1) / kBM * p.B * p.Hq));
+  SSA_D256_LAUNCH(ssa_fwd_d256_kernel, folded_grid((p.N + kBM - 1) / kBM * p.B * p.Hq, 256));
 }
 
 hipError_t launch_bwd_dkdv_d256(const BwdParams& p, int dtype, int D, bool causal, hipStream_t s) {
-  SSA_D256_LAUNCH(ssa_bwd_dkdv_d256_kernel, dim3(dkdv_key_blocks(p.N) * p.B * p.Hkv * 2));
+  SSA_D256_LAUNCH(ssa_bwd_dkdv_d256_kernel, folded_grid(dkdv_key_blocks(p.N) * p.B * p.Hkv * 2, 256));
 }
 
 hipError_t launch_bwd_dq_d256(const BwdParams& p, int dtype, int D, bool causal, hipStream_t s) {
-  SSA_D256_LAUNCH(ssa_bwd_dq_d256_kernel, row_grid((p.N + kBM - 1) / kBM * p.B * p.Hq));
+  SSA_D256_LAUNCH(ssa_bwd_dq_d256_kernel, folded_grid((p.N + kBM - 1) / kBM * p.B * p.Hq, 256));
 }
 
 }  // namespace ssa

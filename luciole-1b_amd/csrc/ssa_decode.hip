@@ -280,7 +280,8 @@ template <typename T, int D>
 static hipError_t launch_decode_t(const DecodeParams& p, hipStream_t s) {
   const int grid = DecodePlan<D>::grid(p);
   hipLaunchKernelGGL((ssa_decode_kernel<T, D>), dim3(grid), dim3(DecodeCfg<D>::NW * 64), 0, s, p);
-  if (p.splits > kMergeFewSplits)
+  // the wide form's 256 threads a head stay below 2^32 in one launch
+  if (p.splits > kMergeFewSplits && static_cast<int64_t>(p.B) * p.Hq < (1 << 24))
     hipLaunchKernelGGL((ssa_decode_merge_kernel<T, D>), dim3(p.B * p.Hq), dim3(256), 0, s, p);
   else if (p.splits > 1)
     hipLaunchKernelGGL((ssa_decode_merge_few_kernel<T, D>), dim3(p.B * p.Hq), dim3(128), 0, s, p);

@@ -119,6 +119,7 @@ struct Cfg {
   static constexpr int QW = 4 / KW;  // waves on different rows (forward, dQ): 32 QW rows per workgroup
   static constexpr int BM = 32 * QW, BN = 32 * KW;
   static constexpr int LDS_BYTES = 2 * KW * 2 * BB;
+  static_assert(BM >= 32, "grids of 2^28 units of 128 rows stay below 2^31 workgroups");
   // dK/dV: two waves per 32 keys up to head dim 64 (two waves per SIMD)
   static constexpr int QS = D <= 64 ? 2 : 1;
   static constexpr int DKDV_THREADS = 256 * QS;
@@ -141,7 +142,7 @@ __global__ __launch_bounds__(256) void ssa_fwd_f32_kernel(FwdParams p) {
   const int l32 = lane & 31, hh = lane >> 5;
   const int kw = wave % KW, qw = wave / KW;
   const int nqb = (p.N + BM - 1) / BM, grid = nqb * p.B * p.Hq;
-  const int block = blockIdx.y * gridDim.x + blockIdx.x;
+  const int block = folded_block();
   if (block >= grid) return;
   const Place pl(block, grid, nqb, p.B, p.cu_seqlens != nullptr);
   const int b = pl.b, h = pl.h, hk = h / (p.Hq / p.Hkv);
@@ -461,15 +462,15 @@ __global__ __launch_bounds__((Cfg<D>::DKDV_THREADS)) void ssa_bwd_dkdv_f32_kerne
   using C = Cfg<D>;
   __shared__ __attribute__((aligned(1024))) char smem[2 * C::DKDV_STAGE];
   __shared__ float red[3][8];
+  const int block = folded_block(), grid = dkdv_key_blocks(p.N) * p.B * p.Hkv;
   if constexpr (ROLES) {
     // dK workgroups (three products per block) before the lighter dV ones
-    const int half = gridDim.x / 2;
-    if (static_cast<int>(blockIdx.x) < half)
-      dkdv_f32_body<D, CAUSAL, true, false>(p, smem, red, blockIdx.x, half);
-    else
-      dkdv_f32_body<D, CAUSAL, false, true>(p, smem, red, blockIdx.x - half, half);
-  } else {
-    dkdv_f32_body<D, CAUSAL, true, true>(p, smem, red, blockIdx.x, gridDim.x);
+    if (block < grid)
+      dkdv_f32_body<D, CAUSAL, true, false>(p, smem, red, block, grid);
+    else if (block < 2 * grid)
+      dkdv_f32_body<D, CAUSAL, false, true>(p, smem, red, block - grid, grid);
+  } else if (block < grid) {
+    dkdv_f32_body<D, CAUSAL, true, true>(p, smem, red, block, grid);
   }
 }
 
@@ -487,7 +488,7 @@ __global__ __launch_bounds__(256) void ssa_bwd_dq_f32_kernel(BwdParams p) {
   const int l32 = lane & 31, hh = lane >> 5;
   const int kw = wave % KW, qw = wave / KW;
   const int nqb = (p.N + BM - 1) / BM, grid = nqb * p.B * p.Hq;
-  const int block = blockIdx.y * gridDim.x + blockIdx.x;
+  const int block = folded_block();
   if (block >= grid) return;
   if (p.fuse_reduce && block == 0) {  // the backward's dn / db sums, before the first load (reduce_partials_body)
     reduce_partials_body(p.partials, static_cast<int64_t>(p.B) * p.Hkv * dkdv_key_blocks(p.N), p.dn, p.db,
@@ -594,7 +595,7 @@ static void launch_pre(const BwdParams& p, hipStream_t s) {
 
 }  // namespace
 
-#define SSA_F32_ROW_GRID(DD) row_grid((p.N + Cfg<DD>::BM - 1) / Cfg<DD>::BM * p.B * p.Hq)
+#define SSA_F32_ROW_GRID(DD) folded_grid((p.N + Cfg<DD>::BM - 1) / Cfg<DD>::BM * p.B * p.Hq, 256)
 #define SSA_F32_THREADS(DD) 256
 
 // dK and dV in one workgroup (four products a block) or in two (three and two).
@@ -610,13 +611,15 @@ constexpr int kRolesGrid = 128;
 template <int D, bool CAUSAL>
 static hipError_t launch_dkdv(const BwdParams& p, hipStream_t s) {
   const int grid = dkdv_key_blocks(p.N) * p.B * p.Hkv;
-  const dim3 threads(Cfg<D>::DKDV_THREADS);
+  constexpr int threads = Cfg<D>::DKDV_THREADS;
   if (D >= 256 || grid <= (CAUSAL ? 2 : 1) * kRolesGrid) {
-    hipLaunchKernelGGL((ssa_bwd_dkdv_f32_kernel<D, CAUSAL, true>), dim3(2 * grid), threads, 0, s, p);
+    hipLaunchKernelGGL((ssa_bwd_dkdv_f32_kernel<D, CAUSAL, true>), folded_grid(2 * grid, threads), dim3(threads), 0,
+                       s, p);
     return hipGetLastError();
   }
   if constexpr (D < 256)
-    hipLaunchKernelGGL((ssa_bwd_dkdv_f32_kernel<D, CAUSAL, false>), dim3(grid), threads, 0, s, p);
+    hipLaunchKernelGGL((ssa_bwd_dkdv_f32_kernel<D, CAUSAL, false>), folded_grid(grid, threads), dim3(threads), 0,
+                       s, p);
   return hipGetLastError();
 }
 

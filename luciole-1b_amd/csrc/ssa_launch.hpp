@@ -88,6 +88,18 @@ inline int decode_splits(int B, int Hq, int Hkv, int cap, int requested) {
   return static_cast<int>((cap + sk - 1) / sk);
 }
 
+// A launch takes fewer than 2^32 threads along x: grids of n workgroups fold over
+// y from 2^31 threads on.  The kernel's block is folded_block(), and those from
+// n on have no work.
+inline dim3 folded_grid(int n, int threads) {
+  const int most = (1 << 30) / threads * 2;
+  const int y = (n - 1) / most + 1;
+  return dim3((n - 1) / y + 1, y);
+}
+#ifdef __HIPCC__
+__device__ __forceinline__ int folded_block() { return blockIdx.y * gridDim.x + blockIdx.x; }
+#endif
+
 // Number of key blocks of the dK/dV kernel (each writes one dn and one db partial).
 __host__ __device__ inline int dkdv_key_blocks(int N) { return (N + 127) / 128; }
 

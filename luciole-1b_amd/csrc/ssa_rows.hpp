@@ -205,13 +205,6 @@ __device__ __forceinline__ void row_dkdv(const BwdParams& p, const SeqView& sv, 
   }
 }
 
-// A launch takes fewer than 2^32 threads along x: larger row grids (from 2^23
-// workgroups) fold over y.
-inline dim3 row_grid(int n) {
-  const int y = (n + (1 << 23) - 1) >> 23;
-  return dim3((n + y - 1) / y, y);
-}
-
 }  // namespace
 
 }  // namespace ssa
