@@ -172,14 +172,6 @@ def _has_ds_path(dtype: torch.dtype, head_dim: int) -> bool:
     return dtype != torch.float32 and head_dim <= 128
 
 
-# Workspaces up to this size are taken without asking for the device's
-# headroom: the allocator's statistics and the driver's free memory take about
-# 90 us, more than the kernels of a small problem, and this is a thousandth of
-# the card.  It is the call's last allocation, is free again when the call
-# returns, and where it fails dq recomputes the scores.
-_DS_UNASKED_BYTES = 256 << 20
-
-
 def _ds_mode(ds):
     """The dS' policy of a call: 0 (never), -1 (always), or the byte cap."""
     if ds is not None:
@@ -192,16 +184,14 @@ def _ds_mode(ds):
     return max(0, int(os.environ.get("SSA_BWD_DS_MAX_BYTES", str(16 << 30))))
 
 
-def _ds_unasked(ds):
-    """The largest dS' workspace the extension module may take for this call."""
-    mode = _ds_mode(ds)
-    return min(mode, _DS_UNASKED_BYTES)
-
-
 def _device_headroom(device) -> int | None:
     """Bytes a new allocation on ``device`` can take without the caching
     allocator asking the driver for more than it has: the driver's free memory
     plus what the allocator holds reserved but unused.  None if unknown."""
+    index = torch.device(device).index
+    room = _lib.native().headroom(torch.cuda.current_device() if index is None else index)
+    if room is not None:
+        return room
     try:
         free, _ = torch.cuda.mem_get_info(device)
         return int(free) + int(torch.cuda.memory_reserved(device)) - int(torch.cuda.memory_allocated(device))
@@ -223,8 +213,6 @@ def _use_ds_workspace(nbytes: int, head_dim: int, ds, device=None) -> bool:
         return True
     if not 0 < nbytes <= limit:
         return False
-    if nbytes <= _DS_UNASKED_BYTES:
-        return True
     room = _device_headroom(device) if device is not None else None
     return room is None or nbytes <= room // 2
 
@@ -311,7 +299,7 @@ def ssa_flash_attn_backward(q, k, v, out, dout, m, softmax_scale, ssa_n, ssa_b, 
     """SSA attention backward.  Returns ``(dq, dk, dv, dn, db)``; dn/db are 0-d fp32 tensors.
     ``ds``: keep dS' in a workspace (True / False; None: the ``SSA_BWD_DS`` policy)."""
     if q.is_cuda:
-        r = _lib.native().bwd(q, k, v, out, dout, m, softmax_scale, ssa_n, ssa_b, bool(causal), _ds_unasked(ds),
+        r = _lib.native().bwd(q, k, v, out, dout, m, softmax_scale, ssa_n, ssa_b, bool(causal), _ds_mode(ds),
                               *_current())
         if r is not None:
             return _native_result(r, "ssa_bwd")
@@ -434,7 +422,7 @@ def ssa_flash_attn_varlen_backward(q, k, v, out, dout, m, cu_seqlens, max_seqlen
     ``ds``: keep dS' in a workspace (True / False; None: the ``SSA_BWD_DS`` policy)."""
     if q.is_cuda:
         r = _lib.native().varlen_bwd(q, k, v, out, dout, m, cu_seqlens, max_seqlen, softmax_scale, ssa_n, ssa_b,
-                                     bool(causal), _ds_unasked(ds), *_current())
+                                     bool(causal), _ds_mode(ds), *_current())
         if r is not None:
             return _native_result(r, "ssa_varlen_bwd")
     cu, docs, T, Hq, Hkv, D, max_seqlen = _check_varlen_inputs(q, k, v, cu_seqlens, max_seqlen)

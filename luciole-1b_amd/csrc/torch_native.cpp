@@ -18,6 +18,7 @@
 #include <ATen/core/Tensor.h>
 #include <ATen/ops/empty.h>
 #include <ATen/ops/empty_like.h>
+#include <c10/core/CachingDeviceAllocator.h>
 #include <c10/core/DispatchKeySet.h>
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
@@ -232,12 +233,51 @@ PyObject* forward(PyObject*, PyObject* const* a, Py_ssize_t n) {
   END_HANDLE_TH_ERRORS
 }
 
+// Bytes that the caching allocator of GPU `dev` holds unused and, with `driver`,
+// those that the driver has free besides.  Throws where they are not known.
+int64_t free_bytes(int dev, bool driver) {
+  c10::DeviceAllocator* a = c10::getDeviceAllocator(c10::DeviceType::CUDA);
+  const auto index = static_cast<c10::DeviceIndex>(dev);
+  const auto st = a->getDeviceStats(index);
+  constexpr auto all = static_cast<size_t>(c10::CachingAllocator::StatType::AGGREGATE);
+  const int64_t held = st.reserved_bytes[all].current - st.allocated_bytes[all].current;
+  return driver ? held + static_cast<int64_t>(a->getMemoryInfo(index).first) : held;
+}
+
+// Whether the dS' workspace stays within half of the headroom: what the allocator
+// holds often answers it without the driver.  The same question through
+// torch.cuda takes 90 us and leaves some hundred Python objects, enough for a full
+// collection by the interpreter (40 ms) every hundred steps or so: a 4 x 16 x 4096
+// x 128 step 5 to 25 of a process took 2.5 ms for 1.4.
+bool ds_fits(int64_t nbytes, int dev) {
+  try {
+    return nbytes <= free_bytes(dev, false) / 2 || nbytes <= free_bytes(dev, true) / 2;
+  } catch (const std::exception&) {
+    return true;  // unknown: the byte cap alone
+  }
+}
+
+// headroom(dev) -> bytes | None (unknown)
+PyObject* headroom(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  Args in{a, 0, nullptr};
+  const int64_t dev = n == 1 ? in.integer(0) : -1;
+  if (n != 1 || !in.good || dev < 0 || dev > 127) return none();
+  int64_t bytes = 0;
+  try {
+    pybind11::gil_scoped_release unlocked;
+    bytes = free_bytes(static_cast<int>(dev), true);
+  } catch (const std::exception&) {
+    return none();
+  }
+  return PyLong_FromLongLong(bytes);
+}
+
 // bwd(q, k, v, out, dout, m, scale, n, b, causal, ds_max, dev, stream)
 // varlen_bwd(q, k, v, out, dout, m, cu, max_seqlen, scale, n, b, causal, ds_max, dev, stream)
 //   -> (dq, dk, dv, dn, db) | status | None
 // ds_max: the dS' workspace is used up to that many bytes (0: never, -1: any
-// size); a larger one returns None (the Python path then asks for the device's
-// headroom).  Where its allocation fails, dq recomputes the scores.
+// size) and half of the device's headroom.  Without one, or where its allocation
+// (the call's last) fails, dq recomputes the scores.
 template <bool VARLEN>
 PyObject* backward(PyObject*, PyObject* const* a, Py_ssize_t n) {
   HANDLE_TH_ERRORS
@@ -273,7 +313,8 @@ PyObject* backward(PyObject*, PyObject* const* a, Py_ssize_t n) {
   int64_t ds_bytes = 0;
   if (p.dtype != SSA_DTYPE_FP32 && p.D <= 128 && ds_max != 0) {  // the fp32-precision kernels use none
     ds_bytes = VARLEN ? abi.varlen_ds_bytes(batch, Hq, seqlen, T, causal) : abi.ds_bytes(batch, Hq, seqlen, causal);
-    if (ds_bytes <= 0 || (ds_max > 0 && ds_bytes > ds_max)) return none();
+    if (ds_bytes <= 0) return none();
+    if (ds_max > 0 && ds_bytes > ds_max) ds_bytes = 0;
   }
   if (count <= 0) return none();
   at::Tensor dq, dk, dv, dn, db;
@@ -294,7 +335,7 @@ PyObject* backward(PyObject*, PyObject* const* a, Py_ssize_t n) {
     if (ds_bytes > 0) {
       if (ds_max < 0) {
         ds = bytes(ds_bytes, *q);
-      } else {
+      } else if (ds_fits(ds_bytes, in.dev)) {
         try {
           ds = bytes(ds_bytes, *q);
         } catch (const c10::OutOfMemoryError&) {
@@ -419,6 +460,7 @@ PyMethodDef methods[] = {{"bind", SSA_FAST(&bind)},
                          {"varlen_bwd", SSA_FAST(&backward<true>)},
                          {"decode", SSA_FAST(&decode)},
                          {"decode_splits", SSA_FAST(&decode_splits)},
+                         {"headroom", SSA_FAST(&headroom)},
                          {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_ssa_native", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
 
