@@ -90,9 +90,8 @@ def build_native() -> Path:
     import torch
     from torch.utils import cpp_extension
 
-    cxx = os.environ.get("CXX") or shutil.which("g++") or shutil.which("c++")
-    if cxx is None:
-        raise RuntimeError("no C++ compiler: the SSA launch extension cannot be built")
+    # host code: any C++17 compiler, hipcc's own where there is no other
+    cxx = os.environ.get("CXX") or shutil.which("g++") or shutil.which("c++") or _hipcc()
     tmp = NATIVE_PATH.with_suffix(".so.tmp")
     cmd = [cxx, "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-fvisibility=hidden",
            f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}"]

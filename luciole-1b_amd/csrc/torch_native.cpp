@@ -23,6 +23,7 @@
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
 #include <torch/csrc/utils/pybind.h>
+#include <torch/headeronly/version.h>
 
 #include <cstring>
 
@@ -466,4 +467,15 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "_ssa_native", nullptr, -1, methods
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit__ssa_native() { return PyModule_Create(&module); }
+// ABI_VERSION and TORCH_VERSION: what the module was built for, checked by its
+// loader (SSA/_lib.py) before bind().
+PyMODINIT_FUNC PyInit__ssa_native() {
+  PyObject* m = PyModule_Create(&module);
+  if (m == nullptr) return nullptr;
+  if (PyModule_AddIntConstant(m, "ABI_VERSION", SSA_ABI_VERSION) < 0 ||
+      PyModule_AddStringConstant(m, "TORCH_VERSION", TORCH_VERSION) < 0) {
+    Py_DECREF(m);
+    return nullptr;
+  }
+  return m;
+}
