@@ -166,21 +166,74 @@ def test_errors_are_the_python_paths(gpu):
 
 
 @pytest.mark.gpu
+def test_takes_the_plain_calls(gpu):
+    """Every fast entry point runs a call in a plain layout itself, and leaves the
+    odd ones (rows not 16-byte aligned, transposed, another dtype) to Python."""
+    from SSA import _lib
+    from SSA.ssa_hip_kernel import _current
+
+    nat = _lib.native()
+    g = torch.Generator(device=gpu).manual_seed(2)
+    n = torch.tensor(1.5, device=gpu)
+    views = dict(_views(torch.randn(1, 2, 40, 64, generator=g, device=gpu).bfloat16()))
+    plain = {"contiguous", "s b h d", "padded rows"}
+    for name, q in views.items():
+        k = v = views["contiguous"]
+        got = nat.fwd(q, k, v, 0.125, n, n, True, *_current())
+        assert (got is not None) == (name in plain), name
+        out, m = nat.fwd(k, k, v, 0.125, n, n, True, *_current())
+        for ds_max in (0, -1, 1 << 30):
+            grads = nat.bwd(k, k, v, out, q, m, 0.125, n, n, True, ds_max, *_current())
+            assert (grads is not None) == (name in plain), (name, ds_max)
+            assert grads is None or len(grads) == 5
+    t = views["contiguous"][0].transpose(0, 1).contiguous()  # [T, H, D]
+    cu = torch.tensor([0, 10, 40], dtype=torch.int32, device=gpu)
+    out, m = nat.varlen_fwd(t, t, t, cu, 30, 0.125, n, n, True, *_current())
+    assert len(nat.varlen_bwd(t, t, t, out, t, m, cu, 30, 0.125, n, n, True, 1 << 30, *_current())) == 5
+    assert nat.varlen_fwd(t, t, t, cu.long(), 30, 0.125, n, n, True, *_current()) is None
+    kc = views["contiguous"]
+    qd, lens = kc[:, :, 0].contiguous(), torch.tensor([40], dtype=torch.int32, device=gpu)
+    assert nat.decode(qd, kc, kc, lens, 0.125, n, n, 0, *_current())[0].shape == qd.shape
+    assert nat.decode(qd.float(), kc, kc, lens, 0.125, n, n, 0, *_current()) is None
+
+
+def _busy(x, ms):
+    """About `ms` milliseconds of matrix products on the current stream."""
+    for _ in range(ms):
+        x = torch.mm(x, x)  # 8192^3: about a millisecond each in fp16
+    return x
+
+
+@pytest.mark.gpu
 def test_runs_on_the_current_stream(gpu):
     """A launch on a side stream waits for that stream's work and for no other's."""
-    from SSA import ssa_flash_attn_forward
+    from SSA import _lib, ssa_flash_attn_forward
 
+    assert not isinstance(_lib.native(), _lib.PythonPath)
     g = torch.Generator(device=gpu).manual_seed(1)
-    q, k, v = (torch.randn(1, 2, 64, 64, generator=g, device=gpu).bfloat16() for _ in range(3))
+    q, k, v, other = (torch.randn(1, 2, 64, 64, generator=g, device=gpu).bfloat16() for _ in range(4))
+    load = torch.zeros(8192, 8192, device=gpu, dtype=torch.float16)
     n = torch.tensor(1.5, device=gpu)
     want, _ = ssa_flash_attn_forward(q, k, v, 0.125, n, n)
+    _busy(load, 2)
     side = torch.cuda.Stream(device=gpu)
-    side.wait_stream(torch.cuda.current_stream(gpu))
+    late = other.clone()
+    torch.cuda.synchronize()
+    # the side stream's earlier work: one copy, long after the host has launched the forward
     with torch.cuda.stream(side):
-        late = torch.zeros_like(q)
-        for _ in range(20):
-            late.copy_(q * 1.0)
+        _busy(load, 30)
+        late.copy_(q)
         got, _ = ssa_flash_attn_forward(late, k, v, 0.125, n, n)
-    torch.cuda.current_stream(gpu).wait_stream(side)
+    torch.cuda.synchronize()
+    assert torch.equal(got, want)
+    # no other stream's: the default stream is still busy when the side stream is done
+    done, busy = torch.cuda.Event(), torch.cuda.Event()
+    _busy(load, 60)
+    busy.record()
+    with torch.cuda.stream(side):
+        got, _ = ssa_flash_attn_forward(q, k, v, 0.125, n, n)
+        done.record()
+    done.synchronize()
+    assert not busy.query()
     torch.cuda.synchronize()
     assert torch.equal(got, want)
