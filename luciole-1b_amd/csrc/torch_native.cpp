@@ -245,14 +245,18 @@ int64_t free_bytes(int dev, bool driver) {
   return driver ? held + static_cast<int64_t>(a->getMemoryInfo(index).first) : held;
 }
 
-// Whether the dS' workspace stays within half of the headroom: what the allocator
-// holds often answers it without the driver.  The same question through
-// torch.cuda takes 90 us and leaves some hundred Python objects, enough for a full
-// collection by the interpreter (40 ms) every hundred steps or so: a 4 x 16 x 4096
-// x 128 step 5 to 25 of a process took 2.5 ms for 1.4.
+// Whether the dS' workspace stays within half of the headroom.  What the allocator
+// holds often answers it without the driver (1 us for 5 to 13, by host): half of it,
+// or all of it up to 256 MiB, a thousandth of the card, as a repeated call finds its
+// last workspace there.  The same question through torch.cuda takes 90 us and leaves
+// some hundred Python objects, enough for a full collection by the interpreter (40
+// ms) every hundred steps or so: steps 6 to 25 of a 4 x 16 x 4096 x 128 forward and
+// backward took 2.5 ms for 1.4.
+constexpr int64_t kSmallWorkspace = int64_t{256} << 20;
 bool ds_fits(int64_t nbytes, int dev) {
   try {
-    return nbytes <= free_bytes(dev, false) / 2 || nbytes <= free_bytes(dev, true) / 2;
+    const int64_t held = free_bytes(dev, false);
+    return nbytes <= held / 2 || (nbytes <= kSmallWorkspace && nbytes <= held) || nbytes <= free_bytes(dev, true) / 2;
   } catch (const std::exception&) {
     return true;  // unknown: the byte cap alone
   }
