@@ -431,7 +431,7 @@ def main():
     ap.add_argument("--kernel-iters", type=int, default=50, help="launches per kernel for per-kernel timing")
     ap.add_argument("--no-cpu-baseline", action="store_true")
     ap.add_argument("--dtype", default="bf16", choices=["bf16", "fp16", "fp32"],
-                    help="fp32 (dense shapes only): the fp32 vector-ALU kernels, against the fp32 peak")
+                    help="fp32 (dense shapes only): the fp32 kernels (matrix cores in fp32), against the fp32 peak")
     ap.add_argument("--counters-summary", nargs="+", metavar="DB",
                     help="print the per-kernel counter table of rocprofv3 --pmc databases of --pmc-pass runs "
                          "(the table of profiles/ssa_counters_<config>.md) and exit")
@@ -464,7 +464,7 @@ def main():
     world = int(os.environ.get("WORLD_SIZE", "1"))
     if args.gpus != 1 or world != 1:
         print(json.dumps({"error": "this build runs on one GPU only: the SSA op has no cross-GPU "
-                                   "communication (see DESIGN.md, sharding); run with --gpus 1"}))
+                                   "communication; run with --gpus 1"}))
         sys.exit(2)
 
     import torch

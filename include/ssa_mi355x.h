@@ -63,10 +63,12 @@ enum {
  * 819-825) -- runs on kernels of its own (head dims 16, 32, 64, 128, 256)
  * that keep every product and sum in fp32: full precision, a fraction of the
  * bf16 throughput.  bf16 / fp16 at head dim 256 (the reference takes every
- * power-of-two head dim, ssa_triton_kernel.py:761-764) run on the same
- * kernels, with fp32 probabilities and score gradients.  On these
- * fp32-precision kernels the dS' workspace is not used (dq recomputes the scores); the
- * decode step takes bf16 / fp16 at head dims 32, 64, 128.
+ * power-of-two head dim, ssa_triton_kernel.py:761-764) run on others of their
+ * own: probabilities and score gradients are computed in fp32 and enter the
+ * 16-bit products as the sum of two 16-bit halves (to 2^-17 of each in bf16, to
+ * 2^-22 of the row's largest in fp16).  Neither uses the dS' workspace (dq
+ * recomputes the scores).  The decode step takes bf16 / fp16 at head dims 32, 64,
+ * 128.
  */
 enum { SSA_DTYPE_BF16 = 0, SSA_DTYPE_FP16 = 1, SSA_DTYPE_FP32 = 2 };
 
@@ -285,8 +287,9 @@ typedef struct ssa_decode_args {
 } ssa_decode_args;
 
 /* Key splits ssa_decode uses for num_splits = `requested` (0 = library
-   choice: about 256 workgroups, splits of at least 256 keys); 0 on invalid
-   arguments. */
+   choice: about 256 workgroups, splits of at least 256 keys; a lone short cache
+   is 10 to 30 % faster with splits of 128, as the Python layer asks for); 0 on
+   invalid arguments. */
 int32_t ssa_decode_num_splits(int32_t batch, int32_t heads_q, int32_t heads_kv, int32_t capacity,
                               int32_t requested);
 

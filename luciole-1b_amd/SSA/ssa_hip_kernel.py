@@ -35,8 +35,9 @@ no score, dP or Delta, and the results are sliced back (the decode step is not
 offered at D = 16).  fp32 inputs (the reference's fp32-operand path) run on
 kernels of their own for head dims 16-256 (fp32 matrix-core products and sums),
 without the dS' workspace; bf16 / fp16 at head dim 256 (the largest power of
-two the reference takes) run on the same kernels, whose fp32 weights enter the
-16-bit products as two halves; the decode step takes bf16 / fp16 only.  Errors:
+two the reference takes) run on kernels of their own, also without it, whose fp32
+weights enter the 16-bit products as two halves; the decode step takes bf16 / fp16
+only.  Errors:
 ``AssertionError`` for ``Hq % Hkv != 0`` and a non-power-of-two head dim, as in
 the reference; ``ValueError`` for other head dims and other dtypes.
 """

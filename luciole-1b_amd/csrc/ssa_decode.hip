@@ -194,8 +194,10 @@ __global__ __launch_bounds__(DecodeCfg<D>::NW * 64) void ssa_decode_kernel(Decod
 // partials in split order, out = sum_s acc_s 2^(m_s - M) / sum_s l_s 2^(m_s - M),
 // in one pass with the running maximum (each split's loads are independent of
 // the running state, so they can all be in flight at once).  Up to
-// kMergeFewSplits splits: 8.0 against 8.5 us of a 2-split step (16 x 24/8 x 700 x
-// 32) by the wide form below.
+// kMergeFewSplits splits; against the wide form below the whole step is shorter by
+// 0.6 to 0.75 us at 2 splits, 0.3 to 0.5 at 3, 0.1 to 0.2 at 4 (one of six shapes
+// even), and longer by 0 to 0.2 at 5, 0.2 to 0.4 at 6, 0.7 to 1.0 at 8 (1 x 16 x 128
+// heads to 32 x 32/8 x 128).
 constexpr int kMergeFewSplits = 4;
 template <typename T, int D>
 __global__ __launch_bounds__(128) void ssa_decode_merge_few_kernel(DecodeParams p) {

@@ -4,8 +4,9 @@
 // (training/train/train_ssa_triton/SSA/ssa_triton_kernel.py:40-260).
 //
 // One workgroup = 4 or 8 waves = 128 or 256 query rows of one (batch, q-head);
-// each wave owns 32 query rows, two waves share a SIMD.  K/V tiles of 64 keys
-// live in four LDS buffers filled by direct-to-LDS loads two tiles ahead and
+// each wave owns 32 query rows; two waves share a SIMD, but for 4-wave workgroups at
+// head dim 128, which have a CU each (launch_fwd_t).  K/V tiles of 64 keys live in
+// four LDS buffers filled by direct-to-LDS loads two tiles ahead and
 // shared by the waves (one barrier per tile).  Everything is computed transposed so
 // that a query row lives in a single lane pair (l, l+32):
 //   S^T = K Q^T      (A = K rows from LDS, B = Q^T fragment held in registers)
@@ -75,8 +76,8 @@ struct FwdTile {
 };
 
 // ---------------------------------------------------------------------------
-// Software-pipelined forward.  One workgroup = NW waves = 32 NW query rows, two
-// waves per SIMD; K/V tiles of 64 keys in NB = 4 LDS buffers shared by the
+// Software-pipelined forward.  One workgroup = NW waves = 32 NW query rows, mostly
+// two waves per SIMD; K/V tiles of 64 keys in NB = 4 LDS buffers shared by the
 // waves, one barrier per tile.  Iteration i of a wave issues
 //   MFMA : S_{i+1} = K_{i+1} Q^T   and   O^T += V_{i-1}^T P_{i-1}^T
 //   VALU : SSA transform, online max / sum and P_i = exp2(...) of S_i

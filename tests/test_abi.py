@@ -624,8 +624,8 @@ def test_ds_workspace_policy_leaves_headroom(monkeypatch):
 
 
 def test_ds_path_by_dtype_and_head_dim():
-    """Only the matrix-core kernels (bf16 / fp16, head dims up to 128) use a dS'
-    workspace; fp32 and head dim 256 run the vector-ALU kernels, whose dq recomputes."""
+    """Only the 16-bit kernels (bf16 / fp16, head dims up to 128) use a dS' workspace;
+    the dq of fp32 and of head dim 256 recomputes."""
     import torch
 
     from SSA.ssa_hip_kernel import _has_ds_path

@@ -68,7 +68,7 @@ def test_two_runs_bitwise_equal(gpu, dtype, dq_path, N, causal, layout, D):
 @pytest.mark.parametrize("dtype", ["bf16", "fp32"])
 @pytest.mark.parametrize("causal", [True, False])
 def test_head_dim_256_bitwise_equal(gpu, dtype, causal):
-    """Head dim 256 runs on the vector-ALU kernels: the same fixed-order reductions."""
+    """Head dim 256 runs on kernels of its own: the same fixed-order reductions."""
     from SSA.ssa_triton_kernel import ssa_flash_attn_backward, ssa_flash_attn_forward
 
     label = f"determinism {dtype} N=300 D=256 causal={int(causal)}"

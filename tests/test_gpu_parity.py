@@ -86,7 +86,7 @@ def test_parity_head_dim_16(gpu, dtype, causal, heads, N):
 @pytest.mark.parametrize("heads", [(4, 4), (8, 2)])
 @pytest.mark.parametrize("N", [7, 256])
 def test_parity_fp32(gpu, D, causal, heads, N):
-    """fp32 operands (the reference's fp32 path) on the fp32 vector-ALU kernels,
+    """fp32 operands (the reference's fp32 path) on the fp32 kernels (matrix cores in fp32),
     at the reference's fp32 tolerances (atol 5e-4, rtol 1e-3; dn / db 5e-5 + 1e-4 |ref|)."""
     _check(*_run(gpu, 1, heads[0], heads[1], N, D, torch.float32, causal))
 
@@ -106,9 +106,9 @@ def test_parity_fp32_trained_n(gpu):
 @pytest.mark.parametrize("heads", [(4, 4), (8, 2)])
 @pytest.mark.parametrize("N", [7, 200])
 def test_parity_head_dim_256(gpu, dtype, causal, heads, N):
-    """Head dim 256 (the largest power of two the reference's Triton tiles take) on the
-    fp32-arithmetic vector-ALU kernels: bf16 / fp16 elements widened on load.  N = 200
-    fills the first 64-key pass of a 128-key block and part of the second."""
+    """Head dim 256 (the largest power of two the reference's Triton tiles take): fp32 on
+    the fp32 kernels, bf16 / fp16 on kernels of their own.  N = 200 ends within a
+    128-key block and a 32-row one."""
     _check(*_run(gpu, 1, heads[0], heads[1], N, 256, dtype, causal))
 
 

@@ -79,7 +79,7 @@ CASES = [
     ((129, 31, 200), 4, 2, 128, False),
     ((40, 90, 257), 2, 2, 32, True),
     ((40, 90, 257), 4, 2, 16, True),  # head dim 16: zero-padded onto the D = 32 kernels
-    ((70, 3, 200), 4, 2, 256, True),  # head dim 256: the vector-ALU kernels (the dS' workspace unused)
+    ((70, 3, 200), 4, 2, 256, True),  # head dim 256: kernels of its own (the dS' workspace unused)
 ]
 
 

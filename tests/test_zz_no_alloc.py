@@ -3,7 +3,7 @@ partials in the library's static device scratch, dQ recomputed).
 
 Called through the C ABI on four problems in a row -- each smaller, so each
 runs on the scratch the previous one left behind, the last two on the
-vector-ALU kernels (fp32 at head dim 16, bf16 at head dim 256) -- and
+kernels of fp32 (head dim 16) and of head dim 256 (bf16) -- and
 compared with ssa_bwd on
 the same arguments (recompute path, caller workspaces): bitwise equal, and
 within the parity bar of the fp64 oracle (tests/parity_util.py).  The
@@ -26,7 +26,7 @@ pytestmark = pytest.mark.gpu
 
 CALLS = [
     # B, Hq, Hkv, N, D, causal, dtype: larger first, then smaller (the last two
-    # on the vector-ALU kernels: fp32 to the fp32 bars, bf16 at head dim 256)
+    # on kernels of their own: fp32 to the fp32 bars, bf16 at head dim 256)
     (2, 8, 4, 700, 128, True, torch.bfloat16),
     (1, 4, 2, 200, 64, False, torch.bfloat16),
     (1, 4, 4, 150, 16, True, torch.float32),
