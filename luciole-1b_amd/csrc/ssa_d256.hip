@@ -157,7 +157,7 @@ struct WeightScale {
 
 // Rows per workgroup (forward, dQ): 64, two waves each on alternate 32-row
 // blocks of a 64-row stage, so that one sequence fills the chip.
-constexpr int kKW = 2, kQW = 2, kBM = 32 * kQW, kBN = 32 * kKW, kStage = kKW * kBB;
+constexpr int kKW = 2, kQW = 2, kBM = 32 * kQW, kBN = 32 * kKW;
 
 // ---------------------------------------------------------------------------
 // Forward.  K in two slots and V in two, turned over separately: iteration st
@@ -169,43 +169,30 @@ template <typename T, bool CAUSAL>
 __global__ __launch_bounds__(256) void ssa_fwd_d256_kernel(FwdParams p) {
   using M = Mat16<T>;
   typedef typename M::frag frag;
-  __shared__ __attribute__((aligned(1024))) char smem[4 * kStage];
+  using Plan = RowPlan<kD, 2, CAUSAL, kKW>;
+  using Loads = RowLoads256<CAUSAL, kKW, 2, 2>;
+  __shared__ __attribute__((aligned(1024))) char smem[Loads::LDS_BYTES];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int l32 = lane & 31, hh = lane >> 5;
   const int kw = wave % kKW, qw = wave / kKW;
-  const int nqb = (p.N + kBM - 1) / kBM, grid = nqb * p.B * p.Hq;
   const int block = folded_block();
-  if (block >= grid) return;
-  const Place pl(block, grid, nqb, p.B, p.cu_seqlens != nullptr);
-  const int b = pl.b, h = pl.h, hk = h / (p.Hq / p.Hkv);
-  const SeqView sv(p.cu_seqlens, p.T, p.N, b);
-  const int N = sv.N;
-  const int q0 = (nqb - 1 - pl.rank) * kBM;
-  if (q0 >= N) return;  // packed: past the end of a shorter document
-  const int wq0 = q0 + 32 * qw, qrow = wq0 + l32;
-  const T* qg = static_cast<const T*>(p.q.ptr) + sv.off(p.q, b) + h * p.q.sh;
-  const T* kg = static_cast<const T*>(p.k.ptr) + sv.off(p.k, b) + hk * p.k.sh;
-  const T* vg = static_cast<const T*>(p.v.ptr) + sv.off(p.v, b) + hk * p.v.sh;
+  if (block >= Plan::grid(p)) return;
+  const Plan pl(p, Plan::place(p, block));  // dispatch and K / V loads (ssa_rows_plan.hpp)
+  const SeqView& sv = pl.sv;
+  const int b = pl.b, h = pl.h, N = pl.N, nst = pl.nst;
+  if (pl.empty()) return;  // packed: past the end of a shorter document
+  const Loads ld(p, pl, lane, wave);
+  const int wq0 = pl.q0 + 32 * qw, qrow = wq0 + l32;
+  const T* qg = reinterpret_cast<const T*>(head_rows<2>(sv, p.q, b, h));
+  const T* kg = reinterpret_cast<const T*>(ld.k.g);
+  const T* vg = reinterpret_cast<const T*>(ld.v.g);
   const float n = *p.n_ptr, c = p.scale * *p.b_ptr;
   const uint32_t lds0 = lds_addr(smem);
-  const LoadLane llk(lane, wave, p.k.ss), llv(lane, wave, p.v.ss);
-  const int kv_end = CAUSAL ? min(N, q0 + kBM) : N;
-  const int nst = (kv_end + kBN - 1) / kBN;
-  auto k_at = [&](int st) { return lds0 + (st & 1) * kStage; };
-  auto v_at = [&](int st) { return lds0 + (2 + (st & 1)) * kStage; };
-  auto load_k = [&](int st) {
-    if (st >= nst) return;
-#pragma unroll
-    for (int i = 0; i < kKW; ++i)
-      tile_load_async<kD, 32, 4>(kg, p.k.ss, st * kBN + 32 * i, N, k_at(st) + i * kBB, wave, llk);
-  };
-  auto load_v = [&](int st) {
-    if (st >= nst) return;
-#pragma unroll
-    for (int i = 0; i < kKW; ++i)
-      tile_load_async<kD, 32, 4>(vg, p.v.ss, st * kBN + 32 * i, N, v_at(st) + i * kBB, wave, llv);
-  };
+  auto k_at = [&](int st) { return Loads::k_at(lds0, st & 1); };
+  auto v_at = [&](int st) { return Loads::v_at(lds0, st & 1); };
+  auto load_k = [&](int st) { ld.load_k(pl, st, st & 1, lds0, wave); };
+  auto load_v = [&](int st) { ld.load_v(pl, st, st & 1, lds0, wave); };
   load_k(0);
   load_k(1);
   load_v(0);
@@ -333,25 +320,22 @@ __global__ __launch_bounds__(256) void ssa_fwd_d256_kernel(FwdParams p) {
 // dV (two); the operand of the outer product is held for one block longer.
 // Per valid pair, as in ssa_bwd.hip: P = exp2(n sL - M), dT = P (dP - Delta),
 // dS' = dT / (1 + c|x|).
-constexpr int kDkdvLds = 5 * kBB + 3 * 256;
-
 template <typename T, bool CAUSAL, bool DK>
-__device__ __forceinline__ void dkdv_d256_body(const BwdParams& p, char* smem, float (*red)[4], int block, int grid) {
+__device__ __forceinline__ void dkdv_d256_body(const BwdParams& p, char* smem, float (*red)[4], int block) {
   using M = Mat16<T>;
   typedef typename M::frag frag;
-  constexpr int RQ = DK ? 3 : 2, RD = DK ? 2 : 3;  // ring slots of Q and of dO
+  using Plan = KeyPlan<kD, 2, CAUSAL, 1, 4>;
+  using Ring = KeyRing256<DK>;
+  constexpr int RQ = Ring::RQ, RD = Ring::RD;  // ring slots of Q and of dO
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int l32 = lane & 31, hh = lane >> 5;
   const int nkb = dkdv_key_blocks(p.N);
-  const Place pl(block, grid, nkb, p.B, p.cu_seqlens != nullptr);
-  const int kb = pl.rank, b = pl.b, hk = pl.h, bhk = hk * p.B + b;
-  const int G = p.Hq / p.Hkv;
-  const SeqView sv(p.cu_seqlens, p.T, p.N, b);
-  const int N = sv.N;
+  const Plan pl(p, Plan::place(p, block));  // dispatch and Q / dO loads (ssa_rows_plan.hpp)
+  const SeqView& sv = pl.sv;
+  const int kb = pl.kb, b = pl.b, hk = pl.hk, bhk = pl.bhk, N = pl.N, k0 = pl.k0;
   const int64_t PP = static_cast<int64_t>(p.B) * p.Hkv * nkb;
-  const int k0 = kb * 128;
-  if (k0 >= N) {  // packed: past the end of a shorter document
+  if (pl.empty()) {  // packed: past the end of a shorter document
     if (DK && tid == 0) {
       p.partials[static_cast<int64_t>(bhk) * nkb + kb] = 0.f;
       p.partials[PP + static_cast<int64_t>(bhk) * nkb + kb] = 0.f;
@@ -364,33 +348,14 @@ __device__ __forceinline__ void dkdv_d256_body(const BwdParams& p, char* smem, f
   const float n = *p.n_ptr, bv = *p.b_ptr, c = p.scale * bv;
   const uint32_t lds0 = lds_addr(smem);
   const LoadLane llq(lane, wave, p.q.ss), lld(lane, wave, p.dout.ss);
-  const int qstart = CAUSAL ? k0 : 0;
-  const int nqs = (N - qstart + 31) / 32, nst = G * nqs;
+  const int qstart = pl.qstart, nst = pl.nst;
   // ring slots of stage st: the slot indices of stages st, st + 1 and st + 2
   // are kept, not divided out
-  auto q_at = [&](int slot) { return lds0 + slot * kBB; };
-  auto d_at = [&](int slot) { return lds0 + (RQ + slot) * kBB; };
-  auto md_at = [&](int slot) { return lds0 + 5 * kBB + slot * 256; };
-  int lg = 0, lq = qstart, ls = 0, lq_slot = 0, ld_slot = 0, lm_slot = 0;  // the next stage to load
-  auto load_next = [&]() {
-    if (ls >= nst) return;
-    const int h = hk * G + lg;
-    const T* qg = static_cast<const T*>(p.q.ptr) + sv.off(p.q, b) + h * p.q.sh;
-    const T* dog = static_cast<const T*>(p.dout.ptr) + sv.off(p.dout, b) + h * p.dout.sh;
-    const int64_t mr = sv.mrow(b, h, p.Hq, p.T, p.N);
-    tile_load_async<kD, 32, 4>(qg, p.q.ss, lq, N, q_at(lq_slot), wave, llq);
-    tile_load_async<kD, 32, 4>(dog, p.dout.ss, lq, N, d_at(ld_slot), wave, lld);
-    if (wave == 3) pair32_load_async(p.m + mr, p.delta + mr, lq, N, md_at(lm_slot), lane);
-    ++ls;
-    lq_slot = lq_slot + 1 == RQ ? 0 : lq_slot + 1;
-    ld_slot = ld_slot + 1 == RD ? 0 : ld_slot + 1;
-    lm_slot = lm_slot == 2 ? 0 : lm_slot + 1;
-    lq += 32;
-    if (lq >= N) {
-      lq = qstart;
-      ++lg;
-    }
-  };
+  auto q_at = [&](int slot) { return Ring::q_at(lds0, slot); };
+  auto d_at = [&](int slot) { return Ring::d_at(lds0, slot); };
+  auto md_at = [&](int slot) { return Ring::md_at(lds0, slot); };
+  Ring ring(qstart);  // the next stage to load
+  auto load_next = [&]() { ring.load_next(p, pl, lds0, llq, lld, wave, lane); };
   load_next();
   load_next();
   const M mat(lane);
@@ -547,14 +512,14 @@ __device__ __forceinline__ void dkdv_d256_body(const BwdParams& p, char* smem, f
 
 template <typename T, bool CAUSAL>
 __global__ __launch_bounds__(256) void ssa_bwd_dkdv_d256_kernel(BwdParams p) {
-  __shared__ __attribute__((aligned(1024))) char smem[kDkdvLds];
+  __shared__ __attribute__((aligned(1024))) char smem[KeyRing256<true>::LDS_BYTES];
   __shared__ float red[2][4];
   // the dK workgroups (three products per block) before the lighter dV ones
   const int grid = dkdv_key_blocks(p.N) * p.B * p.Hkv, block = folded_block();
   if (block < grid)
-    dkdv_d256_body<T, CAUSAL, true>(p, smem, red, block, grid);
+    dkdv_d256_body<T, CAUSAL, true>(p, smem, red, block);
   else if (block < 2 * grid)
-    dkdv_d256_body<T, CAUSAL, false>(p, smem, red, block - grid, grid);
+    dkdv_d256_body<T, CAUSAL, false>(p, smem, red, block - grid);
 }
 
 // ---------------------------------------------------------------------------
@@ -565,47 +530,39 @@ template <typename T, bool CAUSAL>
 __global__ __launch_bounds__(256) void ssa_bwd_dq_d256_kernel(BwdParams p) {
   using M = Mat16<T>;
   typedef typename M::frag frag;
-  __shared__ __attribute__((aligned(1024))) char smem[5 * kStage];
+  using Plan = RowPlan<kD, 2, CAUSAL, kKW>;
+  using Loads = RowLoads256<CAUSAL, kKW, 3, 2>;
+  __shared__ __attribute__((aligned(1024))) char smem[Loads::LDS_BYTES];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int l32 = lane & 31, hh = lane >> 5;
   const int kw = wave % kKW, qw = wave / kKW;
-  const int nqb = (p.N + kBM - 1) / kBM, grid = nqb * p.B * p.Hq;
   const int block = folded_block();
-  if (block >= grid) return;
+  if (block >= Plan::grid(p)) return;
   if (p.fuse_reduce && block == 0) {  // the backward's dn / db sums, before the first load (reduce_partials_body)
     reduce_partials_body(p.partials, static_cast<int64_t>(p.B) * p.Hkv * dkdv_key_blocks(p.N), p.dn, p.db,
                          reinterpret_cast<float(*)[256]>(smem), threadIdx.x);
     __syncthreads();
   }
-  const Place pl(block, grid, nqb, p.B, p.cu_seqlens != nullptr);
-  const int b = pl.b, h = pl.h, hk = h / (p.Hq / p.Hkv);
-  const SeqView sv(p.cu_seqlens, p.T, p.N, b);
-  const int N = sv.N;
-  const int q0 = (nqb - 1 - pl.rank) * kBM;
-  if (q0 >= N) return;  // packed: past the end of a shorter document
-  const int wq0 = q0 + 32 * qw, qrow = wq0 + l32;
-  const T* qg = static_cast<const T*>(p.q.ptr) + sv.off(p.q, b) + h * p.q.sh;
-  const T* dog = static_cast<const T*>(p.dout.ptr) + sv.off(p.dout, b) + h * p.dout.sh;
-  const T* kg = static_cast<const T*>(p.k.ptr) + sv.off(p.k, b) + hk * p.k.sh;
-  const T* vg = static_cast<const T*>(p.v.ptr) + sv.off(p.v, b) + hk * p.v.sh;
+  const Plan pl(p, Plan::place(p, block));
+  const SeqView& sv = pl.sv;
+  const int b = pl.b, h = pl.h, N = pl.N, nst = pl.nst;
+  if (pl.empty()) return;  // packed: past the end of a shorter document
+  const Loads ld(p, pl, lane, wave);
+  const int wq0 = pl.q0 + 32 * qw, qrow = wq0 + l32;
+  const T* qg = reinterpret_cast<const T*>(head_rows<2>(sv, p.q, b, h));
+  const T* dog = reinterpret_cast<const T*>(head_rows<2>(sv, p.dout, b, h));
+  const T* kg = reinterpret_cast<const T*>(ld.k.g);
+  const T* vg = reinterpret_cast<const T*>(ld.v.g);
   const int64_t mr = sv.mrow(b, h, p.Hq, p.T, p.N);
   const float n = *p.n_ptr, bv = *p.b_ptr, c = p.scale * bv;
   const uint32_t lds0 = lds_addr(smem);
-  const LoadLane llk(lane, wave, p.k.ss), llv(lane, wave, p.v.ss);
-  const int kv_end = CAUSAL ? min(N, q0 + kBM) : N;
-  const int nst = (kv_end + kBN - 1) / kBN;
-  auto k_at = [&](int slot) { return lds0 + slot * kStage + kw * kBB; };
-  auto v_at = [&](int st) { return lds0 + (3 + (st & 1)) * kStage + kw * kBB; };
+  auto k_at = [&](int slot) { return Loads::k_at(lds0, slot) + kw * kBB; };
+  auto v_at = [&](int st) { return Loads::v_at(lds0, st & 1) + kw * kBB; };
   int ls = 0, lk_slot = 0;  // the next stage to load
   auto load_next = [&]() {
-    if (ls >= nst) return;
-#pragma unroll
-    for (int i = 0; i < kKW; ++i) {
-      tile_load_async<kD, 32, 4>(kg, p.k.ss, ls * kBN + 32 * i, N, lds0 + lk_slot * kStage + i * kBB, wave, llk);
-      tile_load_async<kD, 32, 4>(vg, p.v.ss, ls * kBN + 32 * i, N, lds0 + (3 + (ls & 1)) * kStage + i * kBB, wave,
-                                 llv);
-    }
+    ld.load_k(pl, ls, lk_slot, lds0, wave);
+    ld.load_v(pl, ls, ls & 1, lds0, wave);
     ++ls;
     lk_slot = lk_slot == 2 ? 0 : lk_slot + 1;
   };

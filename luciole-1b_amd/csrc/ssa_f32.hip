@@ -108,22 +108,11 @@ struct Mat {
   }
 };
 
-// Streamed blocks per stage (= waves that share 32 owned rows) of the forward
-// and dQ, and of dK/dV (whose workgroups own 128 keys, the unit of the dn / db
-// partials).  A stage holds two blocks (K and V, or Q and dO) per kw, twice
-// buffered, in at most 128 KB of LDS.
 template <int D>
-struct Cfg {
-  static constexpr int BB = Mat<D>::BLOCK;
-  static constexpr int KW = 4 * BB <= 32768 ? 4 : (BB <= 16384 ? 2 : 1);
-  static constexpr int QW = 4 / KW;  // waves on different rows (forward, dQ): 32 QW rows per workgroup
-  static constexpr int BM = 32 * QW, BN = 32 * KW;
-  static constexpr int LDS_BYTES = 2 * KW * 2 * BB;
-  static_assert(BM >= 32, "grids of 2^28 units of 128 rows stay below 2^31 workgroups");
-  // dK/dV: two waves per 32 keys up to head dim 64 (two waves per SIMD)
-  static constexpr int QS = D <= 64 ? 2 : 1;
-  static constexpr int DKDV_THREADS = 256 * QS;
-  static constexpr int DKDV_STAGE = QS * (2 * BB + 256);  // Q, dO, M[32], Delta[32] per block
+struct Cfg : SplitF32<D> {
+  static constexpr int QW = 4 / SplitF32<D>::KW;  // waves on different rows (forward, dQ): 32 QW rows per workgroup
+  static constexpr int BM = 32 * QW, BN = 32 * SplitF32<D>::KW;
+  static constexpr int DKDV_THREADS = 256 * SplitF32<D>::QS;  // workgroups own 128 keys, the unit of the partials
 };
 
 // ---------------------------------------------------------------------------
@@ -135,38 +124,29 @@ template <int D, bool CAUSAL>
 __global__ __launch_bounds__(256) void ssa_fwd_f32_kernel(FwdParams p) {
   using M = Mat<D>;
   using C = Cfg<D>;
-  constexpr int KW = C::KW, BM = C::BM, BN = C::BN, BB = C::BB, ND = M::ND;
-  __shared__ __attribute__((aligned(1024))) char smem[C::LDS_BYTES];
+  using Plan = RowPlan<D, 4, CAUSAL, C::KW>;
+  using Loads = RowLoadsF32<D, CAUSAL, C::KW>;
+  constexpr int KW = C::KW, BN = C::BN, BB = C::BB, ND = M::ND;
+  __shared__ __attribute__((aligned(1024))) char smem[Loads::LDS_BYTES];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int l32 = lane & 31, hh = lane >> 5;
   const int kw = wave % KW, qw = wave / KW;
-  const int nqb = (p.N + BM - 1) / BM, grid = nqb * p.B * p.Hq;
   const int block = folded_block();
-  if (block >= grid) return;
-  const Place pl(block, grid, nqb, p.B, p.cu_seqlens != nullptr);
-  const int b = pl.b, h = pl.h, hk = h / (p.Hq / p.Hkv);
-  const SeqView sv(p.cu_seqlens, p.T, p.N, b);
-  const int N = sv.N;
-  const int q0 = (nqb - 1 - pl.rank) * BM;
-  if (q0 >= N) return;  // packed: past the end of a shorter document
-  const int wq0 = q0 + 32 * qw, qrow = wq0 + l32;
-  const float* qg = static_cast<const float*>(p.q.ptr) + sv.off(p.q, b) + h * p.q.sh;
-  const float* kg = static_cast<const float*>(p.k.ptr) + sv.off(p.k, b) + hk * p.k.sh;
-  const float* vg = static_cast<const float*>(p.v.ptr) + sv.off(p.v, b) + hk * p.v.sh;
+  if (block >= Plan::grid(p)) return;
+  const Plan pl(p, Plan::place(p, block));  // dispatch and K / V loads (ssa_rows_plan.hpp)
+  const SeqView& sv = pl.sv;
+  const int b = pl.b, h = pl.h, N = pl.N, nst = pl.nst;
+  if (pl.empty()) return;  // packed: past the end of a shorter document
+  const Loads ld(p, pl, lane, wave);
+  const int wq0 = pl.q0 + 32 * qw, qrow = wq0 + l32;
+  const float* qg = reinterpret_cast<const float*>(head_rows<4>(sv, p.q, b, h));
+  const float* kg = reinterpret_cast<const float*>(ld.k.g);
+  const float* vg = reinterpret_cast<const float*>(ld.v.g);
   const float n = *p.n_ptr, c = p.scale * *p.b_ptr;
   const uint32_t lds0 = lds_addr(smem);
-  const int64_t kss = p.k.ss * 2, vss = p.v.ss * 2;
-  const LoadLane llk(lane, wave, kss), llv(lane, wave, vss);
-  auto k_at = [&](int st, int i) { return lds0 + ((st & 1) * KW + i) * 2 * BB; };
-  auto load_stage = [&](int st) {
-#pragma unroll
-    for (int i = 0; i < KW; ++i) {
-      tile_load_async<M::LD, 32, 4>(kg, kss, st * BN + 32 * i, N, k_at(st, i), wave, llk);
-      tile_load_async<M::LD, 32, 4>(vg, vss, st * BN + 32 * i, N, k_at(st, i) + BB, wave, llv);
-    }
-  };
-  load_stage(0);
+  auto k_at = [&](int st, int i) { return Loads::k_at(lds0, st, i); };
+  ld.load(pl, 0, lds0, wave);
   const M mat(lane);
   typename M::frag qf[M::NF];
 #pragma unroll
@@ -176,12 +156,10 @@ __global__ __launch_bounds__(256) void ssa_fwd_f32_kernel(FwdParams p) {
 #pragma unroll
   for (int d = 0; d < ND; ++d) acc[d] = f32x16{};
   float m = -INFINITY, l = 0.f;
-  const int kv_end = CAUSAL ? min(N, q0 + BM) : N;
-  const int nst = (kv_end + BN - 1) / BN;
   for (int st = 0; st < nst; ++st) {
     __builtin_amdgcn_s_waitcnt(0);
     __syncthreads();  // stage st has landed, stage st - 1 is consumed
-    if (st + 1 < nst) load_stage(st + 1);
+    if (st + 1 < nst) ld.load(pl, st + 1, lds0, wave);
     const int k0 = st * BN + 32 * kw;
     if (k0 >= N || wq0 >= N || (CAUSAL && k0 > wq0 + 31)) continue;
     const f32x16 s = mat.scores(k_at(st, kw), qf);
@@ -279,23 +257,22 @@ __global__ __launch_bounds__(256) void ssa_bwd_preprocess_f32_kernel(BwdParams p
 // Delta), dS' = dT / (1 + c|x|), dV += P dO, dK += dS' q (scaled by scale n b
 // at the end), dn += ln2 dT sL, db += n scale dS' x.
 template <int D, bool CAUSAL, bool DO_DK, bool DO_DV>
-__device__ __forceinline__ void dkdv_f32_body(const BwdParams& p, char* smem, float (*red)[8], int block, int grid) {
+__device__ __forceinline__ void dkdv_f32_body(const BwdParams& p, char* smem, float (*red)[8], int block) {
   using M = Mat<D>;
   using C = Cfg<D>;
   constexpr int QS = C::QS, NWV = 4 * QS, BB = C::BB, ND = M::ND, STEP = 32 * QS;
+  using Plan = KeyPlan<D, 4, CAUSAL, QS, NWV>;
+  using Stage = KeyStageF32<D, QS>;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int l32 = lane & 31, hh = lane >> 5;
   const int qs = wave % QS, kg4 = wave / QS;
   const int nkb = dkdv_key_blocks(p.N);
-  const Place pl(block, grid, nkb, p.B, p.cu_seqlens != nullptr);
-  const int kb = pl.rank, b = pl.b, hk = pl.h, bhk = hk * p.B + b;
-  const int G = p.Hq / p.Hkv;
-  const SeqView sv(p.cu_seqlens, p.T, p.N, b);
-  const int N = sv.N;
+  const Plan pl(p, Plan::place(p, block));  // dispatch and Q / dO loads (ssa_rows_plan.hpp)
+  const SeqView& sv = pl.sv;
+  const int kb = pl.kb, b = pl.b, hk = pl.hk, bhk = pl.bhk, N = pl.N, k0 = pl.k0;
   const int64_t PP = static_cast<int64_t>(p.B) * p.Hkv * nkb;
-  const int k0 = kb * 128;
-  if (k0 >= N) {  // packed: past the end of a shorter document
+  if (pl.empty()) {  // packed: past the end of a shorter document
     if (DO_DK && tid == 0) {
       p.partials[static_cast<int64_t>(bhk) * nkb + kb] = 0.f;
       p.partials[PP + static_cast<int64_t>(bhk) * nkb + kb] = 0.f;
@@ -307,24 +284,10 @@ __device__ __forceinline__ void dkdv_f32_body(const BwdParams& p, char* smem, fl
   const float* vg = static_cast<const float*>(p.v.ptr) + sv.off(p.v, b) + hk * p.v.sh;
   const float n = *p.n_ptr, bv = *p.b_ptr, c = p.scale * bv;
   const uint32_t lds0 = lds_addr(smem);
-  const int64_t qss = p.q.ss * 2, doss = p.dout.ss * 2;
-  const LoadLane llq(lane, wave, qss), lld(lane, wave, doss);
-  const int qstart = CAUSAL ? k0 : 0;
-  const int nqs = (N - qstart + STEP - 1) / STEP, nst = G * nqs;
-  auto blk_at = [&](int st, int i) { return lds0 + (st & 1) * C::DKDV_STAGE + i * (2 * BB + 256); };
-  auto load_stage = [&](int st, int g, int q0) {
-    const int h = hk * G + g;
-    const float* qg = static_cast<const float*>(p.q.ptr) + sv.off(p.q, b) + h * p.q.sh;
-    const float* dog = static_cast<const float*>(p.dout.ptr) + sv.off(p.dout, b) + h * p.dout.sh;
-    const int64_t mr = sv.mrow(b, h, p.Hq, p.T, p.N);
-#pragma unroll
-    for (int i = 0; i < QS; ++i) {
-      const uint32_t at = blk_at(st, i);
-      tile_load_async<M::LD, 32, NWV>(qg, qss, q0 + 32 * i, N, at, wave, llq);
-      tile_load_async<M::LD, 32, NWV>(dog, doss, q0 + 32 * i, N, at + BB, wave, lld);
-      if (wave == NWV - 1 - i) pair32_load_async(p.m + mr, p.delta + mr, q0 + 32 * i, N, at + 2 * BB, lane);
-    }
-  };
+  const LoadLane llq(lane, wave, p.q.ss * 2), lld(lane, wave, p.dout.ss * 2);
+  const int qstart = pl.qstart, nst = pl.nst;
+  auto blk_at = [&](int st, int i) { return Stage::blk_at(lds0, st, i); };
+  auto load_stage = [&](int st, int g, int q0) { Stage::load(p, pl, st, g, q0, lds0, llq, lld, wave, lane); };
   load_stage(0, 0, qstart);
   const M mat(lane);
   typename M::frag kf[M::NF], vf[M::NF];
@@ -460,17 +423,17 @@ __device__ __forceinline__ void dkdv_f32_body(const BwdParams& p, char* smem, fl
 template <int D, bool CAUSAL, bool ROLES>
 __global__ __launch_bounds__((Cfg<D>::DKDV_THREADS)) void ssa_bwd_dkdv_f32_kernel(BwdParams p) {
   using C = Cfg<D>;
-  __shared__ __attribute__((aligned(1024))) char smem[2 * C::DKDV_STAGE];
+  __shared__ __attribute__((aligned(1024))) char smem[KeyStageF32<D, C::QS>::LDS_BYTES];
   __shared__ float red[3][8];
   const int block = folded_block(), grid = dkdv_key_blocks(p.N) * p.B * p.Hkv;
   if constexpr (ROLES) {
     // dK workgroups (three products per block) before the lighter dV ones
     if (block < grid)
-      dkdv_f32_body<D, CAUSAL, true, false>(p, smem, red, block, grid);
+      dkdv_f32_body<D, CAUSAL, true, false>(p, smem, red, block);
     else if (block < 2 * grid)
-      dkdv_f32_body<D, CAUSAL, false, true>(p, smem, red, block - grid, grid);
+      dkdv_f32_body<D, CAUSAL, false, true>(p, smem, red, block - grid);
   } else if (block < grid) {
-    dkdv_f32_body<D, CAUSAL, true, true>(p, smem, red, block, grid);
+    dkdv_f32_body<D, CAUSAL, true, true>(p, smem, red, block);
   }
 }
 
@@ -481,45 +444,36 @@ template <int D, bool CAUSAL>
 __global__ __launch_bounds__(256) void ssa_bwd_dq_f32_kernel(BwdParams p) {
   using M = Mat<D>;
   using C = Cfg<D>;
-  constexpr int KW = C::KW, BM = C::BM, BN = C::BN, BB = C::BB, ND = M::ND;
-  __shared__ __attribute__((aligned(1024))) char smem[C::LDS_BYTES];
+  using Plan = RowPlan<D, 4, CAUSAL, C::KW>;
+  using Loads = RowLoadsF32<D, CAUSAL, C::KW>;
+  constexpr int KW = C::KW, BN = C::BN, BB = C::BB, ND = M::ND;
+  __shared__ __attribute__((aligned(1024))) char smem[Loads::LDS_BYTES];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int l32 = lane & 31, hh = lane >> 5;
   const int kw = wave % KW, qw = wave / KW;
-  const int nqb = (p.N + BM - 1) / BM, grid = nqb * p.B * p.Hq;
   const int block = folded_block();
-  if (block >= grid) return;
+  if (block >= Plan::grid(p)) return;
   if (p.fuse_reduce && block == 0) {  // the backward's dn / db sums, before the first load (reduce_partials_body)
     reduce_partials_body(p.partials, static_cast<int64_t>(p.B) * p.Hkv * dkdv_key_blocks(p.N), p.dn, p.db,
                          reinterpret_cast<float(*)[256]>(smem), threadIdx.x);
     __syncthreads();
   }
-  const Place pl(block, grid, nqb, p.B, p.cu_seqlens != nullptr);
-  const int b = pl.b, h = pl.h, hk = h / (p.Hq / p.Hkv);
-  const SeqView sv(p.cu_seqlens, p.T, p.N, b);
-  const int N = sv.N;
-  const int q0 = (nqb - 1 - pl.rank) * BM;
-  if (q0 >= N) return;  // packed: past the end of a shorter document
-  const int wq0 = q0 + 32 * qw, qrow = wq0 + l32;
-  const float* qg = static_cast<const float*>(p.q.ptr) + sv.off(p.q, b) + h * p.q.sh;
-  const float* dog = static_cast<const float*>(p.dout.ptr) + sv.off(p.dout, b) + h * p.dout.sh;
-  const float* kg = static_cast<const float*>(p.k.ptr) + sv.off(p.k, b) + hk * p.k.sh;
-  const float* vg = static_cast<const float*>(p.v.ptr) + sv.off(p.v, b) + hk * p.v.sh;
+  const Plan pl(p, Plan::place(p, block));
+  const SeqView& sv = pl.sv;
+  const int b = pl.b, h = pl.h, N = pl.N, nst = pl.nst;
+  if (pl.empty()) return;  // packed: past the end of a shorter document
+  const Loads ld(p, pl, lane, wave);
+  const int wq0 = pl.q0 + 32 * qw, qrow = wq0 + l32;
+  const float* qg = reinterpret_cast<const float*>(head_rows<4>(sv, p.q, b, h));
+  const float* dog = reinterpret_cast<const float*>(head_rows<4>(sv, p.dout, b, h));
+  const float* kg = reinterpret_cast<const float*>(ld.k.g);
+  const float* vg = reinterpret_cast<const float*>(ld.v.g);
   const int64_t mr = sv.mrow(b, h, p.Hq, p.T, p.N);
   const float n = *p.n_ptr, bv = *p.b_ptr, c = p.scale * bv;
   const uint32_t lds0 = lds_addr(smem);
-  const int64_t kss = p.k.ss * 2, vss = p.v.ss * 2;
-  const LoadLane llk(lane, wave, kss), llv(lane, wave, vss);
-  auto k_at = [&](int st, int i) { return lds0 + ((st & 1) * KW + i) * 2 * BB; };
-  auto load_stage = [&](int st) {
-#pragma unroll
-    for (int i = 0; i < KW; ++i) {
-      tile_load_async<M::LD, 32, 4>(kg, kss, st * BN + 32 * i, N, k_at(st, i), wave, llk);
-      tile_load_async<M::LD, 32, 4>(vg, vss, st * BN + 32 * i, N, k_at(st, i) + BB, wave, llv);
-    }
-  };
-  load_stage(0);
+  auto k_at = [&](int st, int i) { return Loads::k_at(lds0, st, i); };
+  ld.load(pl, 0, lds0, wave);
   const M mat(lane);
   typename M::frag qf[M::NF], dof[M::NF];
 #pragma unroll
@@ -531,12 +485,10 @@ __global__ __launch_bounds__(256) void ssa_bwd_dq_f32_kernel(BwdParams p) {
   f32x16 dq[ND];
 #pragma unroll
   for (int d = 0; d < ND; ++d) dq[d] = f32x16{};
-  const int kv_end = CAUSAL ? min(N, q0 + BM) : N;
-  const int nst = (kv_end + BN - 1) / BN;
   for (int st = 0; st < nst; ++st) {
     __builtin_amdgcn_s_waitcnt(0);
     __syncthreads();  // stage st has landed, stage st - 1 is consumed
-    if (st + 1 < nst) load_stage(st + 1);
+    if (st + 1 < nst) ld.load(pl, st + 1, lds0, wave);
     const int k0 = st * BN + 32 * kw;
     if (k0 >= N || wq0 >= N || (CAUSAL && k0 > wq0 + 31)) continue;
     const uint32_t at = k_at(st, kw);

@@ -1,4 +1,5 @@
-// Global-memory plans of the kernels that stream tiles: for one workgroup,
+// Global-memory plans of the 16-bit kernels that stream tiles (ssa_rows_plan.hpp: the
+// fp32-precision ones): for one workgroup,
 // wave and lane, the dispatch (which sequence, head and block a workgroup
 // takes), which rows of which tensor every direct-to-LDS load fetches, and
 // where every dS' workspace store goes.  The kernels issue their loads and

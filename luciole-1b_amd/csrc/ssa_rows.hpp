@@ -5,6 +5,7 @@
 
 #include "ssa_common.hpp"
 #include "ssa_launch.hpp"
+#include "ssa_rows_plan.hpp"
 #include "ssa_tile.hpp"
 
 namespace ssa {
@@ -33,19 +34,6 @@ __device__ __forceinline__ void st4(T* p, f32x4 v) {
 
 // sL = sign(x) log2(1 + c|x|) for a raw score x = q.k, c = scale b; u1 = 1 + c|x|
 __device__ __forceinline__ float ssa_sl(float x, float u1) { return copysignf(fast_log2(u1), x); }
-
-// A workgroup's place in a grid of nblk blocks of rows per (sequence, head):
-// XCD-contiguous, the heaviest blocks (rank 0) of a pair of heads first, as
-// FwdPlan and DkdvPlan.
-struct Place {
-  int rank, b, h;
-  __device__ __forceinline__ Place(int block, int grid, int nblk, int B, bool packed) {
-    int hb;
-    dispatch_order(xcd_remap(block, grid), grid / nblk, nblk, packed ? 1 : kOrderGroup, hb, rank);
-    b = hb % B;
-    h = hb / B;
-  }
-};
 
 // Sum of the accumulators of the waves that share owned rows, in the first of them (part == 0): the others leave theirs
 // in LDS, element-major so that every access is contiguous.  Called by every

@@ -1,4 +1,5 @@
-// Host replay of the kernels' global-memory plans (luciole-1b_amd/csrc/ssa_plan.hpp).
+// Host replay of the kernels' global-memory plans (luciole-1b_amd/csrc/ssa_plan.hpp
+// and, of the fp32-precision kernels, ssa_rows_plan.hpp).
 //
 // The plans hold the dispatch and per-lane address arithmetic of every
 // tile-streaming kernel, as __host__ __device__ code that the kernels call
@@ -31,6 +32,7 @@
 // malformed document tables) and the benchmark sizes (a sample of their
 // workgroups, on address-only buffers).  Exit status 0 and "0 failures" when
 // every check holds.
+#include <algorithm>
 #include <cinttypes>
 #include <cstdarg>
 #include <cstdio>
@@ -40,9 +42,12 @@
 #include <memory>
 #include <set>
 #include <string>
+#include <tuple>
+#include <type_traits>
 #include <vector>
 
 #include "ssa_plan.hpp"
+#include "ssa_rows_plan.hpp"
 
 using namespace ssa;
 
@@ -874,6 +879,205 @@ void run_case(const Case& c) {
   fflush(stdout);
 }
 
+// ---------------------------------------------------------------------------
+// The fp32-precision kernels (ssa_f32.hip, ssa_d256.hip).  An fp32 row of D elements
+// is one of 2 D 16-bit columns here; the plans get its strides in elements.
+template <typename P>
+P in_elements(P p, int E) {
+  auto half = [&](Tensor4& t) { t.sb /= E / 2, t.sh /= E / 2, t.ss /= E / 2; };
+  half(p.q), half(p.k), half(p.v);
+  if constexpr (std::is_same_v<P, BwdParams>) half(p.dout);
+  return p;
+}
+
+// Forward and dQ: one call of `load` issues stage st of K and V into the slots that
+// `at` names.
+template <typename Plan, typename Loads, typename Params, typename Load, typename At>
+void run_rows(Problem& P, const Params& p, const char* what, Load load, At at) {
+  const int grid = Plan::grid(p);
+  Replay R;
+  g_r = &R;
+  std::set<std::tuple<int, int, int>> units;
+  for (int blk = 0; blk < grid; ++blk) {
+    const Plan pl(p, Plan::place(p, blk));
+    CHECK(units.insert({pl.b, pl.h, pl.q0}).second, "%s: unit (b %d, h %d, q0 %d) dispatched twice", what, pl.b, pl.h,
+          pl.q0);
+    CHECK(pl.q0 >= 0 && pl.q0 % Plan::BM == 0, "%s: first query %d", what, pl.q0);
+    if (pl.empty()) continue;
+    g_ctx = fmt("%s %s columns=%d block %d (b %d h %d q0 %d)", P.c.name.c_str(), what, Plan::LD, blk, pl.b, pl.h, pl.q0);
+    R.reset_lds(Loads::LDS_BYTES);
+    for (int st = 0; st < pl.nst; ++st) {
+      for (int w = 0; w < Plan::NW; ++w)
+        for (int l = 0; l < 64; ++l) {
+          R.start_lane(l);
+          const Loads ld(p, pl, l, w);
+          load(ld, pl, st, w);
+        }
+      std::vector<Region> regs;
+      for (int i = 0; i < Plan::BN / 32; ++i)
+        for (Tensor* t : {&P.k, &P.v})
+          regs.push_back(Region{t, pl.b, pl.sv.tok0, P.packed, pl.hk, st * Plan::BN + 32 * i, 32, pl.N,
+                                at(st, i, t == &P.v)});
+      check_regions(R, regs);
+    }
+    CHECK(pl.nst * Plan::BN >= (P.c.causal ? std::min(pl.N, pl.q0 + Plan::BM) : pl.N), "%s: %d stages for %d keys", what,
+          pl.nst, pl.N);
+  }
+  CHECK(static_cast<int64_t>(units.size()) == grid, "%s: %zu units for %d workgroups", what, units.size(), grid);
+}
+
+template <int D, bool CAUSAL>
+void run_rows_f32(Problem& P) {
+  constexpr int KW = SplitF32<D>::KW;
+  using Plan = RowPlan<D, 4, CAUSAL, KW>;
+  using Loads = RowLoadsF32<D, CAUSAL, KW>;
+  auto load = [](const Loads& ld, const Plan& pl, int st, int w) { ld.load(pl, st, 0u, w, HostMem()); };
+  auto at = [](int st, int i, bool v) { return static_cast<uint32_t>(((st & 1) * KW + i) * 2 * Plan::BB + (v ? Plan::BB : 0)); };
+  run_rows<Plan, Loads>(P, in_elements(P.fp, 4), "fp32 forward", load, at);
+  run_rows<Plan, Loads>(P, in_elements(P.bp, 4), "fp32 dQ", load, at);
+}
+
+template <bool CAUSAL, int KS, typename Params>
+void run_rows_256(Problem& P, const Params& p, const char* what) {
+  using Plan = RowPlan<256, 2, CAUSAL, 2>;
+  using Loads = RowLoads256<CAUSAL, 2, KS, 2>;
+  run_rows<Plan, Loads>(
+      P, p, what,
+      [](const Loads& ld, const Plan& pl, int st, int w) {
+        ld.load_k(pl, st, st % KS, 0u, w, HostMem());
+        ld.load_v(pl, st, st % 2, 0u, w, HostMem());
+        ld.load_k(pl, pl.nst, 0, 0u, w, HostMem());  // past the last stage: nothing
+        ld.load_v(pl, pl.nst + 1, 0, 0u, w, HostMem());
+      },
+      [](int st, int i, bool v) {
+        return static_cast<uint32_t>(((v ? KS + st % 2 : st % KS) * 2 + i) * Plan::BB);
+      });
+}
+
+// dK/dV: stages over the queries of every q-head of the group.
+template <typename Plan, int QS, int LDS, typename Load, typename At>
+void run_keys(Problem& P, const BwdParams& p, const char* what, int NW, Load load, At at) {
+  const int grid = Plan::grid(p);
+  Replay R;
+  g_r = &R;
+  std::set<std::tuple<int, int, int>> units;
+  for (int blk = 0; blk < grid; ++blk) {
+    const Plan pl(p, Plan::place(p, blk));
+    CHECK(units.insert({pl.b, pl.hk, pl.kb}).second, "%s: unit dispatched twice", what);
+    CHECK(pl.bhk == pl.hk * p.B + pl.b && pl.k0 == pl.kb * 128, "%s: key block %d of %d", what, pl.kb, pl.bhk);
+    if (pl.empty()) continue;
+    g_ctx = fmt("%s %s columns=%d block %d (b %d hk %d kb %d)", P.c.name.c_str(), what, Plan::LD, blk, pl.b, pl.hk, pl.kb);
+    R.reset_lds(LDS);
+    const int first = P.c.causal ? pl.k0 : 0, per = (pl.N - first + 32 * QS - 1) / (32 * QS);
+    CHECK(pl.nst == per * (p.Hq / p.Hkv), "%s: %d stages, want %d a head", what, pl.nst, per);
+    auto state = load.start(pl);
+    for (int st = 0; st < pl.nst + 2; ++st) {
+      const int g = st / per, q0 = first + st % per * 32 * QS;
+      for (int w = 0; w < NW; ++w)
+        for (int l = 0; l < 64; ++l) {
+          R.start_lane(l);
+          load(state, p, pl, st, g, q0, w, l);
+        }
+      if (st >= pl.nst) {
+        CHECK(R.log.empty(), "%s issues loads for stage %d past the last (%d)", what, st, pl.nst);
+        continue;
+      }
+      const int h = pl.hk * (p.Hq / p.Hkv) + g;
+      std::vector<Region> regs;
+      for (int i = 0; i < QS; ++i) {
+        const auto [ql, dl, ml] = at(st, i);
+        regs.push_back(Region{&P.q, pl.b, pl.sv.tok0, P.packed, h, q0 + 32 * i, 32, pl.N, ql});
+        regs.push_back(Region{&P.dout, pl.b, pl.sv.tok0, P.packed, h, q0 + 32 * i, 32, pl.N, dl});
+        md_regions(regs, P, pl.b, pl.sv, h, q0 + 32 * i, 32, pl.N, ml);
+      }
+      check_regions(R, regs);
+    }
+  }
+  CHECK(static_cast<int64_t>(units.size()) == grid, "%s: %zu units for %d workgroups", what, units.size(), grid);
+}
+
+template <int D, bool CAUSAL>
+struct KeyLoadF32 {
+  static constexpr int QS = SplitF32<D>::QS;
+  using Plan = KeyPlan<D, 4, CAUSAL, QS, 4 * QS>;
+  using Stage = KeyStageF32<D, QS>;
+  int start(const Plan&) const { return 0; }
+  void operator()(int, const BwdParams& p, const Plan& pl, int st, int g, int q0, int w, int l) const {
+    const LoadLane llq(l, w, p.q.ss * 2), lld(l, w, p.dout.ss * 2);
+    if (st < pl.nst) Stage::load(p, pl, st, g, q0, 0u, llq, lld, w, l, HostMem());  // the kernel's guard
+  }
+};
+template <int D, bool CAUSAL>
+void run_keys_f32(Problem& P) {
+  typedef KeyLoadF32<D, CAUSAL> L;
+  run_keys<typename L::Plan, L::QS, L::Stage::LDS_BYTES>(
+      P, in_elements(P.bp, 4), "fp32 dK/dV", 4 * L::QS, L(), [](int st, int i) {
+        const uint32_t at = static_cast<uint32_t>(((st & 1) * L::QS + i) * (2 * L::Plan::BB + 256));
+        return std::tuple<uint32_t, uint32_t, uint32_t>(at, at + L::Plan::BB, at + 2 * L::Plan::BB);
+      });
+}
+
+template <bool CAUSAL, bool DK>
+struct KeyLoad256 {
+  using Plan = KeyPlan<256, 2, CAUSAL, 1, 4>;
+  using Ring = KeyRing256<DK>;
+  std::vector<Ring> start(const Plan& pl) const { return std::vector<Ring>(256, Ring(pl.qstart)); }
+  void operator()(std::vector<Ring>& r, const BwdParams& p, const Plan& pl, int, int, int, int w, int l) const {
+    const LoadLane llq(l, w, p.q.ss), lld(l, w, p.dout.ss);
+    r[w * 64 + l].load_next(p, pl, 0u, llq, lld, w, l, HostMem());
+  }
+};
+template <bool CAUSAL, bool DK>
+void run_keys_256(Problem& P) {
+  typedef KeyLoad256<CAUSAL, DK> L;
+  run_keys<typename L::Plan, 1, L::Ring::LDS_BYTES>(P, P.bp, DK ? "head dim 256 dK" : "head dim 256 dV", 4, L(),
+                                                    [](int st, int) {
+    constexpr uint32_t BB = L::Plan::BB;
+    return std::tuple<uint32_t, uint32_t, uint32_t>(st % (DK ? 3 : 2) * BB, ((DK ? 3 : 2) + st % (DK ? 2 : 3)) * BB,
+                                                    5 * BB + st % 3 * 256);
+  });
+}
+
+template <int D, bool CAUSAL>
+void run_f32_dc(Problem& P) {
+  run_rows_f32<D, CAUSAL>(P);
+  run_keys_f32<D, CAUSAL>(P);
+}
+template <bool CAUSAL>
+void run_256_c(Problem& P) {
+  run_rows_256<CAUSAL, 2>(P, P.fp, "head dim 256 forward");
+  run_rows_256<CAUSAL, 3>(P, P.bp, "head dim 256 dQ");
+  run_keys_256<CAUSAL, true>(P);
+  run_keys_256<CAUSAL, false>(P);
+}
+
+// fp32 at head dim D (0: 16-bit at 256) on the case's shape, whose own head dim does not count
+void run_precise(Case c, int D) {
+  c.D = D == 0 ? 256 : 2 * D;
+  Problem P;
+  P.c = c;
+  setup(P);
+  const long f0 = g_fail;
+  switch (D * 2 + c.causal) {
+    case 0: run_256_c<false>(P); break;
+    case 1: run_256_c<true>(P); break;
+    case 32: run_f32_dc<16, false>(P); break;
+    case 33: run_f32_dc<16, true>(P); break;
+    case 64: run_f32_dc<32, false>(P); break;
+    case 65: run_f32_dc<32, true>(P); break;
+    case 128: run_f32_dc<64, false>(P); break;
+    case 129: run_f32_dc<64, true>(P); break;
+    case 256: run_f32_dc<128, false>(P); break;
+    case 257: run_f32_dc<128, true>(P); break;
+    case 512: run_f32_dc<256, false>(P); break;
+    case 513: run_f32_dc<256, true>(P); break;
+    default: failf("fp32 head dim %d not built", D);
+  }
+  printf("case %-34s %s\n", fmt("%s as %s %d", c.name.c_str(), D == 0 ? "16-bit" : "fp32", D == 0 ? 256 : D).c_str(),
+         g_fail == f0 ? "ok" : "FAILED");
+  fflush(stdout);
+}
+
 Case dense(const char* name, int B, int Hq, int Hkv, int N, int D, bool causal, int layout) {
   return Case{name, B, Hq, Hkv, N, D, causal, layout, {}, 0, 0};
 }
@@ -918,6 +1122,11 @@ int main(int argc, char** argv) {
     cases.push_back(c);
   }
   for (const Case& c : cases) run_case(c);
+  // the fp32-precision kernels: every head dim; with and without the mask, GQA,
+  // strided, ragged, packed and malformed, on the smaller of the shapes
+  const std::vector<std::pair<int, int>> precise = {{1, 64}, {2, 0},  {4, 256}, {4, 0},  {5, 128},
+                                                    {6, 16}, {10, 0}, {13, 16}, {14, 32}};
+  for (const auto& [k, dim] : precise) run_precise(cases[k], dim);
   // decode against a KV cache: ragged lengths, lengths beyond the capacity
   // and below zero (clamped), one and several splits, q-head groups past 32
   g_ctx = "decode";

@@ -2,9 +2,11 @@
 and UndefinedBehaviorSanitizer.
 
 luciole-1b_amd/csrc/ssa_plan.hpp holds the dispatch and per-lane load / store
-addressing of every tile-streaming kernel (forward, both dK/dV kernels, the dS'
-K pass, the recompute dQ pass, decode) as __host__ __device__ code; the
-kernels call it with the device memory policy.  tests/host_addr/addr_replay.cpp
+addressing of the 16-bit tile-streaming kernels (forward, both dK/dV kernels, the
+dS' K pass, the recompute dQ pass, decode) as __host__ __device__ code, and
+ssa_rows_plan.hpp the dispatch, stage rings and tile loads of the fp32-precision
+ones (fp32; head dim 256: forward, dQ, dK/dV); the kernels call it with the
+device memory policy.  tests/host_addr/addr_replay.cpp
 calls the same code for every workgroup, wave and lane of dense, GQA,
 Megatron-strided, ragged and packed problems (and a sample of the benchmark
 sizes), performing each access on exact-size host buffers and checking rows,
@@ -79,6 +81,14 @@ MUTATIONS = [
      "const int soff = mem.uniform(g * ds_tph1k + (CAUSAL ? qt * (qt + 1) : qt * 2 * nq32) * 1024 + "
      "static_cast<int>((ds_voff >> 4) & 1));",
      "a per-lane value passed where the kernel states a wave-uniform one"),
+    ("ssa_rows_plan.hpp", "k(head_rows<4>(pl.sv, p.k, pl.b, pl.hk), p.k.ss * 2, lane, wave)",
+     "k(head_rows<4>(pl.sv, p.k, pl.b, pl.h), p.k.ss * 2, lane, wave)",
+     "fp32 K rows of the q-head's number instead of its kv-head's"),
+    ("ssa_rows_plan.hpp", "d_slot = d_slot + 1 == RD ? 0 : d_slot + 1;", "d_slot = d_slot + 1 == RQ ? 0 : d_slot + 1;",
+     "head dim 256 dK/dV: the dO ring turns over with Q's"),
+    ("ssa_rows_plan.hpp", "const int kv_end = CAUSAL ? (N < q0 + BM ? N : q0 + BM) : N;",
+     "const int kv_end = CAUSAL ? (N < q0 + BM ? N : q0) : N;",
+     "the causal diagonal's keys left out"),
 ]
 
 
