@@ -5,7 +5,7 @@ A "step" is one forward + backward of the SSA attention op through the
 reference-compatible kernel API (ssa_flash_attn_forward +
 ssa_flash_attn_backward) on synthetic inputs already resident in HBM:
 B=4, H=16, S=4096, D=128, bf16, causal, Q/K/V = 0.5 N(0,1), dO ~ N(0,1),
-n=1.5, b=0.8, scale=1/sqrt(D) (the shape BASELINE.json's metric is quoted on).
+n=1.5, b=0.8, scale=1/sqrt(D) (the headline shape).
 
 value = algorithmic fwd+bwd FLOPs / step time, with fwd = 4 D pairs and
 bwd = 10 D pairs (pairs = unmasked (q, k) pairs), i.e. 14 D pairs per step.
@@ -52,20 +52,20 @@ PEAK_FP32_VALU_TFLOPS = 78.6
 
 CONFIGS = {
     # name: (B, Hq, Hkv, S, D, causal)
-    "s4096": (4, 16, 16, 4096, 128, True),   # north star: BASELINE.json metric shape
-    "s2048": (4, 16, 16, 2048, 128, True),
-    "s16384": (1, 16, 16, 16384, 128, True),
+    "s4096": (4, 16, 16, 4096, 128, True),   # the headline shape
+    "s2048": (4, 16, 16, 2048, 128, True),   # shorter sequences
+    "s16384": (1, 16, 16, 16384, 128, True),  # long context
     "gqa_d64": (4, 32, 8, 4096, 64, True),   # production Luciole-1B attention shape
 }
-# packed sequences, 16384 tokens per micro-batch,
+# Packed sequences, 16384 tokens per micro-batch,
 # document lengths uniform in [64, 4096] from random.Random(1234), the last
 # document truncated to fill; H = 16, D = 128, causal inside each document.
 VARLEN_CONFIGS = {"varlen16k": (16384, 16, 16, 128, 64, 4096)}
+# One optimizer step of a 1B Llama-style decoder with SSA attention
+# (SSA/ssa_decoder.py defaults), micro-batch 4 x 4096 tokens.
+TRAIN_CONFIGS = {"train1b": 4}
 # Decode step against a KV cache (no reference kernel: the reference re-runs the
 # prefix per generated token): name: (B, Hq, Hkv, cache length, D).
-# one optimizer step of a 1B Llama-style decoder with
-# SSA attention (SSA/ssa_decoder.py defaults), micro-batch 4 x 4096 tokens.
-TRAIN_CONFIGS = {"train1b": 4}
 DECODE_CONFIGS = {
     "decode_s4096": (16, 16, 16, 4096, 128),
     "decode_gqa_d64": (16, 32, 8, 4096, 64),
@@ -381,7 +381,7 @@ def cpu_baseline(B, H, S, D, causal, budget_s=20.0):
     """The fp32 PyTorch-eager oracle (oracle/ssa_oracle_torch.py, fwd + autograd
     bwd) on the host cores, as a reported baseline:
 
-    * BASELINE.json configs[0] (B=1, H=4, S=256, D=64, fp32, causal; N(0,1)
+    * a small problem (B=1, H=4, S=256, D=64, fp32, causal; N(0,1)
       inputs) timed in full: 3 warm-up runs, median of 10;
     * the GPU workload timed on (b, h) slices -- one slice's S x S fp32
       intermediates are what fit -- with the number of slices timed and the
@@ -413,7 +413,7 @@ def cpu_baseline(B, H, S, D, causal, budget_s=20.0):
         "full_step_s_extrapolated": slices * med,
         "cpu_model": model,
         "os_cpu_count": threads,
-        "config0": {"workload": "BASELINE.json configs[0]: B=1 H=4 S=256 D=64 fp32 causal, timed in full",
+        "config0": {"workload": "B=1 H=4 S=256 D=64 fp32 causal, timed in full",
                     "ms": c1_med * 1e3, "runs": c1_runs, "tflops": c1_flop / c1_med / 1e12,
                     "alg_mflop": c1_flop / 1e6},
     }
@@ -635,7 +635,7 @@ def device_clock_and_peak():
 
 
 def bench_varlen(args, dev):
-    """Packed-sequence fwd + bwd step; same JSON line."""
+    """Packed-sequence fwd + bwd step (16384 tokens, --config varlen16k); same JSON line."""
     import torch
 
     from SSA.ssa_hip_kernel import ssa_flash_attn_varlen_backward, ssa_flash_attn_varlen_forward

@@ -2,7 +2,7 @@
 
 TEST INFRASTRUCTURE ONLY.  Only ``tests/``, ``__graft_entry__.smoke()`` and the
 ``cpu_baseline`` leg of ``bench.py`` may import this module, and only as the
-checker.  The product path (``luciole-1b_amd/SSA``) never imports it and fails
+oracle.  The product path (``luciole-1b_amd/SSA``) never imports it and fails
 loudly when the HIP library is missing.
 
 This is a closed-form restatement of the reference's SSA math:

@@ -24,7 +24,7 @@ import torch
 
 from oracle import ssa_oracle as so
 
-# max abs error <= 2e-2 in bf16 against the fp32/fp64 oracle.
+# The bar: max abs error <= 2e-2 in bf16 against the fp32/fp64 oracle.
 MAX_ABS = 2e-2
 # Reference harness allclose tolerances for bf16/fp16 tensors and scalars
 # (check_ssa_triton_parity.py:1060-1069).

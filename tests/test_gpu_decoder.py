@@ -117,7 +117,7 @@ def test_decoder_cached_generation_equals_prefix_recompute(gpu):
 
 
 def test_decoder_full_size_train_steps(gpu):
-    """BASELINE.json configs[4] at its real size: ``SSADecoderConfig()`` (24
+    """The 1B train step at its real size: ``SSADecoderConfig()`` (24
     layers, hidden 2048, 16 x 128 heads, SwiGLU 5632, vocab 65536), micro-batch
     4 x 4096 tokens, three ``train_step`` calls with fused AdamW (the layer
     order of ssa_triton_layer_specs.py:96-127).  The first loss is

@@ -1,4 +1,4 @@
-"""GPU parity at the benchmark's full sizes (BASELINE.json configs).
+"""GPU parity at the benchmark's full sizes.
 
 The kernels run on the whole problem (every head, every key block, the real
 dispatch order and workspace sizes), and one (batch, kv-head group) slice of

@@ -1,9 +1,9 @@
-"""GPU parity for the long-context configuration (BASELINE.json configs[2]):
+"""GPU parity for the long-context configuration:
 B=1, H=16, S=16384, D=128, bf16, causal, Q/K/V = 0.5 N(0,1), dO ~ N(0,1).
 
 At this length SSA's sequence-dependent scores matter most, and dn / db sum
 over ~2e9 (query, key) pairs per step.  The dense oracle cannot build its
-16k x 16k float64 matrices, so the checker is the row-block evaluation
+16k x 16k float64 matrices, so the oracle is the row-block evaluation
 ``ssa_forward_backward_chunked`` (pinned against the dense oracle in
 tests/test_oracle.py):
 

@@ -188,7 +188,7 @@ def test_parity_divergent_layer_n_m302(gpu):
 
 
 def test_parity_baseline_distribution(gpu):
-    # BASELINE.json config distribution: Q/K/V = 0.5 N(0,1), dO ~ N(0,1)
+    # The benchmark's distribution: Q/K/V = 0.5 N(0,1), dO ~ N(0,1)
     _check(*_run(gpu, 1, 4, 4, 1024, 128, torch.bfloat16, True, qkv_scale=0.5))
 
 

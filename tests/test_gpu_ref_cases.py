@@ -116,7 +116,7 @@ def main(path):
     ok = all(r["passed"] for r in report)
     Path(path).write_text(
         "# Parity on the reference harness's 96 kernel case shapes: this build vs the reference Triton kernel\n\n"
-        f"Command (repo root, GPU box): `python tests/test_gpu_ref_cases.py {path}`, which also writes\n"
+        f"Command (repo root, on an MI355X): `python tests/test_gpu_ref_cases.py {path}`, which also writes\n"
         f"`{Path(path).with_suffix('.json')}` (per case: the shape, seed, pass flag, this build's errors against the "
         "fp64\noracle and the kernel-level backward, the reference's recorded errors; the limits at the top).\n"
         f"{'All' if ok else 'NOT all'} {len(report)} cases pass (`overall_passed: {str(ok).lower()}`).  Inputs are "

@@ -36,7 +36,7 @@ def _run(cmd, cwd):
     return res
 
 
-@pytest.mark.skipif(os.path.exists("/dev/kfd"), reason="a GPU is visible; the driver passes fake device pointers")
+@pytest.mark.skipif(os.path.exists("/dev/kfd"), reason="a GPU is visible; the validation program passes fake device pointers")
 def test_validation_is_ub_free_under_sanitizers(tmp_path):
     if not (Path(HIPCC).exists() and Path(CLANG).exists()):
         pytest.skip("hipcc / ROCm clang not found")
